@@ -190,10 +190,17 @@ struct eos_scene {
     eos::DevBuf verts, normals, matidx;
     eos::DevBuf mats, lights;
     // LBVH and sorted layouts
-    eos::DevBuf nodes, geo, shade;
+    // tree: the 4-wide nodes, then the triangle geometry records, in one allocation:
+    // the traversal addresses both from one base with 32-bit byte offsets (a tree
+    // past 4 GiB, about 45 million triangles, takes kernels with 64-bit addresses)
+    eos::DevBuf nodes, tree, shade;
+    size_t tree_bytes() const { return 128 * (size_t)n_nodes4 + 48 * (size_t)n_tri; }
+    bool tree_big() const { return tree_bytes() > (size_t)UINT32_MAX; }
+    eos::Node4* nodes4() const { return tree.as<eos::Node4>(); }
+    float4* geo() const { return reinterpret_cast<float4*>(tree.as<char>() + 128 * (size_t)n_nodes4); }
     eos::DevBuf codes, codes_sorted, perm, kchild, kparent, first_last, ibox, lbox, flags, cbounds;
     eos::DevBuf sort_tmp_k, sort_tmp_v, sort_hist, bounds_part;
-    eos::DevBuf nodes4, flags4, scan_tmp;
+    eos::DevBuf flags4, scan_tmp;
     // per-triangle transformations: xf [n_xf][kXfRows] float4, xf_index [N]
     // (original order, -1 = none), world-space vertices for the build
     eos::DevBuf xf, xf_index, wverts;

@@ -549,7 +549,6 @@ eos_status build_lbvh(eos_scene* s, int leaf_max, int width, eos_build_stats* st
     EOS_TRY(s->cbounds.ensure(64));
     EOS_TRY(s->bounds_part.ensure(24 * (size_t)nparts));
     EOS_TRY(s->nodes.ensure(64 * m));
-    EOS_TRY(s->geo.ensure(48 * un));
     EOS_TRY(s->shade.ensure(48 * un));
     EOS_HIP(hipEventRecord(s->ev[0], S));
     int32_t* err = s->cbounds.as<int32_t>() + 8;
@@ -613,10 +612,6 @@ eos_status build_lbvh(eos_scene* s, int leaf_max, int width, eos_build_stats* st
             hipLaunchKernelGGL(k_nodes, dim3(blocks(m, 256)), dim3(256), 0, S, s->kchild.as<const int2>(),
                                s->first_last.as<const int2>(), s->ibox.as<const float>(), s->lbox.as<const float>(),
                                cb, n, leaf_max, s->nodes.as<Node>());
-        hipLaunchKernelGGL(k_tris, dim3(blocks(un, 256)), dim3(256), 0, S, s->verts.as<const float>(),
-                           s->normals.as<const float>(), s->matidx.as<const int32_t>(), vA, n, s->n_mat,
-                           xf ? s->xf_index.as<const int32_t>() : nullptr, s->n_xf, s->geo.as<float4>(),
-                           s->shade.as<float4>(), err);
         if (n > leaf_max) {
             // 4-wide collapse: flags, their exclusive scan (node numbers), node count, nodes
             const int nb = (int)blocks(m, kScanBlock);
@@ -635,11 +630,16 @@ eos_status build_lbvh(eos_scene* s, int leaf_max, int width, eos_build_stats* st
             EOS_HIP(hipMemcpyAsync(&tail[1], idx + (m - 1), 4, hipMemcpyDeviceToHost, S));
             EOS_HIP(hipStreamSynchronize(S));
             s->n_nodes4 = tail[0] + tail[1];
-            EOS_TRY(s->nodes4.ensure(128 * (size_t)std::max(s->n_nodes4, 1)));
+            EOS_TRY(s->tree.ensure(s->tree_bytes()));
             hipLaunchKernelGGL(k_nodes4, dim3(blocks(m, 256)), dim3(256), 0, S, s->kchild.as<const int2>(),
                                s->first_last.as<const int2>(), s->ibox.as<const float>(), s->lbox.as<const float>(),
-                               cb, flags, idx, n, leaf_max, s->nodes4.as<Node4>());
+                               cb, flags, idx, n, leaf_max, s->nodes4());
         }
+        EOS_TRY(s->tree.ensure(s->tree_bytes()));
+        hipLaunchKernelGGL(k_tris, dim3(blocks(un, 256)), dim3(256), 0, S, s->verts.as<const float>(),
+                           s->normals.as<const float>(), s->matidx.as<const int32_t>(), vA, n, s->n_mat,
+                           xf ? s->xf_index.as<const int32_t>() : nullptr, s->n_xf, s->geo(),
+                           s->shade.as<float4>(), err);
     }
     EOS_HIP(hipGetLastError());
     EOS_HIP(hipEventRecord(s->ev[1], S));
@@ -1129,7 +1129,6 @@ eos_status build_lbvh_batch(eos_scene* const* scenes, int n_scenes, int leaf_max
         if (N + un > (size_t)INT_MAX / 2)
             return fail(EOS_ERR_LIMIT, "eos_build_lbvh_batch: more than 2^30 triangles in one batch");
         EOS_TRY(s->nodes.ensure(64 * (un - 1)));
-        EOS_TRY(s->geo.ensure(48 * un));
         EOS_TRY(s->shade.ensure(48 * un));
         EOS_TRY(s->perm.ensure(4 * un));
         EOS_TRY(s->codes_sorted.ensure(4 * un));
@@ -1147,7 +1146,6 @@ eos_status build_lbvh_batch(eos_scene* const* scenes, int n_scenes, int leaf_max
         g.xf = s->n_xf > 0 ? s->xf.as<const float4>() : nullptr;
         g.n_xf = s->n_xf;
         g.nodes = s->nodes.as<Node>();
-        g.geo = s->geo.as<float4>();
         g.shade = s->shade.as<float4>();
         g.perm = s->perm.as<int32_t>();
         g.codes_sorted = s->codes_sorted.as<uint32_t>();
@@ -1261,7 +1259,6 @@ eos_status build_lbvh_batch(eos_scene* const* scenes, int n_scenes, int leaf_max
             hipLaunchKernelGGL(k_bnodes, dim3(blocks(M, 256)), dim3(256), 0, S, kchild, fl, B.ibox.as<const float>(),
                                B.lbox.as<const float>(), B.cb.as<const float>(), T, o_node, nseg, Mi, leaf_max);
         }
-        hipLaunchKernelGGL(k_btris, dim3(blocks(N, 256)), dim3(256), 0, S, vS, T, o_tri, nseg, Ni, err);
         int32_t* flags = B.flags4.as<int32_t>();
         int32_t* idx = flags + M + 1;
         if (M > 0) {
@@ -1277,18 +1274,21 @@ eos_status build_lbvh_batch(eos_scene* const* scenes, int n_scenes, int leaf_max
                                B.counts.as<int32_t>());
             EOS_HIP(hipMemcpyAsync(cnt4.data(), B.counts.ptr, 8 * (size_t)nseg, hipMemcpyDeviceToHost, S));
             EOS_HIP(hipStreamSynchronize(S));
-            for (int k = 0; k < nseg; ++k) {
-                eos_scene* s = scenes[seg_scene[k]];
-                s->n_nodes4 = cnt4[2 * k];
-                EOS_TRY(s->nodes4.ensure(128 * (size_t)std::max(s->n_nodes4, 1)));
-                segs[k].nodes4 = s->nodes4.as<Node4>();
-                segs[k].base4 = cnt4[2 * k + 1];
-            }
-            EOS_HIP(hipMemcpyAsync(B.table.ptr, segs.data(), sizeof(BuildSeg) * nseg, hipMemcpyHostToDevice, S));
+        }
+        for (int k = 0; k < nseg; ++k) {
+            eos_scene* s = scenes[seg_scene[k]];
+            s->n_nodes4 = cnt4[2 * k];
+            EOS_TRY(s->tree.ensure(s->tree_bytes()));
+            segs[k].nodes4 = s->nodes4();
+            segs[k].geo = s->geo();
+            segs[k].base4 = cnt4[2 * k + 1];
+        }
+        EOS_HIP(hipMemcpyAsync(B.table.ptr, segs.data(), sizeof(BuildSeg) * nseg, hipMemcpyHostToDevice, S));
+        if (M > 0)
             hipLaunchKernelGGL(k_bnodes4, dim3(blocks(M, 256)), dim3(256), 0, S, kchild, fl, B.ibox.as<const float>(),
                                B.lbox.as<const float>(), B.cb.as<const float>(), flags, idx, T, o_node, nseg, Mi,
                                leaf_max);
-        }
+        hipLaunchKernelGGL(k_btris, dim3(blocks(N, 256)), dim3(256), 0, S, vS, T, o_tri, nseg, Ni, err);
         EOS_HIP(hipGetLastError());
         EOS_HIP(hipMemcpyAsync(herr, err, 12, hipMemcpyDeviceToHost, S));
     }

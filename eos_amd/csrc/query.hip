@@ -144,8 +144,10 @@ __global__ __launch_bounds__(kLinTile) void k_query_linear(int n, const float* r
 // The BVH traversal for caller-given rays: the default launch shape (256
 // threads, 16 LDS stack entries), the scene's tree width and transformations.
 template <int MODE>
-void launch_rays(int width, bool xf, int grid, hipStream_t s, const TraceArgs& a) {
-    if (width == 2) {
+void launch_rays(int width, bool xf, bool big, int grid, hipStream_t s, const TraceArgs& a) {
+    if (width == 4 && big) {
+        hipLaunchKernelGGL((k_trace<MODE, 256, 16, false, false, 4, true, false, true>), dim3(grid), dim3(256), 0, s, a);
+    } else if (width == 2) {
         if (xf) hipLaunchKernelGGL((k_trace<MODE, 256, 16, false, false, 2, true>), dim3(grid), dim3(256), 0, s, a);
         else hipLaunchKernelGGL((k_trace<MODE, 256, 16, false, false, 2, false>), dim3(grid), dim3(256), 0, s, a);
     } else {
@@ -233,7 +235,7 @@ eos_status trace_rays_static(eos_scene* s, int n, const float* o, const float* d
             if (xf) hipLaunchKernelGGL((k_trace<MODE_RAYS_ANY, 256, kMaxStack, false, false, 2, true>), dim3(grid), dim3(256), 0, S, a);
             else hipLaunchKernelGGL((k_trace<MODE_RAYS_ANY, 256, kMaxStack, false, false, 2, false>), dim3(grid), dim3(256), 0, S, a);
         } else {
-            launch_rays<MODE_RAYS_ANY>(4, xf, grid, S, a);
+            launch_rays<MODE_RAYS_ANY>(4, xf, s->tree_big(), grid, S, a);
         }
     } else {
         a.hit_out = rec;
@@ -241,10 +243,10 @@ eos_status trace_rays_static(eos_scene* s, int n, const float* o, const float* d
             if (xf) hipLaunchKernelGGL((k_trace<MODE_RAYS, 256, kMaxStack, false, false, 2, true>), dim3(grid), dim3(256), 0, S, a);
             else hipLaunchKernelGGL((k_trace<MODE_RAYS, 256, kMaxStack, false, false, 2, false>), dim3(grid), dim3(256), 0, S, a);
         } else {
-            launch_rays<MODE_RAYS>(4, xf, grid, S, a);
+            launch_rays<MODE_RAYS>(4, xf, s->tree_big(), grid, S, a);
         }
         hipLaunchKernelGGL(k_query_hits, dim3(blocks), dim3(256), 0, S, n, o, d, rec, s->shade.as<const float4>(),
-                           s->geo.as<const float4>(), xf ? s->xf.as<const float4>() : nullptr, out);
+                           s->geo(), xf ? s->xf.as<const float4>() : nullptr, out);
     }
     EOS_HIP(hipGetLastError());
     int err = 0;
@@ -321,13 +323,13 @@ eos_status trace_rays(eos_scene* s, int n, const float* o, const float* d, const
         a.ray_d = rd;
         if (mode == EOS_QUERY_OCCLUDED) {
             a.vis_out = occ_dev;
-            launch_rays<MODE_RAYS_ANY>(s->width, s->n_xf > 0, grid, S, a);
+            launch_rays<MODE_RAYS_ANY>(s->width, s->n_xf > 0, s->tree_big(), grid, S, a);
         } else {
             EOS_TRY(s->q_rec.ensure(16 * nn));
             a.hit_out = s->q_rec.as<float4>();
-            launch_rays<MODE_RAYS>(s->width, s->n_xf > 0, grid, S, a);
+            launch_rays<MODE_RAYS>(s->width, s->n_xf > 0, s->tree_big(), grid, S, a);
             hipLaunchKernelGGL(k_query_hits, dim3(blocks), dim3(256), 0, S, n, ro, rd, s->q_rec.as<const float4>(),
-                               s->shade.as<const float4>(), s->geo.as<const float4>(),
+                               s->shade.as<const float4>(), s->geo(),
                                s->n_xf > 0 ? s->xf.as<const float4>() : nullptr, out);
         }
         EOS_HIP(hipGetLastError());

@@ -672,22 +672,25 @@ __global__ __launch_bounds__(256) void k_cull_compact(CullArgs a) {
 // ---- traversal launch table ------------------------------------------------
 // 4-wide trees: every workgroup / LDS-stack configuration; binary trees: the
 // default configuration only (they exist for comparison and parity checks).
-// Scenes with transformations: the default configuration (256 threads, 16 LDS
-// stack entries), no packets; the frame sets its configuration to match.
+// Scenes with transformations, and scenes whose tree is past 4 GiB (big: 64-bit
+// addresses): the default configuration (256 threads, 16 LDS stack entries), no
+// packets; the frame sets its configuration to match.
 // lean (shadow rays, single scenes): the default configuration's kernel without
 // the group walk (less LDS per workgroup, for a launch that shares the GPU with
 // another stream's).
 template <int MODE, bool COUNT, bool BATCH>
-eos_status launch_trace(const LaunchCfg& cfg, int width, bool xf, int grid, hipStream_t s, const TraceArgs& a,
-                        bool lean) {
+eos_status launch_trace(const LaunchCfg& cfg, int width, bool xf, bool big, int grid, hipStream_t s,
+                        const TraceArgs& a, bool lean) {
 #define EOS_TRACE_CASE(WG, SL)                                                                             \
     case WG * 100 + SL:                                                                                     \
         hipLaunchKernelGGL((k_trace<MODE, WG, SL, COUNT, BATCH, 4, false>), dim3(grid), dim3(WG), 0, s, a); \
         break;
-    if (xf) {
+    if (xf || (big && width == 4)) {
         if (cfg.workgroup != 256 || cfg.stack_lds != 16 || cfg.packets)
             return fail(EOS_ERR_INVALID, "transformed scenes trace with the default launch configuration");
-        if (width == 2) hipLaunchKernelGGL((k_trace<MODE, 256, 16, COUNT, BATCH, 2, true>), dim3(grid), dim3(256), 0, s, a);
+        if (big && width == 4)
+            hipLaunchKernelGGL((k_trace<MODE, 256, 16, COUNT, BATCH, 4, true, false, true>), dim3(grid), dim3(256), 0, s, a);
+        else if (width == 2) hipLaunchKernelGGL((k_trace<MODE, 256, 16, COUNT, BATCH, 2, true>), dim3(grid), dim3(256), 0, s, a);
         else hipLaunchKernelGGL((k_trace<MODE, 256, 16, COUNT, BATCH, 4, true>), dim3(grid), dim3(256), 0, s, a);
     } else if (MODE == MODE_PRIMARY && width == 4 && cfg.packets) {
         hipLaunchKernelGGL((k_trace_packet<256, COUNT, BATCH>), dim3(std::max(1, grid * cfg.workgroup / 256)),
@@ -718,14 +721,6 @@ eos_status launch_trace(const LaunchCfg& cfg, int width, bool xf, int grid, hipS
     return EOS_OK;
 }
 
-template <int MODE>
-eos_status launch_trace_any(bool count, bool batch, int width, bool xf, const LaunchCfg& cfg, int grid, hipStream_t s,
-                            const TraceArgs& a, bool lean = false) {
-    if (batch) return launch_trace<MODE, false, true>(cfg, width, xf, grid, s, a, false);
-    return count ? launch_trace<MODE, true, false>(cfg, width, xf, grid, s, a, false)
-                 : launch_trace<MODE, false, false>(cfg, width, xf, grid, s, a, lean);
-}
-
 inline unsigned blocks_for(size_t n, unsigned t, unsigned cap) {
     size_t b = (n + t - 1) / t;
     if (b < 1) b = 1;
@@ -745,6 +740,7 @@ struct Frame {
     int lstride = 0;       // light slots per hit (max lights over the batch)
     int width = 4;         // tree width walked by the traversal
     bool xf = false;       // some triangle has a transformation
+    bool big = false;      // single scene: its tree is past 4 GiB
     bool tree = false;     // some material is transparent: rays may have two children
     AaSample aa;           // anti-aliasing sample of this frame (mode AA_NONE: plain frame)
     int row0 = 0, band_h = 0;  // single scene: camera rows [row0, row0 + band_h) of the frame
@@ -758,6 +754,13 @@ struct Frame {
     float* rgb = nullptr;
     int32_t* hits = nullptr;
 };
+
+template <int MODE>
+eos_status launch_trace_any(const Frame& f, int grid, hipStream_t s, const TraceArgs& a, bool lean = false) {
+    if (f.batch) return launch_trace<MODE, false, true>(f.cfg, f.width, f.xf, false, grid, s, a, false);
+    return f.count ? launch_trace<MODE, true, false>(f.cfg, f.width, f.xf, f.big, grid, s, a, false)
+                   : launch_trace<MODE, false, false>(f.cfg, f.width, f.xf, f.big, grid, s, a, lean);
+}
 
 // Overflow stack entries of one persistent traversal grid.
 size_t gstack_ints(const Frame& f, int trace_grid) {
@@ -901,7 +904,7 @@ eos_status enqueue_frame(eos_frame_buffers& fb, const Frame& f, const FrameStrea
             // workgroups room (hit-dense 4K frame 17.3 -> 16.5 ms, config E
             // 1.84 -> 1.80 ms); its launches are large, so the group walk would
             // not be taken there anyway
-            EOS_TRY(launch_trace_any<MODE_SHADOW>(f.count, f.batch, f.width, f.xf, f.cfg, trace_grid, st, sh,
+            EOS_TRY(launch_trace_any<MODE_SHADOW>(f, trace_grid, st, sh,
                                                   st != S));
         }
         F.s[2 * slot + 1] = rec(st);
@@ -1002,8 +1005,8 @@ eos_status enqueue_frame(eos_frame_buffers& fb, const Frame& f, const FrameStrea
             ta.count_mul = 64;
             ta.live = ca.live;
         }
-        if (l == 0) EOS_TRY(launch_trace_any<MODE_PRIMARY>(f.count, f.batch, f.width, f.xf, f.cfg, trace_grid, S, ta));
-        else EOS_TRY(launch_trace_any<MODE_QUEUE>(f.count, f.batch, f.width, f.xf, f.cfg, trace_grid, S, ta));
+        if (l == 0) EOS_TRY(launch_trace_any<MODE_PRIMARY>(f, trace_grid, S, ta));
+        else EOS_TRY(launch_trace_any<MODE_QUEUE>(f, trace_grid, S, ta));
         if (l == 0 && f.first_ev[1]) EOS_HIP(hipEventRecord(f.first_ev[1], S));
         F.c[2 * l + 1] = rec(S);
         SetupArgs sa{};
@@ -1190,12 +1193,13 @@ Frame make_frame(eos_scene* s, const eos_camera* camp, int depth, bool count, uc
     f.cfg = s->cfg;
     f.width = s->width;
     f.xf = s->n_xf > 0;
+    f.big = s->tree_big();
     f.tree = s->any_transparent;
-    if (count || f.width == 2 || f.xf) {
+    if (count || f.width == 2 || f.xf || f.big) {
         f.cfg.workgroup = 256;
         f.cfg.stack_lds = 16;
     }
-    if (f.xf) f.cfg.packets = 0;
+    if (f.xf || f.big) f.cfg.packets = 0;
     f.num_cu = s->num_cu;
     f.rgba = rgba_dev;
     f.rgb = rgb_dev;

@@ -63,6 +63,18 @@ __device__ __forceinline__ bool tile_pixel(int r, int tiles_x, int W, int H, int
     return x < W && y < H;
 }
 
+// 1.0f / x, correctly rounded: the hardware's estimate and one Newton step with
+// fused multiply-adds give the IEEE quotient for every x with 2^-126 <= |x| < 2^126
+// (all such floats checked against the division); larger ones divide.  Below
+// 2^-126 the value differs (the one caller rejects those determinants whatever
+// their reciprocal).  Three instructions instead of the division's eleven.
+__device__ __forceinline__ float reciprocal(float x) {
+    float r = __builtin_amdgcn_rcpf(x);
+    r = __builtin_fmaf(__builtin_fmaf(-x, r, 1.0f), r, r);
+    if (__builtin_expect(fabsf(x) >= 0x1p126f, 0)) r = 1.0f / x;
+    return r;
+}
+
 // src/Triangle.cpp:57-91 with e1 = v2 - v1, e2 = v3 - v1 precomputed (the same
 // float subtractions, done once at build time).  Branch-free: every quantity is
 // computed with the reference's operations and the reference's early-outs
@@ -73,7 +85,7 @@ __device__ __forceinline__ bool tile_pixel(int r, int tiles_x, int W, int H, int
 __device__ __forceinline__ bool moller_trumbore(F3 o, F3 d, F3 v1, F3 e1, F3 e2, float& t, float& u, float& v) {
     const F3 P = cross3(d, e2);
     const float det = dot3(e1, P);
-    const float inv = 1.0f / det;
+    const float inv = reciprocal(det);
     const F3 T = sub(o, v1);
     const F3 Q = cross3(T, e1);
     t = dot3(e2, Q) * inv;
@@ -313,6 +325,15 @@ __device__ __forceinline__ void cmpswap(float& ta, int& ka, int& ra, float& tb, 
     const int r0 = sw ? rb : ra, r1 = sw ? ra : rb;
     ta = t0; tb = t1;
     ka = k0; kb = k1;
+    ra = r0; rb = r1;
+}
+
+// Compare-exchange of (key, reference) pairs by key.
+__device__ __forceinline__ void keyswap(uint32_t& qa, int& ra, uint32_t& qb, int& rb) {
+    const bool sw = qb < qa;
+    const uint32_t q0 = sw ? qb : qa, q1 = sw ? qa : qb;
+    const int r0 = sw ? rb : ra, r1 = sw ? ra : rb;
+    qa = q0; qb = q1;
     ra = r0; rb = r1;
 }
 
@@ -984,32 +1005,16 @@ __device__ __forceinline__ void trace_group(const TraceArgs& a, int n, int32_t* 
     }
 }
 
-// Entries of a lane's traversal stack kept in registers, above the LDS and
-// global parts (0: the whole stack is in LDS / global memory).  Measured on the
-// 4K frame of the 4M-triangle sphere: 0 entries 2.18 ms for the primary launch,
-// 2 entries 2.23 ms, 4 entries 2.28 ms (VGPRs 86 -> 91, occupancy unchanged at
-// 5 waves per SIMD): the shifts of a register stack cost more issue slots under
-// divergence than the LDS read latency they save, which the other waves of the
-// SIMD already hide.
-#ifndef EOS_REG_STACK
-#define EOS_REG_STACK 0
-#endif
-constexpr int kRegStack = EOS_REG_STACK;
-
-// Node-step pushes while the lane's LDS stack has room: all slots written
+// Node-step pushes while the lane's LDS stack has room write all slots
 // without branches (measured on the 4K sphere frame: primary launch 1.61 ->
 // 1.57 ms).  Any-hit launches push hit children in slot order instead of
 // sorting them by entry distance: every box the ray meets is walked whatever
 // the order, so only the (rare) occluded rays can end sooner or later (hit-dense
 // 4K frame 19.4 -> 18.65 ms).  Both leave every result unchanged; launches that
 // count visits keep the sorted order.
-#ifndef EOS_FASTPUSH
-#define EOS_FASTPUSH 1
-#endif
 #ifndef EOS_ANY_NOSORT
 #define EOS_ANY_NOSORT 1
 #endif
-constexpr bool kFastPush = EOS_FASTPUSH != 0;
 // Idle lanes a wave needs before its walking lanes lend subtrees (measured,
 // frames identical: at 1, 16, 32, 48 idle lanes config C's single frame took
 // 2.21, 2.11, 2.11, 2.28 ms and config D's 64 sequential frames 102, 93, 84, 87 ms).
@@ -1019,67 +1024,74 @@ constexpr bool kFastPush = EOS_FASTPUSH != 0;
 constexpr int kStealIdle = EOS_STEAL_IDLE;
 constexpr bool kAnyNoSort = EOS_ANY_NOSORT != 0;
 
-// A lane's traversal stack: the top kRegStack entries in registers (r[0] the
-// top), the rest in LDS (STACK_LDS entries, column per lane) and then in the
-// lane's global overflow area.  The memory part is non-empty only while the
-// register part is full, so a pop takes its result from a register and refills
-// the register bottom from memory off the dependent chain (the value is needed
-// kRegStack pops later); a push spills the register bottom.  LIFO order is
-// the same as a memory-only stack, so every ray's walk is unchanged.
-template <int R, int WG, int STACK_LDS>
+// LDS in its own address space: a load whose address could be LDS or global
+// memory (the pop of a stack that overflows from one into the other) would
+// otherwise be merged into one flat load, which is slower than either and is
+// waited for on both counters.  (The host pass only type-checks kernel bodies.)
+#if defined(__HIP_DEVICE_COMPILE__)
+typedef __attribute__((address_space(3))) int32_t LdsInt;
+typedef __attribute__((address_space(3))) uint16_t LdsHalf;
+#else
+typedef int32_t LdsInt;
+typedef uint16_t LdsHalf;
+#endif
+
+// A lane's traversal stack: entries [base, sp), the first STACK_LDS in LDS (column
+// per lane), the rest in the lane's global overflow area.  KEYS: an entry in
+// LDS carries its box's entry distance, rounded down to the float's upper half,
+// so that a pop drops entries that lie behind the nearest hit found since they
+// were pushed without fetching their nodes.  Lending takes the entry at `base`;
+// the entries above keep their places, so the index of an entry is the one it
+// has in a walk that lends nothing and stays within the proven depth.
+template <int WG, int STACK_LDS, bool KEYS>
 struct LaneStack {
-    int r[R > 0 ? R : 1];
-    int nreg = 0, sp = 0;   // entries in registers, entries in memory
-    __device__ __forceinline__ void clear() { nreg = sp = 0; }
-    __device__ __forceinline__ int depth() const { return nreg + sp; }
-    __device__ __forceinline__ void mem_push(int32_t* lds, int32_t* gst, int tid, int v) {
-        if (sp < STACK_LDS) lds[sp * WG + tid] = v;
+    int sp = 0, base = 0;
+    __device__ __forceinline__ void clear() { sp = base = 0; }
+    __device__ __forceinline__ int depth() const { return sp - base; }
+    __device__ __forceinline__ bool lds_room(int k) const { return sp + k <= STACK_LDS; }
+    // slot j above the top, which lds_room has found to be in LDS
+    __device__ __forceinline__ void put(LdsInt* lds, LdsHalf* ldt, int tid, int j, int v, uint32_t key) {
+        lds[(sp + j) * WG + tid] = v;
+        if (KEYS) ldt[(sp + j) * WG + tid] = (uint16_t)(key >> 16);
+    }
+    __device__ __forceinline__ void push(LdsInt* lds, LdsHalf* ldt, int32_t* gst, int tid, int v, uint32_t key) {
+        if (sp < STACK_LDS) put(lds, ldt, tid, 0, v, key);
         else gst[sp - STACK_LDS] = v;
         ++sp;
     }
-    __device__ __forceinline__ int mem_pop(const int32_t* lds, const int32_t* gst, int tid) {
-        --sp;
-        return sp < STACK_LDS ? lds[sp * WG + tid] : gst[sp - STACK_LDS];
-    }
-    __device__ __forceinline__ void push(int32_t* lds, int32_t* gst, int tid, int v) {
-        if (R == 0) {
-            mem_push(lds, gst, tid, v);
-            return;
+    // Takes the top entry off.  v, key: the top entry if it is in LDS, read
+    // beforehand (peek); entries behind best_t are dropped (KEYS).
+    __device__ __forceinline__ int pop(const LdsInt* lds, const LdsHalf* ldt, const int32_t* gst, int tid, int v,
+                                       uint32_t key, float best_t) {
+        for (;;) {
+            if (sp == base) {
+                sp = base = 0;
+                return kDone;
+            }
+            --sp;
+            if (sp >= STACK_LDS) return gst[sp - STACK_LDS];
+            if (!KEYS || __uint_as_float(key << 16) <= best_t) return v;
+            const int q = (sp > 0 ? sp - 1 : 0) * WG + tid;
+            v = lds[q];
+            key = ldt[q];
         }
-        if (nreg == R) mem_push(lds, gst, tid, r[R - 1]);
-        else ++nreg;
-#pragma unroll
-        for (int k = R - 1; k > 0; --k) r[k] = r[k - 1];
-        r[0] = v;
     }
-    // the next node to visit, kDone when the stack is empty
-    __device__ __forceinline__ int pop(const int32_t* lds, const int32_t* gst, int tid) {
-        if (R == 0) return sp == 0 ? kDone : mem_pop(lds, gst, tid);
-        if (nreg == 0) return kDone;
-        const int top = r[0];
-#pragma unroll
-        for (int k = 0; k + 1 < R; ++k) r[k] = r[k + 1];
-        if (sp > 0) r[R - 1] = mem_pop(lds, gst, tid);
-        else --nreg;
-        return top;
+    // The top entry (anything if the stack is empty or the top is not in LDS),
+    // read at the start of a step: a step that pops has pushed nothing.
+    __device__ __forceinline__ void peek(const LdsInt* lds, const LdsHalf* ldt, int tid, int& v, uint32_t& key) const {
+        int q = sp - 1;
+        q = q < 0 ? 0 : (q >= STACK_LDS ? STACK_LDS - 1 : q);
+        v = lds[q * WG + tid];
+        key = KEYS ? ldt[q * WG + tid] : 0u;
     }
-    // Memory-only stacks (R == 0): room for k more entries in LDS; the slot j
-    // above the top; k more entries on the stack (written with put first).
-    __device__ __forceinline__ bool lds_room(int k) const { return R == 0 && sp + k <= STACK_LDS; }
-    __device__ __forceinline__ void put(int32_t* lds, int tid, int j, int v) { lds[(sp + j) * WG + tid] = v; }
-    __device__ __forceinline__ void grow(int k) { sp += k; }
     // Removes and returns the bottom entry (the oldest: the farthest sibling
-    // pushed nearest the root, usually the largest pending subtree); the
-    // entries above move down one place, keeping their order.  depth() > 0,
-    // memory-only stacks (R == 0).
-    __device__ __forceinline__ int take_bottom(int32_t* lds, int32_t* gst, int tid) {
-        const int v = STACK_LDS > 0 ? lds[tid] : gst[0];
-        for (int j = 1; j < sp; ++j) {
-            const int x = j < STACK_LDS ? lds[j * WG + tid] : gst[j - STACK_LDS];
-            if (j - 1 < STACK_LDS) lds[(j - 1) * WG + tid] = x;
-            else gst[j - 1 - STACK_LDS] = x;
-        }
-        --sp;
+    // pushed nearest the root, usually the largest pending subtree).  depth() > 0.
+    __device__ __forceinline__ int take_bottom(const LdsInt* lds, const int32_t* gst, int tid) {
+        int v;
+        if (base < STACK_LDS) v = lds[base * WG + tid];
+        else v = gst[base - STACK_LDS];
+        ++base;
+        if (base == sp) sp = base = 0;
         return v;
     }
 };
@@ -1099,17 +1111,20 @@ struct LaneStack {
 // triangle's local space.  LEAN: no group walk, and so no LDS for its stacks
 // (24 instead of 32 KiB per 256-thread workgroup), for a launch that runs
 // beside another stream's launches.
-template <int MODE, int WG, int STACK_LDS, bool COUNT, bool BATCH, int WIDTH, bool XF, bool LEAN = false>
-__global__ __launch_bounds__(WG) void k_trace(TraceArgs a) {
+template <int MODE, int WG, int STACK_LDS, bool COUNT, bool BATCH, int WIDTH, bool XF, bool LEAN = false,
+          bool A64 = BATCH>
+__global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(XF ? 4 : 5))) void k_trace(TraceArgs a) {
     constexpr bool ANY = any_hit_mode(MODE);
     constexpr int MAXS = max_stack<WIDTH>();
-    constexpr int LDS_LANE = STACK_LDS * WG, LDS_COOP = WIDTH == 4 ? (WG / 4) * kMaxStack4 : 0;
+    // closest-hit walks keep the entry distance of every stack entry (16 bits each)
+    constexpr bool KEYS = WIDTH == 4 && !ANY && !COUNT;
+    constexpr int LDS_LANE = STACK_LDS * WG + (KEYS ? STACK_LDS * WG / 2 : 0), LDS_COOP = WIDTH == 4 ? (WG / 4) * kMaxStack4 : 0;
     // the group walk serves the short launches after the primary rays, never the
     // primary launch, and not batched frames, whose launches hold every scene's
     // rays (its LDS stacks, 32 KiB per workgroup, cost a batched frame 4%)
     constexpr bool GROUP = WIDTH == 4 && !COUNT && MODE != MODE_PRIMARY && !BATCH && !LEAN;
     // work stealing visits nodes in another order (never in launches that count visits)
-    constexpr bool STEAL = !COUNT && kRegStack == 0;
+    constexpr bool STEAL = !COUNT;
     constexpr int LDS_GROUP = GROUP ? (WG / 64) * kWaveGroupStack : 0;
     constexpr int LDS_A = LDS_LANE > LDS_COOP ? LDS_LANE : LDS_COOP;
     __shared__ int32_t lds[LDS_A > LDS_GROUP ? LDS_A : LDS_GROUP];
@@ -1144,10 +1159,15 @@ __global__ __launch_bounds__(WG) void k_trace(TraceArgs a) {
         trace_coop<MODE, WG, COUNT, BATCH, XF>(a, n, lds + (tid >> 6) * 16 * kMaxStack4, visits, tests);
     } else {
         int32_t* gst = a.gstack + (size_t)(blockIdx.x * WG + tid) * (MAXS - STACK_LDS);
+        LdsInt* const sref = (LdsInt*)lds;
+        LdsHalf* const skey = (LdsHalf*)(lds + STACK_LDS * WG);
         const Node* __restrict__ nodes = a.sc.nodes;
         const Node4* __restrict__ nodes4 = a.sc.nodes4;
         const float4* __restrict__ geo = a.sc.geo;
         const float4* __restrict__ xf = a.sc.xf;
+        // the 4-wide nodes and the geometry records lie in one allocation
+        const char* const tree = reinterpret_cast<const char*>(a.sc.nodes4);
+        const uint32_t geo_off = (uint32_t)(reinterpret_cast<const char*>(a.sc.geo) - tree);
         int item = -1;
         size_t out_idx = 0;
         Fetch f = fetch_start(a, n);
@@ -1159,10 +1179,10 @@ __global__ __launch_bounds__(WG) void k_trace(TraceArgs a) {
         float best_t = INFINITY, bu = 0.0f, bv = 0.0f;
         int best_slot = -1, best_orig = 0x7FFFFFFF;
         int cur = kDone;
-        LaneStack<kRegStack, WG, STACK_LDS> stk;
+        LaneStack<WG, STACK_LDS, KEYS> stk;
         int lpos = -1;   // next triangle of the current leaf (-1: not in a leaf)
         bool farf = false;   // any hit: walk the farthest hit child first (RayItem::far_first)
-        int sgx = 0, sgy = 0, sgz = 0;   // 1 where the inverse direction is negative (hi plane nearer)
+        int sgx = 0, sgy = 0, sgz = 0;   // 16 (bytes) where the inverse direction is negative (hi plane nearer)
         int budget = 0;  // node visits left for this ray: a tree visits each internal node at most once
         // XF: the ray in the local space of transformation lxi, kept while the
         // walk stays among that transformation's triangles (-1: none yet)
@@ -1213,9 +1233,9 @@ __global__ __launch_bounds__(WG) void k_trace(TraceArgs a) {
                     px = o.x * ix;
                     py = o.y * iy;
                     pz = o.z * iz;
-                    sgx = ix < 0.0f ? 1 : 0;
-                    sgy = iy < 0.0f ? 1 : 0;
-                    sgz = iz < 0.0f ? 1 : 0;
+                    sgx = ix < 0.0f ? 16 : 0;
+                    sgy = iy < 0.0f ? 16 : 0;
+                    sgz = iz < 0.0f ? 16 : 0;
                     best_t = INFINITY;
                     best_slot = -1;
                     best_orig = 0x7FFFFFFF;
@@ -1252,39 +1272,72 @@ __global__ __launch_bounds__(WG) void k_trace(TraceArgs a) {
                     }
                 }
                 if (item >= 0) {
-                    if (cur >= 0 && cur != kDone && --budget < 0) {
-                        atomicOr(a.err, 2);
-                        cur = kDone;
-                    } else if (cur >= 0 && cur != kDone) {
-                        if (COUNT) ++visits;
-                        const float tmax = ANY ? INFINITY : best_t;
-                        if (WIDTH == 4) {
-                            // the near and far planes of each axis fetched by the ray's
-                            // direction signs (float4 0/1: x lo/hi, 2/3: y, 4/5: z);
-                            // batched frames keep the plain test (measured faster there)
-                            const float4* nd = reinterpret_cast<const float4*>(nodes4 + cur);
-                            const int4 rf = reinterpret_cast<const int4*>(nd)[6];
-                            float t0, t1, t2, t3;
-                            bool h0, h1, h2, h3;
-                            // all four tests unconditionally (no load sinking), empty slots masked after
-                            if (BATCH) {
-                                const float4 lx = nd[0], hx = nd[1], ly = nd[2], hy = nd[3], lz = nd[4], hz = nd[5];
-                                h0 = slab(lx.x, hx.x, ly.x, hy.x, lz.x, hz.x, ix, iy, iz, px, py, pz, tmax, t0) & (rf.x != kEmpty);
-                                h1 = slab(lx.y, hx.y, ly.y, hy.y, lz.y, hz.y, ix, iy, iz, px, py, pz, tmax, t1) & (rf.y != kEmpty);
-                                h2 = slab(lx.z, hx.z, ly.z, hy.z, lz.z, hz.z, ix, iy, iz, px, py, pz, tmax, t2) & (rf.z != kEmpty);
-                                h3 = slab(lx.w, hx.w, ly.w, hy.w, lz.w, hz.w, ix, iy, iz, px, py, pz, tmax, t3) & (rf.w != kEmpty);
+                    bool pop = false;
+                    int top;
+                    uint32_t topkey;
+                    stk.peek(sref, skey, tid, top, topkey);
+                    // One fetch serves the lanes at a node and the lanes at a leaf:
+                    // 112 bytes of the node, or the 96 bytes of a pair of triangle
+                    // records, which lie next to each other (the last triangle of an odd
+                    // leaf is fetched twice).  Fetched each in its own branch, a step of a
+                    // wave with lanes at both would wait for memory twice.
+                    const bool inner = cur >= 0;   // kDone: a home waiting for its helpers
+                    const bool walk = cur != kDone;
+                    float4 g0, g1, g2, g3, g4, g5;
+                    int4 rf = make_int4(kEmpty, kEmpty, kEmpty, kEmpty);
+                    int s0 = 0, last = 0;
+                    if (WIDTH == 4) {
+                        if (walk) {
+                            // inner: the near and far planes of each axis by the ray's direction
+                            // signs; A64: per-lane pointers, else 32-bit offsets from the tree's base
+                            const int ox = inner ? sgx : 0, oy = inner ? sgy : 0, oz = inner ? sgz : 0;
+                            const int e = ~cur;
+                            const int first = e & ((1 << kLeafShift) - 1);
+                            last = first + ((e >> kLeafShift) & 7);
+                            s0 = lpos < 0 ? first : lpos;
+                            const int second = inner || s0 < last ? 48 : 0;
+                            auto fetch = [&](auto at) {
+                                g0 = at(ox);
+                                g1 = at(16 - ox);
+                                g2 = at(32 + oy);
+                                g3 = at(second - oy);
+                                g4 = at(16 + second + oz);
+                                g5 = at(32 + second - oz);
+                                if (inner) {
+                                    const float4 r = at(96);
+                                    rf = make_int4(__float_as_int(r.x), __float_as_int(r.y), __float_as_int(r.z),
+                                                   __float_as_int(r.w));
+                                }
+                            };
+                            if constexpr (A64) {
+                                const char* p = inner ? reinterpret_cast<const char*>(nodes4 + cur)
+                                                      : reinterpret_cast<const char*>(geo + 3 * (size_t)s0);
+                                fetch([p](int off) { return *reinterpret_cast<const float4*>(p + off); });
                             } else {
-                                const float4 nx = nd[sgx], fx = nd[1 - sgx], ny = nd[2 + sgy], fy = nd[3 - sgy],
-                                             nz = nd[4 + sgz], fz = nd[5 - sgz];
-                                h0 = slab_nf(nx.x, fx.x, ny.x, fy.x, nz.x, fz.x, ix, iy, iz, px, py, pz, tmax, t0) & (rf.x != kEmpty);
-                                h1 = slab_nf(nx.y, fx.y, ny.y, fy.y, nz.y, fz.y, ix, iy, iz, px, py, pz, tmax, t1) & (rf.y != kEmpty);
-                                h2 = slab_nf(nx.z, fx.z, ny.z, fy.z, nz.z, fz.z, ix, iy, iz, px, py, pz, tmax, t2) & (rf.z != kEmpty);
-                                h3 = slab_nf(nx.w, fx.w, ny.w, fy.w, nz.w, fz.w, ix, iy, iz, px, py, pz, tmax, t3) & (rf.w != kEmpty);
+                                const uint32_t b = inner ? (uint32_t)cur << 7 : geo_off + 48u * (uint32_t)s0;
+                                fetch([tree, b](int off) {
+                                    return *reinterpret_cast<const float4*>(tree + (uint32_t)(b + (uint32_t)off));
+                                });
                             }
+                        }
+                    }
+                    if (inner && walk) {
+                        const float tmax = ANY ? INFINITY : best_t;
+                        if (COUNT) ++visits;
+                        if (--budget < 0) {
+                            atomicOr(a.err, 2);
+                            cur = kDone;
+                        } else if (WIDTH == 4) {
+                            float t0, t1, t2, t3;
+                            // all four tests unconditionally, empty slots masked after
+                            const bool h0 = slab_nf(g0.x, g1.x, g2.x, g3.x, g4.x, g5.x, ix, iy, iz, px, py, pz, tmax, t0) & (rf.x != kEmpty);
+                            const bool h1 = slab_nf(g0.y, g1.y, g2.y, g3.y, g4.y, g5.y, ix, iy, iz, px, py, pz, tmax, t1) & (rf.y != kEmpty);
+                            const bool h2 = slab_nf(g0.z, g1.z, g2.z, g3.z, g4.z, g5.z, ix, iy, iz, px, py, pz, tmax, t2) & (rf.z != kEmpty);
+                            const bool h3 = slab_nf(g0.w, g1.w, g2.w, g3.w, g4.w, g5.w, ix, iy, iz, px, py, pz, tmax, t3) & (rf.w != kEmpty);
                             const int nh = (int)h0 + (int)h1 + (int)h2 + (int)h3;
                             if (nh == 0) {
-                                cur = stk.pop(lds, gst, tid);
-                            } else if (stk.depth() + nh - 1 > MAXS) {
+                                pop = true;
+                            } else if (!stk.lds_room(4) && stk.sp + nh - 1 > MAXS) {
                                 atomicOr(a.err, 1);
                                 cur = kDone;
                             } else if (ANY && !COUNT && kAnyNoSort && !farf && stk.lds_room(4)) {
@@ -1293,46 +1346,63 @@ __global__ __launch_bounds__(WG) void k_trace(TraceArgs a) {
                                 // in slot order (non-hits to a slot above the new top)
                                 const int c1 = (int)h0, c2 = c1 + (int)h1, c3 = c2 + (int)h2;
                                 cur = h0 ? rf.x : (h1 ? rf.y : (h2 ? rf.z : rf.w));
-                                stk.put(lds, tid, h1 && c1 >= 1 ? c1 - 1 : 3, rf.y);
-                                stk.put(lds, tid, h2 && c2 >= 1 ? c2 - 1 : 3, rf.z);
-                                stk.put(lds, tid, h3 && c3 >= 1 ? c3 - 1 : 3, rf.w);
-                                stk.grow(nh - 1);
+                                stk.put(sref, skey, tid, h1 && c1 >= 1 ? c1 - 1 : 3, rf.y, 0u);
+                                stk.put(sref, skey, tid, h2 && c2 >= 1 ? c2 - 1 : 3, rf.z, 0u);
+                                stk.put(sref, skey, tid, h3 && c3 >= 1 ? c3 - 1 : 3, rf.w, 0u);
+                                stk.sp += nh - 1;
                             } else {
-                                float e0 = h0 ? t0 : INFINITY, e1 = h1 ? t1 : INFINITY, e2 = h2 ? t2 : INFINITY,
-                                      e3 = h3 ? t3 : INFINITY;
-                                int k0 = 0, k1 = 1, k2 = 2, k3 = 3;
                                 int r0 = rf.x, r1 = rf.y, r2 = rf.z, r3 = rf.w;
-                                cmpswap(e0, k0, r0, e1, k1, r1);
-                                cmpswap(e2, k2, r2, e3, k3, r3);
-                                cmpswap(e0, k0, r0, e2, k2, r2);
-                                cmpswap(e1, k1, r1, e3, k3, r3);
-                                cmpswap(e1, k1, r1, e2, k2, r2);
+                                uint32_t q0, q1, q2, q3;
+                                if (COUNT) {
+                                    // the counted order: (entry distance, slot)
+                                    float e0 = h0 ? t0 : INFINITY, e1 = h1 ? t1 : INFINITY, e2 = h2 ? t2 : INFINITY,
+                                          e3 = h3 ? t3 : INFINITY;
+                                    int k0 = 0, k1 = 1, k2 = 2, k3 = 3;
+                                    cmpswap(e0, k0, r0, e1, k1, r1);
+                                    cmpswap(e2, k2, r2, e3, k3, r3);
+                                    cmpswap(e0, k0, r0, e2, k2, r2);
+                                    cmpswap(e1, k1, r1, e3, k3, r3);
+                                    cmpswap(e1, k1, r1, e2, k2, r2);
+                                    q0 = q1 = q2 = q3 = 0u;
+                                } else {
+                                    // by entry distance; a distance is not negative, so its bits
+                                    // order as unsigned integers
+                                    q0 = h0 ? __float_as_uint(t0) : 0xFFFFFFFFu;
+                                    q1 = h1 ? __float_as_uint(t1) : 0xFFFFFFFFu;
+                                    q2 = h2 ? __float_as_uint(t2) : 0xFFFFFFFFu;
+                                    q3 = h3 ? __float_as_uint(t3) : 0xFFFFFFFFu;
+                                    keyswap(q0, r0, q1, r1);
+                                    keyswap(q2, r2, q3, r3);
+                                    keyswap(q0, r0, q2, r2);
+                                    keyswap(q1, r1, q3, r3);
+                                    keyswap(q1, r1, q2, r2);
+                                }
                                 if (ANY && !COUNT && farf) {
                                     // farthest hit child next; the nearer ones pushed nearest
                                     // first, so the next farthest is popped next
                                     const int far = nh > 3 ? r3 : (nh > 2 ? r2 : (nh > 1 ? r1 : r0));
-                                    if (kFastPush && stk.lds_room(3)) {
-                                        stk.put(lds, tid, 0, r0);
-                                        stk.put(lds, tid, 1, r1);
-                                        stk.put(lds, tid, 2, r2);
-                                        stk.grow(nh - 1);
+                                    if (stk.lds_room(3)) {
+                                        stk.put(sref, skey, tid, 0, r0, 0u);
+                                        stk.put(sref, skey, tid, 1, r1, 0u);
+                                        stk.put(sref, skey, tid, 2, r2, 0u);
+                                        stk.sp += nh - 1;
                                     } else {
-                                        if (nh > 1) stk.push(lds, gst, tid, r0);
-                                        if (nh > 2) stk.push(lds, gst, tid, r1);
-                                        if (nh > 3) stk.push(lds, gst, tid, r2);
+                                        if (nh > 1) stk.push(sref, skey, gst, tid, r0, 0u);
+                                        if (nh > 2) stk.push(sref, skey, gst, tid, r1, 0u);
+                                        if (nh > 3) stk.push(sref, skey, gst, tid, r2, 0u);
                                     }
                                     r0 = far;
-                                } else if (kFastPush && stk.lds_room(3)) {
+                                } else if (stk.lds_room(3)) {
                                     // farthest first, all three slots written (those above
                                     // the new top are overwritten later)
-                                    stk.put(lds, tid, 0, nh > 3 ? r3 : (nh > 2 ? r2 : r1));
-                                    stk.put(lds, tid, 1, nh > 3 ? r2 : r1);
-                                    stk.put(lds, tid, 2, r1);
-                                    stk.grow(nh - 1);
+                                    stk.put(sref, skey, tid, 0, nh > 3 ? r3 : (nh > 2 ? r2 : r1), nh > 3 ? q3 : (nh > 2 ? q2 : q1));
+                                    stk.put(sref, skey, tid, 1, nh > 3 ? r2 : r1, nh > 3 ? q2 : q1);
+                                    stk.put(sref, skey, tid, 2, r1, q1);
+                                    stk.sp += nh - 1;
                                 } else {
-                                    if (nh > 3) stk.push(lds, gst, tid, r3);
-                                    if (nh > 2) stk.push(lds, gst, tid, r2);
-                                    if (nh > 1) stk.push(lds, gst, tid, r1);
+                                    if (nh > 3) stk.push(sref, skey, gst, tid, r3, q3);
+                                    if (nh > 2) stk.push(sref, skey, gst, tid, r2, q2);
+                                    if (nh > 1) stk.push(sref, skey, gst, tid, r1, q1);
                                 }
                                 cur = r0;
                             }
@@ -1346,11 +1416,11 @@ __global__ __launch_bounds__(WG) void k_trace(TraceArgs a) {
                             if (h0 && h1) {
                                 const bool swap = t1 < t0;
                                 const int nearc = swap ? c.y : c.x, farc = swap ? c.x : c.y;
-                                if (stk.depth() >= MAXS) {
+                                if (stk.sp >= MAXS) {
                                     atomicOr(a.err, 1);
                                     cur = kDone;
                                 } else {
-                                    stk.push(lds, gst, tid, farc);
+                                    stk.push(sref, skey, gst, tid, farc, 0u);
                                     cur = nearc;
                                 }
                             } else if (h0) {
@@ -1358,75 +1428,79 @@ __global__ __launch_bounds__(WG) void k_trace(TraceArgs a) {
                             } else if (h1) {
                                 cur = c.y;
                             } else {
-                                cur = stk.pop(lds, gst, tid);
+                                pop = true;
                             }
                         }
-                    } else if (cur != kDone) {
+                    } else if (walk) {
                         // One pair of triangles per step (a longer leaf takes several
                         // steps, so leaf steps cost about what node steps cost and the
-                        // lanes of a wave diverge less); both triangles are fetched
-                        // before either is tested; an odd leaf tests its last triangle
-                        // twice (same result, counted once).
-                        const int e = ~cur;
-                        const int first = e & ((1 << kLeafShift) - 1);
-                        const int cnt = ((e >> kLeafShift) & 7) + 1;
+                        // lanes of a wave diverge less); an odd leaf tests its last
+                        // triangle twice (same result, counted once).
+                        if (WIDTH != 4) {
+                            const int e = ~cur;
+                            const int first = e & ((1 << kLeafShift) - 1);
+                            last = first + ((e >> kLeafShift) & 7);
+                            s0 = lpos < 0 ? first : lpos;
+                            const float4* p = geo + 3 * (size_t)s0;
+                            const float4* r = s0 < last ? p + 3 : p;
+                            g0 = p[0];
+                            g1 = p[1];
+                            g2 = p[2];
+                            g3 = r[0];
+                            g4 = r[1];
+                            g5 = r[2];
+                        }
                         bool occluded = false;
-                        const int last = first + cnt - 1;
-                        {
-                            const int s0 = lpos < 0 ? first : lpos;
-                            const int s1 = s0 + 1 <= last ? s0 + 1 : s0;
-                            lpos = s0 + 2 <= last ? s0 + 2 : -1;
-                            const float4 a0 = geo[3 * (size_t)s0], a1 = geo[3 * (size_t)s0 + 1], a2 = geo[3 * (size_t)s0 + 2];
-                            const float4 b0 = geo[3 * (size_t)s1], b1 = geo[3 * (size_t)s1 + 1], b2 = geo[3 * (size_t)s1 + 2];
-                            float ta, ua, va, tb, ub, vb;
-                            F3 oa = o, da = d, ob = o, db = d;
-                            if (XF) {
-                                const int xa = __float_as_int(a2.z), xb = __float_as_int(b2.z);
-                                if (xa >= 0 && xa != lxi) {
-                                    lo_o = o;
-                                    lo_d = d;
-                                    to_local<XF>(xf, xa, lo_o, lo_d);
-                                    lxi = xa;
-                                }
-                                if (xa >= 0) {
-                                    oa = lo_o;
-                                    da = lo_d;
-                                }
-                                if (xb >= 0 && xb != lxi) {
-                                    lo_o = o;
-                                    lo_d = d;
-                                    to_local<XF>(xf, xb, lo_o, lo_d);
-                                    lxi = xb;
-                                }
-                                if (xb >= 0) {
-                                    ob = lo_o;
-                                    db = lo_d;
-                                }
+                        const bool two = s0 < last;
+                        lpos = s0 + 2 <= last ? s0 + 2 : -1;
+                        float ta, ua, va, tb, ub, vb;
+                        F3 oa = o, da = d, ob = o, db = d;
+                        if (XF) {
+                            const int xa = __float_as_int(g2.z), xb = __float_as_int(g5.z);
+                            if (xa >= 0 && xa != lxi) {
+                                lo_o = o;
+                                lo_d = d;
+                                to_local<XF>(xf, xa, lo_o, lo_d);
+                                lxi = xa;
                             }
-                            const bool ha = moller_trumbore(oa, da, f3(a0.x, a0.y, a0.z), f3(a0.w, a1.x, a1.y),
-                                                            f3(a1.z, a1.w, a2.x), ta, ua, va);
-                            const bool hb = moller_trumbore(ob, db, f3(b0.x, b0.y, b0.z), f3(b0.w, b1.x, b1.y),
-                                                            f3(b1.z, b1.w, b2.x), tb, ub, vb);
-                            // counted as the one-at-a-time walk would: an any-hit ray stops at its first hit
-                            if (COUNT) tests += (ANY && ha) ? 1 : (s1 != s0 ? 2 : 1);
-                            if (ANY) {
-                                if (ha | hb) occluded = true;
-                            } else {
-                                const int oa = __float_as_int(a2.y), ob = __float_as_int(b2.y);
-                                if (ha && (ta < best_t || (ta == best_t && oa < best_orig))) {
-                                    best_t = ta;
-                                    best_orig = oa;
-                                    best_slot = s0;
-                                    bu = ua;
-                                    bv = va;
-                                }
-                                if (hb && (tb < best_t || (tb == best_t && ob < best_orig))) {
-                                    best_t = tb;
-                                    best_orig = ob;
-                                    best_slot = s1;
-                                    bu = ub;
-                                    bv = vb;
-                                }
+                            if (xa >= 0) {
+                                oa = lo_o;
+                                da = lo_d;
+                            }
+                            if (xb >= 0 && xb != lxi) {
+                                lo_o = o;
+                                lo_d = d;
+                                to_local<XF>(xf, xb, lo_o, lo_d);
+                                lxi = xb;
+                            }
+                            if (xb >= 0) {
+                                ob = lo_o;
+                                db = lo_d;
+                            }
+                        }
+                        const bool ha = moller_trumbore(oa, da, f3(g0.x, g0.y, g0.z), f3(g0.w, g1.x, g1.y),
+                                                        f3(g1.z, g1.w, g2.x), ta, ua, va);
+                        const bool hb = moller_trumbore(ob, db, f3(g3.x, g3.y, g3.z), f3(g3.w, g4.x, g4.y),
+                                                        f3(g4.z, g4.w, g5.x), tb, ub, vb);
+                        // counted as the one-at-a-time walk would: an any-hit ray stops at its first hit
+                        if (COUNT) tests += (ANY && ha) ? 1 : (two ? 2 : 1);
+                        if (ANY) {
+                            if (ha | hb) occluded = true;
+                        } else {
+                            const int og_a = __float_as_int(g2.y), og_b = __float_as_int(g5.y);
+                            if (ha && (ta < best_t || (ta == best_t && og_a < best_orig))) {
+                                best_t = ta;
+                                best_orig = og_a;
+                                best_slot = s0;
+                                bu = ua;
+                                bv = va;
+                            }
+                            if (hb && (tb < best_t || (tb == best_t && og_b < best_orig))) {
+                                best_t = tb;
+                                best_orig = og_b;
+                                best_slot = two ? s0 + 1 : s0;
+                                bu = ub;
+                                bv = vb;
                             }
                         }
                         if (ANY && occluded) {
@@ -1434,9 +1508,10 @@ __global__ __launch_bounds__(WG) void k_trace(TraceArgs a) {
                             lpos = -1;
                             cur = kDone;
                         } else if (lpos < 0) {
-                            cur = stk.pop(lds, gst, tid);
+                            pop = true;
                         }
                     }
+                    if (pop) cur = stk.pop(sref, skey, gst, tid, top, topkey, best_t);
                     if (cur == kDone) {
                         if (STEAL && home >= 0) fin = true;   // merged below
                         else if (!STEAL || pending == 0 || (ANY && best_slot >= 0)) emit();
@@ -1493,7 +1568,7 @@ __global__ __launch_bounds__(WG) void k_trace(TraceArgs a) {
                         const bool donor = ((dm >> lane) & 1) && __popcll(dm & lanemask_lt()) < np;
                         const int src = thief ? nth_set_bit(dm, irank) : lane;
                         int give = kDone;
-                        if (donor) give = stk.take_bottom(lds, gst, tid);
+                        if (donor) give = stk.take_bottom(sref, gst, tid);
                         const int g_ref = __shfl(give, src), g_item = __shfl(item, src);
                         const int g_home = __shfl(home >= 0 ? home : lane, src);
                         const float g_ox = __shfl(o.x, src), g_oy = __shfl(o.y, src), g_oz = __shfl(o.z, src);
@@ -1526,9 +1601,9 @@ __global__ __launch_bounds__(WG) void k_trace(TraceArgs a) {
                             px = o.x * ix;
                             py = o.y * iy;
                             pz = o.z * iz;
-                            sgx = ix < 0.0f ? 1 : 0;
-                            sgy = iy < 0.0f ? 1 : 0;
-                            sgz = iz < 0.0f ? 1 : 0;
+                            sgx = ix < 0.0f ? 16 : 0;
+                            sgy = iy < 0.0f ? 16 : 0;
+                            sgz = iz < 0.0f ? 16 : 0;
                             // only hits better than the lender's best so far count
                             best_t = g_t;
                             best_orig = g_orig;
