@@ -9,8 +9,8 @@
 // MODE_RAYS / MODE_RAYS_ANY modes, rays read straight from the caller's
 // arrays), then one thread per ray turns the hit record into the reference's
 // RayIntersection fields with the same arithmetic the frame's set-up kernel
-// uses.  The linear query tests every triangle in index order, workgroup tiles
-// of triangles staged in LDS and read by every lane as broadcasts.
+// uses.  The linear query tests every triangle, split into chunks whose results
+// combine in index order.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -59,86 +59,263 @@ __global__ __launch_bounds__(256) void k_query_hits(int n, const float* ro, cons
 
 constexpr int kLinTile = 256;
 
-// src/Scene.cpp:159-201.  For each triangle in index order: the ray in the
-// triangle's local space, Moller-Trumbore (src/Triangle.cpp:26-91) against the
-// running distance the reference passes as Triangle::hit's `distance`
-// (minTemp: a hit farther than the last accepted one is rejected; the first
-// hit is always accepted, the reading of its uninitialised start value), and
-// the hit is kept when t < minDist (999999 at first) and t > 0.  found: some
-// triangle accepted a hit (the query's return value), even when none was kept.
-// The kept hit's point goes through M and its normal through transpose(inverse)
-// without a second normalisation.  verts / normals / matidx / xfi are the
-// scene's triangles in their original order.
-__global__ __launch_bounds__(kLinTile) void k_query_linear(int n, const float* ro, const float* rd, int n_tri,
-                                                            const float* verts, const float* normals,
-                                                            const int32_t* matidx, const int32_t* xfi,
-                                                            const float4* xf, float4* out) {
-    __shared__ float tv[9][kLinTile];   // component-major: lane j of the staging writes word j of each row
-    __shared__ int32_t tx[kLinTile];
-    const int i = blockIdx.x * kLinTile + (int)threadIdx.x;
-    const bool act = i < n;
-    F3 o = {0, 0, 0}, d = {0, 0, 0};
-    if (act) {
-        o = f3(ro[3 * (size_t)i], ro[3 * (size_t)i + 1], ro[3 * (size_t)i + 2]);
-        d = f3(rd[3 * (size_t)i], rd[3 * (size_t)i + 1], rd[3 * (size_t)i + 2]);
-    }
-    float min_temp = INFINITY, min_dist = 999999.0f, bu = 0.0f, bv = 0.0f;
-    bool found = false;
+// src/Scene.cpp:159-201 in parallel.  The reference walks the triangles in index
+// order with two running bounds: Triangle::hit's `distance` (minTemp: a hit
+// farther than the last accepted one is rejected; the first hit is always
+// accepted, the reading of its uninitialised start value) and minDist (999999
+// at first): an accepted hit is kept when 0 < t < minDist.  found: some triangle
+// accepted a hit (the query's return value), even when none was kept.
+//   While no accepted hit had t = 0, minDist <= minTemp, so a hit is kept when
+// 0 < t < minDist; after a hit at t = 0 nothing is kept any more.  So a run of
+// consecutive triangles is summed up by its first least t in (0, 999999) before
+// its first hit at t = 0, and two neighbouring runs combine in order.  Only a
+// hit whose t is not a number (a NaN passes Moller-Trumbore's comparisons, and
+// lifts both bounds) does not fit: it is flagged, and its ray is walked again in
+// index order.
+struct LinRun {
+    float t = 999999.0f, u = 0.0f, v = 0.0f;
     int best = -1;
+    bool found = false, zero = false, nan = false;
+    __device__ __forceinline__ void hit(float ht, float hu, float hv, int tri) {
+        found = true;
+        if (!(ht == ht)) nan = true;
+        if (!zero && ht < t && ht > 0.0f) {
+            t = ht;
+            u = hu;
+            v = hv;
+            best = tri;
+        }
+        zero |= ht <= 0.0f;
+    }
+    // this run, then the one of the triangles after it
+    __device__ __forceinline__ void then(const LinRun& o) {
+        if (!zero && o.t < t) {
+            t = o.t;
+            u = o.u;
+            v = o.v;
+            best = o.best;
+        }
+        found |= o.found;
+        zero |= o.zero;
+        nan |= o.nan;
+    }
+    // 16 bytes in memory: t, u, v, then the triangle + 1 (at most 2^28) and the flags
+    __device__ __forceinline__ float4 pack() const {
+        const uint32_t w = (uint32_t)(best + 1) | (found ? 1u << 29 : 0u) | (zero ? 1u << 30 : 0u) | (nan ? 1u << 31 : 0u);
+        return make_float4(t, u, v, __uint_as_float(w));
+    }
+    __device__ __forceinline__ static LinRun unpack(float4 p) {
+        const uint32_t w = __float_as_uint(p.w);
+        LinRun r;
+        r.t = p.x;
+        r.u = p.y;
+        r.v = p.z;
+        r.best = (int)(w & 0x1FFFFFFFu) - 1;
+        r.found = (w >> 29) & 1u;
+        r.zero = (w >> 30) & 1u;
+        r.nan = (w >> 31) & 1u;
+        return r;
+    }
+};
+
+// The ray as triangle xi meets it: in the triangle's local space, kept while the
+// transformation stays the same.
+struct LinRay {
+    F3 o, d, lo, ld;
     int lxi = -1;
-    F3 lo = o, ld = d;
-    for (int base = 0; base < n_tri; base += kLinTile) {
+    __device__ __forceinline__ void load(const float* ro, const float* rd, size_t i) {
+        lo = o = f3(ro[3 * i], ro[3 * i + 1], ro[3 * i + 2]);
+        ld = d = f3(rd[3 * i], rd[3 * i + 1], rd[3 * i + 2]);
+    }
+    __device__ __forceinline__ bool test(const float4* xf, int xi, F3 v1, F3 e1, F3 e2, float& t, float& u, float& v) {
+        F3 oo = o, dd = d;
+        if (xi >= 0) {
+            if (xi != lxi) {
+                lo = o;
+                ld = d;
+                to_local<true>(xf, xi, lo, ld);
+                lxi = xi;
+            }
+            oo = lo;
+            dd = ld;
+        }
+        return moller_trumbore(oo, dd, v1, e1, e2, t, u, v);
+    }
+};
+
+struct LinArgs {
+    int n, n_tri, chunk, n_chunks;   // triangles per chunk, a multiple of kLinTile
+    const float *ro, *rd;
+    const float *verts, *normals;    // the scene's triangles in their original order
+    const int32_t *matidx, *xfi;
+    const float4* xf;
+    float4* part;                    // [n_chunks][n] runs
+    float4* out;
+};
+
+// One run per ray and chunk of triangles, a workgroup per 256 rays and chunk:
+// every lane tests every triangle of the chunk, staged in LDS as (v1, e1, e2,
+// transformation) and read as broadcasts.  Bound by the tests' arithmetic (about
+// 60 instructions each), so what counts is that every CU has rays: the
+// triangles are split until the launch has kLinBlocks workgroups.
+__global__ __launch_bounds__(kLinTile) void k_query_linear(LinArgs a) {
+    __shared__ float4 tri[3 * kLinTile];
+    const int i = blockIdx.x * kLinTile + (int)threadIdx.x;
+    const bool act = i < a.n;
+    LinRay ray;
+    if (act) ray.load(a.ro, a.rd, (size_t)i);
+    LinRun run;
+    const int c0 = (int)blockIdx.y * a.chunk, c1 = min(a.n_tri, c0 + a.chunk);
+    for (int base = c0; base < c1; base += kLinTile) {
         __syncthreads();
         const int k = base + (int)threadIdx.x;
-        if (k < n_tri) {
-            for (int c = 0; c < 9; ++c) tv[c][threadIdx.x] = verts[9 * (size_t)k + c];
-            tx[threadIdx.x] = xfi ? xfi[k] : -1;
+        if (k < c1) {
+            const float* w = a.verts + 9 * (size_t)k;
+            const F3 v1 = f3(w[0], w[1], w[2]);
+            const F3 e1 = sub(f3(w[3], w[4], w[5]), v1), e2 = sub(f3(w[6], w[7], w[8]), v1);
+            tri[3 * threadIdx.x] = make_float4(v1.x, v1.y, v1.z, e1.x);
+            tri[3 * threadIdx.x + 1] = make_float4(e1.y, e1.z, e2.x, e2.y);
+            tri[3 * threadIdx.x + 2] = make_float4(e2.z, __int_as_float(a.xfi ? a.xfi[k] : -1), 0.0f, 0.0f);
         }
         __syncthreads();
-        const int cnt = min(kLinTile, n_tri - base);
         if (!act) continue;
+        const int cnt = min(kLinTile, c1 - base);
         for (int j = 0; j < cnt; ++j) {
-            const int xi = tx[j];
-            F3 oo = o, dd = d;
-            if (xi >= 0) {
-                if (xi != lxi) {
-                    lo = o;
-                    ld = d;
-                    to_local<true>(xf, xi, lo, ld);
-                    lxi = xi;
-                }
-                oo = lo;
-                dd = ld;
-            }
-            const F3 v1 = f3(tv[0][j], tv[1][j], tv[2][j]);
-            const F3 e1 = sub(f3(tv[3][j], tv[4][j], tv[5][j]), v1);
-            const F3 e2 = sub(f3(tv[6][j], tv[7][j], tv[8][j]), v1);
+            const float4 p = tri[3 * j], q = tri[3 * j + 1], r = tri[3 * j + 2];
             float t, u, v;
-            if (moller_trumbore(oo, dd, v1, e1, e2, t, u, v) && !(t > min_temp)) {
-                found = true;
+            if (ray.test(a.xf, __float_as_int(r.y), f3(p.x, p.y, p.z), f3(p.w, q.x, q.y), f3(q.z, q.w, r.x), t, u, v))
+                run.hit(t, u, v, base + j);
+        }
+    }
+    if (act) a.part[(size_t)blockIdx.y * a.n + i] = run.pack();
+}
+
+// The same with few rays: P lanes (a power of two) share a ray, each a slice of
+// consecutive triangles of the chunk, and combine their runs in order.
+__global__ __launch_bounds__(kLinTile) void k_query_linear_few(LinArgs a, int P) {
+    const int lane_p = (int)threadIdx.x & (P - 1);
+    const int i = (int)(blockIdx.x * (kLinTile / P)) + (int)threadIdx.x / P;
+    const bool act = i < a.n;
+    const int c0 = (int)blockIdx.y * a.chunk, c1 = min(a.n_tri, c0 + a.chunk);
+    const int len = a.chunk / P;
+    LinRun run;
+    if (act) {
+        LinRay ray;
+        ray.load(a.ro, a.rd, (size_t)i);
+        const int k1 = min(c1, c0 + (lane_p + 1) * len);
+        for (int k = c0 + lane_p * len; k < k1; ++k) {
+            const float* w = a.verts + 9 * (size_t)k;
+            const F3 v1 = f3(w[0], w[1], w[2]);
+            const F3 e1 = sub(f3(w[3], w[4], w[5]), v1), e2 = sub(f3(w[6], w[7], w[8]), v1);
+            float t, u, v;
+            if (ray.test(a.xf, a.xfi ? a.xfi[k] : -1, v1, e1, e2, t, u, v)) run.hit(t, u, v, k);
+        }
+    }
+    float4 mine = run.pack();
+    for (int off = 1; off < P; off <<= 1) {
+        const float4 o = make_float4(__shfl_down(mine.x, off), __shfl_down(mine.y, off), __shfl_down(mine.z, off),
+                                     __shfl_down(mine.w, off));
+        run.then(LinRun::unpack(o));   // right for the lanes the next steps read
+        mine = run.pack();
+    }
+    if (act && lane_p == 0) a.part[(size_t)blockIdx.y * a.n + i] = mine;
+}
+
+// A wave per ray: the chunks' runs combined in order (each lane a stretch of
+// chunks, then the lanes), then the answer.  The kept hit's point goes through M
+// and its normal through transpose(inverse) without a second normalisation.
+__global__ __launch_bounds__(256) void k_linear_merge(LinArgs a) {
+    const int i = blockIdx.x * 4 + (int)(threadIdx.x >> 6);
+    if (i >= a.n) return;
+    const int lane = __lane_id();
+    const int per = (a.n_chunks + 63) / 64;
+    const int b1 = min(a.n_chunks, (lane + 1) * per);
+    LinRun run;
+    for (int b = lane * per; b < b1; ++b) run.then(LinRun::unpack(a.part[(size_t)b * a.n + i]));
+    float4 mine = run.pack();
+    for (int off = 1; off < 64; off <<= 1) {
+        const float4 o = make_float4(__shfl_down(mine.x, off), __shfl_down(mine.y, off), __shfl_down(mine.z, off),
+                                     __shfl_down(mine.w, off));
+        run.then(LinRun::unpack(o));
+        mine = run.pack();
+    }
+    if (lane != 0) return;
+    LinRay ray;
+    ray.load(a.ro, a.rd, (size_t)i);
+    if (run.nan) {
+        // in index order, with both of the reference's bounds
+        float min_temp = INFINITY;
+        run = LinRun();
+        run.found = true;
+        for (int k = 0; k < a.n_tri; ++k) {
+            const float* w = a.verts + 9 * (size_t)k;
+            const F3 v1 = f3(w[0], w[1], w[2]);
+            const F3 e1 = sub(f3(w[3], w[4], w[5]), v1), e2 = sub(f3(w[6], w[7], w[8]), v1);
+            float t, u, v;
+            if (ray.test(a.xf, a.xfi ? a.xfi[k] : -1, v1, e1, e2, t, u, v) && !(t > min_temp)) {
                 min_temp = t;
-                if (t < min_dist && t > 0.0f) {
-                    min_dist = t;
-                    best = base + j;
-                    bu = u;
-                    bv = v;
+                if (t < run.t && t > 0.0f) {
+                    run.t = t;
+                    run.u = u;
+                    run.v = v;
+                    run.best = k;
                 }
             }
         }
     }
-    if (!act) return;
     F3 P = {0, 0, 0}, N = {0, 0, 0};
-    if (best < 0) {
-        write_hit(out, (size_t)i, found, P, N, -1, INFINITY, 0.0f, 0.0f, -1);
+    if (run.best < 0) {
+        write_hit(a.out, (size_t)i, run.found, P, N, -1, INFINITY, 0.0f, 0.0f, -1);
         return;
     }
-    const float* nn = normals + 9 * (size_t)best;
-    const int xi = xfi ? xfi[best] : -1;
+    const float* nn = a.normals + 9 * (size_t)run.best;
+    const int xi = a.xfi ? a.xfi[run.best] : -1;
     const float4 s0 = make_float4(nn[0], nn[1], nn[2], 0.0f);
     const float4 s1 = make_float4(nn[3], nn[4], nn[5], __int_as_float(xi));
     const float4 s2 = make_float4(nn[6], nn[7], nn[8], 0.0f);
-    hit_surface(s0, s1, s2, xf, o, d, min_dist, bu, bv, false, P, N);
-    write_hit(out, (size_t)i, found, P, N, matidx[best], min_dist, bu, bv, best);
+    hit_surface(s0, s1, s2, a.xf, ray.o, ray.d, run.t, run.u, run.v, false, P, N);
+    write_hit(a.out, (size_t)i, run.found, P, N, a.matidx[run.best], run.t, run.u, run.v, run.best);
+}
+
+// How a linear query is split: workgroups wanted, the most runs kept (16 bytes
+// each), and the most rays whose triangles are shared out over lanes as well.
+constexpr size_t kLinBlocks = 2048;
+constexpr size_t kLinParts = (size_t)EOS_STATIC_MAX_RAYS;
+constexpr int kLinFewRays = 128;
+
+// Chunks of triangles per ray, for n rays (n >= 1): as many as give kLinBlocks
+// workgroups, at most one per kLinTile triangles, and runs within kLinParts (one
+// chunk always).
+LinArgs linear_split(const eos_scene* s, int n, int& lanes_per_ray) {
+    LinArgs a{};
+    a.n = n;
+    a.n_tri = s->n_tri;
+    int P = 1;
+    if (n <= kLinFewRays)
+        while (P < 64 && 2 * P * n <= kLinTile) P *= 2;
+    lanes_per_ray = P;
+    const size_t ray_blocks = ((size_t)n * P + kLinTile - 1) / kLinTile;
+    const size_t tiles = std::max<size_t>(1, ((size_t)s->n_tri + kLinTile - 1) / kLinTile);
+    size_t c = std::min(tiles, (kLinBlocks + ray_blocks - 1) / ray_blocks);
+    c = std::max<size_t>(1, std::min({c, kLinParts / (size_t)n, (size_t)65535}));
+    const size_t per = (tiles + c - 1) / c;
+    a.chunk = (int)(per * kLinTile);
+    a.n_chunks = (int)((tiles + per - 1) / per);
+    a.verts = s->verts.as<const float>();
+    a.normals = s->normals.as<const float>();
+    a.matidx = s->matidx.as<const int32_t>();
+    a.xfi = s->n_xf > 0 ? s->xf_index.as<const int32_t>() : nullptr;
+    a.xf = s->n_xf > 0 ? s->xf.as<const float4>() : nullptr;
+    return a;
+}
+
+void launch_linear(const LinArgs& a, int P, hipStream_t S) {
+    const unsigned gx = (unsigned)(((size_t)a.n * P + kLinTile - 1) / kLinTile);
+    if (P > 1)
+        hipLaunchKernelGGL(k_query_linear_few, dim3(gx, (unsigned)a.n_chunks), dim3(kLinTile), 0, S, a, P);
+    else
+        hipLaunchKernelGGL(k_query_linear, dim3(gx, (unsigned)a.n_chunks), dim3(kLinTile), 0, S, a);
+    hipLaunchKernelGGL(k_linear_merge, dim3((unsigned)(((size_t)a.n + 3) / 4)), dim3(256), 0, S, a);
 }
 
 // The BVH traversal for caller-given rays: the default launch shape (256
@@ -202,10 +379,13 @@ eos_status trace_rays_static(eos_scene* s, int n, const float* o, const float* d
     float4* out = reinterpret_cast<float4*>(hits);
     const unsigned blocks = (unsigned)(((size_t)n + 255) / 256);
     if (opts->mode == EOS_QUERY_NEAREST_LINEAR) {
-        hipLaunchKernelGGL(k_query_linear, dim3(blocks), dim3(kLinTile), 0, S, n, o, d, s->n_tri,
-                           s->verts.as<const float>(), s->normals.as<const float>(), s->matidx.as<const int32_t>(),
-                           s->n_xf > 0 ? s->xf_index.as<const int32_t>() : nullptr,
-                           s->n_xf > 0 ? s->xf.as<const float4>() : nullptr, out);
+        int P = 1;
+        LinArgs la = linear_split(s, n, P);
+        la.ro = o;
+        la.rd = d;
+        la.part = rec;
+        la.out = out;
+        launch_linear(la, P, S);
         EOS_HIP(hipGetLastError());
         EOS_HIP(hipStreamSynchronize(S));
         return EOS_OK;
@@ -289,10 +469,14 @@ eos_status trace_rays(eos_scene* s, int n, const float* o, const float* d, const
     const unsigned blocks = (unsigned)((nn + 255) / 256);
     int err = 0;
     if (mode == EOS_QUERY_NEAREST_LINEAR) {
-        hipLaunchKernelGGL(k_query_linear, dim3(blocks), dim3(kLinTile), 0, S, n, ro, rd, s->n_tri,
-                           s->verts.as<const float>(), s->normals.as<const float>(), s->matidx.as<const int32_t>(),
-                           s->n_xf > 0 ? s->xf_index.as<const int32_t>() : nullptr,
-                           s->n_xf > 0 ? s->xf.as<const float4>() : nullptr, out);
+        int P = 1;
+        LinArgs la = linear_split(s, n, P);
+        EOS_TRY(s->q_rec.ensure(16 * nn * (size_t)la.n_chunks));
+        la.ro = ro;
+        la.rd = rd;
+        la.part = s->q_rec.as<float4>();
+        la.out = out;
+        launch_linear(la, P, S);
         EOS_HIP(hipGetLastError());
     } else {
         const LaunchCfg& cfg = s->cfg;
