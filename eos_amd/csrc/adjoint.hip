@@ -30,6 +30,8 @@
 namespace eos {
 namespace {
 
+constexpr int kErrOpen = 16;
+
 struct AdjArgs {
     SceneView sc;
     DevCamera cam;
@@ -40,7 +42,8 @@ struct AdjArgs {
     const float4* levcol;          // weights of the levels above
     const float* dl;               // [npix][3]
     unsigned long long* gout;      // [3][M*7 + L*6] limbs of the exact sums
-    int* err;                      // bit 8: a contribution out of range (non-finite or >= 2^31)
+    int* err;                      // bit 8: a contribution out of range (non-finite or >= 2^31); bit 16: a
+                                   // visibility that the frame left open matters (kErrOpen)
     int lds_acc;                   // accumulate in LDS (else straight to global)
 };
 
@@ -84,7 +87,11 @@ __global__ __launch_bounds__(256) void k_adjoint(AdjArgs a) {
         float gkd[3] = {0, 0, 0}, gks[3] = {0, 0, 0}, gs = 0.0f;
         bool any = false;
         for (int i = 0; i < L; ++i) {
-            if (!a.vis[(size_t)j * L + i]) continue;
+            const uint8_t vis = a.vis[(size_t)j * L + i];
+            // a light that adds nothing: every term below is zero times a finite
+            // upstream gradient; with another one it matters whether it is visible
+            if (vis == kVisDark && !(g0 - g0 == 0.0f && g1 - g1 == 0.0f && g2 - g2 == 0.0f)) atomicOr(a.err, kErrOpen);
+            if (vis != kVisVisible) continue;
             any = true;
             const DevLight& lt = a.sc.lights[i];
             const F3 D = sub(f3(lt.position[0], lt.position[1], lt.position[2]), P);
@@ -155,9 +162,11 @@ __global__ void k_zero_u64(unsigned long long* p, int n) {
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = 0ull;
 }
 
-// dst_m[M][7] += value of limbs i < 7M, dst_l[L][6] += the rest
-__global__ void k_accumulate_out(const unsigned long long* g, int M, int L, double* dm, double* dlg) {
+// dst_m[M][7] += value of limbs i < 7M, dst_l[L][6] += the rest (unless the
+// records have to be traced again)
+__global__ void k_accumulate_out(const unsigned long long* g, const int* err, int M, int L, double* dm, double* dlg) {
     const int nacc = 7 * M + 6 * L;
+    if (*err & kErrOpen) return;   // replayed again
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < nacc; i += gridDim.x * blockDim.x) {
         const double v = limb_value(g, nacc, i);
         if (i < 7 * M) dm[i] += v;
@@ -169,19 +178,19 @@ constexpr int kLdsAccParams = 2048;   // 48 KiB of limbs (3 x int64 per paramete
 
 }  // namespace
 
-eos_status render_adjoint(eos_scene* s, const eos_camera* cam, const eos_adjoint_opts* o, const float* dl,
-                          double* gm, double* gl, eos_adjoint_stats* st) {
+static eos_status adjoint_once(eos_scene* s, const eos_camera* cam, const eos_adjoint_opts* o, const float* dl,
+                          double* gm, double* gl, eos_adjoint_stats* st, bool walk_all, bool& open) {
     eos_frame_buffers& fb = s->fb;
     hipStream_t S = s->stream;
     const size_t npix = (size_t)cam->width * cam->height;
     const int M = s->n_mat, L = s->n_light;
     const int nacc = 7 * M + 6 * L;
-    const bool replay = !o->recompute && fb.rec_valid && fb.depth == o->depth && fb.n_light == L &&
+    const bool replay = !walk_all && !o->recompute && fb.rec_valid && fb.depth == o->depth && fb.n_light == L &&
                         std::memcmp(&fb.rec_cam, cam, sizeof(eos_camera)) == 0;
     double retrace_ms = 0.0;
     if (!replay) {
         eos_render_stats rs;
-        EOS_TRY(run_frame(s, cam, o->depth, false, nullptr, nullptr, nullptr, &rs));
+        EOS_TRY(run_frame(s, cam, o->depth, false, nullptr, nullptr, nullptr, &rs, AaSample(), 0, -1, true, walk_all));
         retrace_ms = rs.render_ms;
         fb.rec_valid = 1;
         fb.rec_cam = *cam;
@@ -227,15 +236,19 @@ eos_status render_adjoint(eos_scene* s, const eos_camera* cam, const eos_adjoint
     EOS_HIP(hipMemcpyAsync(&herr, err, sizeof herr, hipMemcpyDeviceToHost, S));
     if (o->memory == EOS_MEM_DEVICE) {
         hipLaunchKernelGGL(k_accumulate_out, dim3(std::max(1, std::min(64, (nacc + 255) / 256))), dim3(256), 0, S,
-                           g_dev.as<const unsigned long long>(), M, L, gm, gl);
+                           g_dev.as<const unsigned long long>(), err, M, L, gm, gl);
         EOS_HIP(hipStreamSynchronize(S));
+        open = (herr & kErrOpen) != 0;
     } else {
         std::vector<unsigned long long> h((size_t)std::max(3 * nacc, 1));
         EOS_HIP(hipMemcpyAsync(h.data(), g_dev.ptr, 8 * 3 * (size_t)nacc, hipMemcpyDeviceToHost, S));
         EOS_HIP(hipStreamSynchronize(S));
+        open = (herr & kErrOpen) != 0;
+        if (open) return EOS_OK;
         for (int i = 0; i < 7 * M; ++i) gm[i] += limb_value(h.data(), nacc, i);
         for (int i = 0; i < 6 * L; ++i) gl[i] += limb_value(h.data(), nacc, 7 * M + i);
     }
+    if (open) return EOS_OK;
     if (herr & 8)
         return fail(EOS_ERR_LIMIT, "eos_render_adjoint: a gradient contribution is not finite or exceeds 2^31 "
                                    "(a light on a surface?); the gradients are incomplete");
@@ -249,6 +262,16 @@ eos_status render_adjoint(eos_scene* s, const eos_camera* cam, const eos_adjoint
         st->records = 0;
         for (int l = 0; l <= o->depth; ++l) st->records += hits[l];
     }
+    return EOS_OK;
+}
+
+eos_status render_adjoint(eos_scene* s, const eos_camera* cam, const eos_adjoint_opts* o, const float* dl,
+                          double* gm, double* gl, eos_adjoint_stats* st) {
+    bool open = false;
+    EOS_TRY(adjoint_once(s, cam, o, dl, gm, gl, st, false, open));
+    // an upstream gradient that is not finite reached a surface whose visibility
+    // records leave a light open: once more over records with every shadow ray walked
+    if (open) EOS_TRY(adjoint_once(s, cam, o, dl, gm, gl, st, true, open));
     return EOS_OK;
 }
 

@@ -144,7 +144,7 @@ struct eos_frame_buffers {
     eos::DevBuf hitq;       // float4 [cap]        hit records of queued rays
     // Per level l, at fixed strides so one launch can address several levels:
     eos::DevBuf surf;       // float4 [D+1][cap][2] hit surfaces (P.xyz pixel | N.xyz mat)
-    eos::DevBuf vis;        // uint8  [D+1][cap][L] light visible from the hit surface
+    eos::DevBuf vis;        // uint8  [D+1][cap][L] light visible from the hit surface (kVis*)
     size_t cap = 0;         // surfaces per level (pixels of the frame)
     int lslots = 1;         // light slots per surface
     size_t surf_stride() const { return 2 * cap; }                // float4 per level
@@ -267,8 +267,9 @@ struct AaSample {
 };
 // One frame of the wavefront pipeline (render.hip); outputs may be null.
 // launch_times: timing events around every launch (else only around the frame
-// and its primary-ray launch).
+// and its primary-ray launch).  walk_all: shadow rays
+// toward lights that add nothing to their surface are walked too.
 eos_status run_frame(eos_scene* s, const eos_camera* cam, int depth, bool count, uchar4* rgba_dev, float* rgb_dev,
                      int32_t* hits_dev, eos_render_stats* st, const AaSample& aa = AaSample(), int row0 = 0,
-                     int row1 = -1, bool launch_times = true);
+                     int row1 = -1, bool launch_times = true, bool walk_all = false);
 }  // namespace eos

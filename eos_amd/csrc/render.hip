@@ -46,6 +46,9 @@ struct SetupArgs {
     int* q_out_ctr;
     int q_cap;                // rays the next level's queue holds (appends beyond it are dropped and counted)
     int* shadow_ctr;
+    uint8_t* vis_out;         // per hit and light slot: kVisDark where the light adds nothing, else kVisVisible (the
+                              // shadow launch answers those); null: every shadow ray is walked
+    int lstride;
     uint8_t* levels;
     int32_t* hit_ids;         // level 0, optional
     const uint8_t* tile_live; // level 0, single scene, optional: 0 = the tile test resolved the tile (misses)
@@ -67,6 +70,27 @@ __device__ __forceinline__ float fresnel(F3 incident, F3 normal, float n1, float
     const float rOrth = (n1 * cosI - n2 * cosT) / (n1 * cosI + n2 * cosT);
     const float rPar = (n2 * cosI - n1 * cosT) / (n2 * cosI + n1 * cosT);
     return (rOrth * rOrth + rPar * rPar) / 2.0f;
+}
+
+// Whether a light adds anything to a surface it reaches: false when both of
+// phong()'s terms are exactly zero -- the light behind the surface and no
+// highlight (V.R <= 0; values that are not numbers, or an infinite colour, count
+// as adding).  The shadow ray toward such a light is not walked: its answer
+// changes no colour, and no gradient of a finite upstream gradient.  These are
+// the rays sent into their own surface, which walk far: four 1080p frames close to
+// a 1M-triangle mesh, four lights, 9.9 -> 8.9 ms, 16 random scenes batched
+// 5.10 -> 4.75 ms.
+__device__ __forceinline__ bool light_adds(const DevMaterial& m, const DevLight& l, F3 cam, F3 P, F3 N) {
+    const F3 L = normalize3(sub(f3(l.position[0], l.position[1], l.position[2]), P));
+    const float dNL = dot3(N, L);
+    if (!(dNL <= 0.0f)) return true;
+    const F3 V = normalize3(sub(cam, P));
+    const float s2 = 2.0f * dNL;
+    const F3 R = normalize3(sub(f3(s2 * N.x, s2 * N.y, s2 * N.z), L));
+    bool none = dot3(V, R) <= 0.0f;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) none = none && (0.0f * m.kd[k]) * l.color[k] == 0.0f && 0.0f * m.ks[k] == 0.0f;
+    return !none;
 }
 
 // Hit set-up of one level: the hit surface (hit_surface, the reference's
@@ -200,6 +224,15 @@ __global__ __launch_bounds__(kSetupWG) void k_setup(SetupArgs a) {
         if (hit) {
             a.surf_out[2 * (size_t)j] = make_float4(P.x, P.y, P.z, __int_as_float(pixel));
             a.surf_out[2 * (size_t)j + 1] = make_float4(N.x, N.y, N.z, __int_as_float(pack_mat(mat, scene)));
+            if (a.vis_out) {
+                const DevLight* lights = BATCH ? a.table[scene].sc.lights : a.sc.lights;
+                const DevCamera& cm = BATCH ? a.table[scene].cam : a.cam;
+                const int nlt = BATCH ? a.table[scene].sc.n_light : a.sc.n_light;
+                const F3 cam = f3(cm.position[0], cm.position[1], cm.position[2]);
+                for (int li = 0; li < a.lstride; ++li)
+                    a.vis_out[(size_t)j * a.lstride + li] =
+                        li < nlt && light_adds(mats[mat], lights[li], cam, P, N) ? kVisVisible : kVisDark;
+            }
         }
         if (refl && k < a.q_cap) {
             // src/RayTracer.cpp:350-355
@@ -302,7 +335,7 @@ __global__ __launch_bounds__(256) void k_phong(PhongArgs a) {
             const int L = sc.n_light;
             float acc[3] = {0.0f, 0.0f, 0.0f};
             for (int i = 0; i < L; ++i) {
-                if (!vis[(size_t)j * a.lstride + i]) continue;
+                if (vis[(size_t)j * a.lstride + i] != kVisVisible) continue;
                 float c[3];
                 phong(m, sc.lights[i], cam, P, N, c);
 #pragma unroll
@@ -748,6 +781,7 @@ struct Frame {
     hipEvent_t resolve_done = nullptr;    // and record this one after it
     hipEvent_t first_ev[2] = {nullptr, nullptr};   // frames in flight: around the primary-ray launch
     bool count = false;
+    bool walk_all = false; // every shadow ray is walked (else not those of lights that add nothing)
     LaunchCfg cfg;
     int num_cu = 256;
     uchar4* rgba = nullptr;
@@ -889,6 +923,7 @@ eos_status enqueue_frame(eos_frame_buffers& fb, const Frame& f, const FrameStrea
             sh.group_lanes = f.cfg.group_lanes;
             sh.steal = f.count ? 0 : f.cfg.steal;
             sh.scatter = f.cfg.scatter;
+            sh.skip_dark = f.count || f.walk_all ? 0 : 1;
             sh.cursor = cursors(16 + l0);
             sh.stats = stats + 2 * (16 + l0);
             sh.count_ptr = ctr + CTR_HITS + l0;
@@ -1035,6 +1070,8 @@ eos_status enqueue_frame(eos_frame_buffers& fb, const Frame& f, const FrameStrea
             sa.aux = fb.aux.as<float4>() + fb.toff[l];
         }
         sa.shadow_ctr = ctr + CTR_SHADOW + l;
+        sa.vis_out = f.count || f.walk_all ? nullptr : fb.vis_at(f.tree ? 0 : l);
+        sa.lstride = f.lstride;
         sa.levels = fb.levels.as<uint8_t>();
         sa.hit_ids = l == 0 ? f.hits : nullptr;
         sa.tile_live = l == 0 && cull ? fb.tile_flags(f.n_ids) : nullptr;
@@ -1212,8 +1249,9 @@ int trace_grid_of(const Frame& f) { return std::max(1, f.num_cu * f.cfg.waves_pe
 
 eos_status run_frame(eos_scene* s, const eos_camera* camp, int depth, bool count, uchar4* rgba_dev,
                      float* rgb_dev, int32_t* hits_dev, eos_render_stats* st, const AaSample& aa, int row0, int row1,
-                     bool launch_times) {
+                     bool launch_times, bool walk_all) {
     Frame f = make_frame(s, camp, depth, count, rgba_dev, rgb_dev, hits_dev, aa, row0, row1);
+    f.walk_all = walk_all;
     EOS_TRY(ensure_buffers(s->fb, f, trace_grid_of(f)));
     FrameEvents fe;
     FrameStreams fs{s->stream, s->stream2, s->sync};

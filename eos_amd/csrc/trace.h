@@ -300,7 +300,7 @@ struct TraceArgs {
     const float* ray_d;      // MODE_RAYS(_ANY): directions [n][3]
     float4* hit_out;         // closest: (t, slot, u, v)
     const float4* surf;      // MODE_SHADOW: hit surfaces (P.xyz pixel | N.xyz mat) of the first level
-    uint8_t* vis_out;        // MODE_SHADOW: 1 = light visible, first level; MODE_RAYS_ANY: 1 = occluded
+    uint8_t* vis_out;        // MODE_SHADOW: kVis*, first level; MODE_RAYS_ANY: 1 = occluded
     int nlev;                // MODE_SHADOW: consecutive levels in this launch (count_ptr[0..nlev))
     long long surf_stride;   // MODE_SHADOW: float4 between levels' surfaces
     long long vis_stride;    // MODE_SHADOW: bytes between levels' visibility
@@ -313,6 +313,8 @@ struct TraceArgs {
     int group;               // group walk (16 lanes per ray) for launches of at most group x lanes/16 items (0: never)
     int group_lanes;         // 64: launches of at most group x lanes/64 items walk each ray with a whole wave
     int steal;               // per-lane walk: idle lanes of a drained wave take pending subtrees of its rays
+    int skip_dark;           // MODE_SHADOW: the set-up kernel wrote kVisDark where a light adds nothing to its
+                             // surface, visible or not; those rays are not walked
     int scatter;             // launches of at most scatter x lanes items claim them in scattered order (0: never)
 };
 
@@ -466,13 +468,6 @@ struct Scatter {
     }
 };
 
-// Any-hit rays sent into their own surface walk the farthest child first (see
-// setup_item); a switch for measuring it.
-#ifndef EOS_FAR_FIRST
-#define EOS_FAR_FIRST 1
-#endif
-constexpr bool kFarFirst = EOS_FAR_FIRST != 0;
-
 // Order of a shadow launch's items within a level: tiles of kLightTile hit
 // surfaces, light by light inside a tile (item = tile, light slot, surface in
 // the tile), so that lanes refilled together trace neighbouring surfaces toward
@@ -490,6 +485,11 @@ constexpr bool kFarFirst = EOS_FAR_FIRST != 0;
 #endif
 constexpr int kLightTile = EOS_LIGHT_TILE;
 
+// Visibility bytes of a hit and light slot: the shadow ray's answer, or that the
+// light adds nothing to the surface whether it reaches it or not, and its ray was
+// not walked (frames that do not walk every shadow ray).
+enum : uint8_t { kVisOccluded = 0, kVisVisible = 1, kVisDark = 2 };
+
 // One traversal item, set up: the ray and the scene it runs in.
 struct RayItem {
     F3 o, d;
@@ -500,7 +500,7 @@ struct RayItem {
     const float4* geo;
     const float4* xf;        // transformations of the scene (null: none)
     size_t out_idx;          // any hit: result byte of the item
-    bool far_first;          // shadow ray into its own surface: walk the farthest child first
+    bool dark;               // shadow ray whose answer is kVisDark: not walked
 };
 
 // Item of a primary launch whose tiles went through the tile test: the launch
@@ -524,7 +524,7 @@ __device__ __forceinline__ void setup_item(const TraceArgs& a, int my, RayItem& 
     r.root = WIDTH == 4 ? a.sc.root4 : a.sc.root;
     r.max_visits = a.sc.n_tri + 64;
     r.out_idx = 0;
-    r.far_first = false;
+    r.dark = false;
     auto use_scene = [&](const BatchScene& B) {
         r.nodes = B.sc.nodes;
         r.nodes4 = B.sc.nodes4;
@@ -583,6 +583,12 @@ __device__ __forceinline__ void setup_item(const TraceArgs& a, int my, RayItem& 
         }
         // the result byte keeps the surface-by-surface layout the shading reads
         r.out_idx = (size_t)lev * (size_t)a.vis_stride + (size_t)j * (size_t)a.count_mul + (size_t)li;
+        if (a.skip_dark && a.vis_out[r.out_idx] == kVisDark) {
+            r.dark = true;
+            r.valid = false;
+            r.o = r.d = f3(0.0f, 0.0f, 1.0f);
+            return;
+        }
         const float4 s0 = surf[2 * (size_t)j];
         const F3 P = f3(s0.x, s0.y, s0.z);
         const DevLight* lights = a.sc.lights;
@@ -597,11 +603,6 @@ __device__ __forceinline__ void setup_item(const TraceArgs& a, int my, RayItem& 
             const DevLight& L = lights[li];
             r.d = normalize3(sub(f3(L.position[0], L.position[1], L.position[2]), P));
             r.o = add(P, scale(1e-3f, r.d));
-            // a light behind the surface sends the ray into the object: its
-            // occluder, if any, is most likely far away (the far wall), so that
-            // ray walks the farthest child first (any order gives the same answer)
-            const float4 s1 = surf[2 * (size_t)j + 1];
-            r.far_first = kFarFirst && dot3(f3(s1.x, s1.y, s1.z), r.d) < 0.0f;
         } else {
             r.valid = false;
             r.d = f3(0.0f, 0.0f, 1.0f);
@@ -688,6 +689,7 @@ __device__ __forceinline__ void trace_coop(const TraceArgs& a, int n, int32_t* w
                 sp = 0;
                 budget = r.max_visits;
                 cur = r.valid ? r.root : kDone;
+                if (r.dark) item = -1;   // answered already
             }
         }
         if (__ballot(item >= 0) == 0) {
@@ -891,6 +893,7 @@ __device__ __forceinline__ void trace_group(const TraceArgs& a, int n, int32_t* 
                     if (gsub == 0) stk[0] = r.root;
                     sp = 1;
                 }
+                if (r.dark) item = -1;   // answered already
             }
         }
         if (__ballot(item >= 0) == 0) {
@@ -1012,9 +1015,6 @@ __device__ __forceinline__ void trace_group(const TraceArgs& a, int n, int32_t* 
 // the order, so only the (rare) occluded rays can end sooner or later (hit-dense
 // 4K frame 19.4 -> 18.65 ms).  Both leave every result unchanged; launches that
 // count visits keep the sorted order.
-#ifndef EOS_ANY_NOSORT
-#define EOS_ANY_NOSORT 1
-#endif
 // Idle lanes a wave needs before its walking lanes lend subtrees (measured,
 // frames identical: at 1, 16, 32, 48 idle lanes config C's single frame took
 // 2.21, 2.11, 2.11, 2.28 ms and config D's 64 sequential frames 102, 93, 84, 87 ms).
@@ -1022,7 +1022,6 @@ __device__ __forceinline__ void trace_group(const TraceArgs& a, int n, int32_t* 
 #define EOS_STEAL_IDLE 32
 #endif
 constexpr int kStealIdle = EOS_STEAL_IDLE;
-constexpr bool kAnyNoSort = EOS_ANY_NOSORT != 0;
 
 // LDS in its own address space: a load whose address could be LDS or global
 // memory (the pop of a stack that overflows from one into the other) would
@@ -1181,7 +1180,6 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(XF ? 4 : 5))
         int cur = kDone;
         LaneStack<WG, STACK_LDS, KEYS> stk;
         int lpos = -1;   // next triangle of the current leaf (-1: not in a leaf)
-        bool farf = false;   // any hit: walk the farthest hit child first (RayItem::far_first)
         int sgx = 0, sgy = 0, sgz = 0;   // 16 (bytes) where the inverse direction is negative (hi plane nearer)
         int budget = 0;  // node visits left for this ray: a tree visits each internal node at most once
         // XF: the ray in the local space of transformation lxi, kept while the
@@ -1245,9 +1243,9 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(XF ? 4 : 5))
                     lxi = -1;
                     budget = r.max_visits;
                     cur = r.valid ? r.root : kDone;
-                    farf = ANY && !COUNT && r.far_first;
                     home = -1;
                     pending = 0;
+                    if (r.dark) item = -1;   // answered already
                 }
             }
             if (__ballot(item >= 0) == 0) {
@@ -1340,7 +1338,7 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(XF ? 4 : 5))
                             } else if (!stk.lds_room(4) && stk.sp + nh - 1 > MAXS) {
                                 atomicOr(a.err, 1);
                                 cur = kDone;
-                            } else if (ANY && !COUNT && kAnyNoSort && !farf && stk.lds_room(4)) {
+                            } else if (ANY && !COUNT && stk.lds_room(4)) {
                                 // any hit: the order of the children does not change the
                                 // answer; the first hit child next, the others onto the stack
                                 // in slot order (non-hits to a slot above the new top)
@@ -1377,22 +1375,7 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(XF ? 4 : 5))
                                     keyswap(q1, r1, q3, r3);
                                     keyswap(q1, r1, q2, r2);
                                 }
-                                if (ANY && !COUNT && farf) {
-                                    // farthest hit child next; the nearer ones pushed nearest
-                                    // first, so the next farthest is popped next
-                                    const int far = nh > 3 ? r3 : (nh > 2 ? r2 : (nh > 1 ? r1 : r0));
-                                    if (stk.lds_room(3)) {
-                                        stk.put(sref, skey, tid, 0, r0, 0u);
-                                        stk.put(sref, skey, tid, 1, r1, 0u);
-                                        stk.put(sref, skey, tid, 2, r2, 0u);
-                                        stk.sp += nh - 1;
-                                    } else {
-                                        if (nh > 1) stk.push(sref, skey, gst, tid, r0, 0u);
-                                        if (nh > 2) stk.push(sref, skey, gst, tid, r1, 0u);
-                                        if (nh > 3) stk.push(sref, skey, gst, tid, r2, 0u);
-                                    }
-                                    r0 = far;
-                                } else if (stk.lds_room(3)) {
+                                if (stk.lds_room(3)) {
                                     // farthest first, all three slots written (those above
                                     // the new top are overwritten later)
                                     stk.put(sref, skey, tid, 0, nh > 3 ? r3 : (nh > 2 ? r2 : r1), nh > 3 ? q3 : (nh > 2 ? q2 : q1));
@@ -1612,7 +1595,6 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(XF ? 4 : 5))
                             budget = g_budget;
                             stk.clear();
                             lpos = -1;
-                            farf = false;
                             lxi = -1;
                             pending = 0;
                         }
