@@ -796,6 +796,14 @@ eos_status launch_trace_any(const Frame& f, int grid, hipStream_t s, const Trace
                    : launch_trace<MODE, false, false>(f.cfg, f.width, f.xf, f.big, grid, s, a, lean);
 }
 
+// Workgroups of a persistent traversal grid of `waves` waves per CU.
+int trace_grid_waves(const Frame& f, int waves) { return std::max(1, f.num_cu * waves / (f.cfg.workgroup / 64)); }
+// Waves per SIMD that the traversal kernels' registers allow (k_trace's
+// amdgpu_waves_per_eu), without and with transformations.
+constexpr int kResident = 5, kResidentXf = 4;
+int trace_grid_of(const Frame& f) {
+    return trace_grid_waves(f, f.cfg.waves_per_cu);
+}
 // Overflow stack entries of one persistent traversal grid.
 size_t gstack_ints(const Frame& f, int trace_grid) {
     const int maxs = f.width == 4 ? kMaxStack4 : kMaxStack;
@@ -882,7 +890,7 @@ eos_status ensure_buffers(eos_frame_buffers& fb, const Frame& f, int trace_grid)
 // non-null (not while a graph is being captured).
 eos_status enqueue_frame(eos_frame_buffers& fb, const Frame& f, const FrameStreams& fs, hipEvent_t* E,
                          FrameEvents* fe) {
-    const int trace_grid = std::max(1, f.num_cu * f.cfg.waves_per_cu / (f.cfg.workgroup / 64));
+    const int trace_grid = trace_grid_of(f);
     int* ctr = fb.counters.as<int>();
     unsigned long long* stats = reinterpret_cast<unsigned long long*>(fb.counters.as<char>() + 4 * CTR_COUNT);
     const unsigned shade_grid = (unsigned)f.num_cu * 8;
@@ -939,7 +947,15 @@ eos_status enqueue_frame(eos_frame_buffers& fb, const Frame& f, const FrameStrea
             // workgroups room (hit-dense 4K frame 17.3 -> 16.5 ms, config E
             // 1.84 -> 1.80 ms); its launches are large, so the group walk would
             // not be taken there anyway
-            EOS_TRY(launch_trace_any<MODE_SHADOW>(f, trace_grid, st, sh,
+            // and its grid leaves one wave slot per SIMD free: with every slot taken
+            // (a set-up workgroup of the chain has no registers left either) the
+            // chain waits for the end of this launch: 64 moving instances 2535 ->
+            // 2448 us, 4K frame 1821 -> 1807, training step 1904 -> 1899; smaller grids
+            // cost the frames whose shadow rays are most of the work (12 waves per CU:
+            // four close 1080p frames 8382 -> 8563)
+            const int resident = f.xf || f.big ? kResidentXf : kResident;
+            const int sgrid = st != S ? trace_grid_waves(f, std::min(f.cfg.waves_per_cu, 4 * (resident - 1))) : trace_grid;
+            EOS_TRY(launch_trace_any<MODE_SHADOW>(f, sgrid, st, sh,
                                                   st != S));
         }
         F.s[2 * slot + 1] = rec(st);
@@ -1243,8 +1259,6 @@ Frame make_frame(eos_scene* s, const eos_camera* camp, int depth, bool count, uc
     f.hits = hits_dev;
     return f;
 }
-
-int trace_grid_of(const Frame& f) { return std::max(1, f.num_cu * f.cfg.waves_per_cu / (f.cfg.workgroup / 64)); }
 }  // namespace
 
 eos_status run_frame(eos_scene* s, const eos_camera* camp, int depth, bool count, uchar4* rgba_dev,
@@ -1577,8 +1591,7 @@ eos_status render_batch(eos_scene* const* scenes, const eos_camera* cams, int n,
         f.rgba = b.rgba.as<uchar4>();
         f.sc = view_of(s0);
         f.cam = b.host_table[0].cam;
-        const int trace_grid = std::max(1, f.num_cu * f.cfg.waves_per_cu / (f.cfg.workgroup / 64));
-        EOS_TRY(ensure_buffers(b.fb, f, trace_grid));
+        EOS_TRY(ensure_buffers(b.fb, f, trace_grid_of(f)));
         b.scenes.assign(scenes, scenes + n);
         b.mat_gens.resize(n);
         for (int i = 0; i < n; ++i) b.mat_gens[i] = scenes[i]->mat_generation;
