@@ -69,8 +69,8 @@ static eos_status copy_in(DevBuf& dst, const void* src, size_t bytes, int memory
 static void free_scene(eos_scene* s) {
     DevBuf* bufs[] = {&s->verts, &s->normals, &s->matidx, &s->mats, &s->lights, &s->nodes, &s->tree,
                       &s->shade, &s->codes, &s->codes_sorted, &s->perm, &s->kchild, &s->kparent,
-                      &s->first_last, &s->ibox, &s->lbox, &s->flags, &s->cbounds, &s->sort_tmp_k,
-                      &s->sort_tmp_v, &s->sort_hist, &s->bounds_part, &s->flags4, &s->scan_tmp,
+                      &s->first_last, &s->ibox, &s->lbox, &s->cbounds, &s->sort_tmp_k,
+                      &s->sort_tmp_v, &s->sort_hist, &s->bounds_part, &s->pyramid, &s->masks4,
                       &s->xf, &s->xf_index, &s->wverts, &s->q_rays, &s->q_out, &s->q_rec, &s->q_ctr, &s->q_gstack,
                       &s->fb.hit0, &s->fb.q[0], &s->fb.q[1],
                       &s->fb.hitq, &s->fb.levcol, &s->fb.levels, &s->fb.counters, &s->fb.gstack, &s->fb.aa_acc,
@@ -553,9 +553,9 @@ eos_status eos_debug_read(const eos_scene* s, int32_t what, void* dst, int64_t b
         case EOS_DBG_KPARENT: b = &s->kparent; need = 4 * (2 * n - (n ? 1 : 0)); break;
         case EOS_DBG_IBOX: b = &s->ibox; need = 24 * m; break;
         case EOS_DBG_NODES: b = &s->nodes; need = 64 * m; break;
-        case EOS_DBG_TRIS: b = &s->tree; need = 48 * n; off = 128 * (size_t)s->n_nodes4; break;
+        case EOS_DBG_TRIS: b = &s->tree; need = 48 * n; break;
         case EOS_DBG_MORTON: b = &s->codes; need = 4 * n; break;
-        case EOS_DBG_NODES4: b = &s->tree; need = 128 * (size_t)s->n_nodes4; break;
+        case EOS_DBG_NODES4: b = &s->tree; need = 128 * (size_t)s->n_nodes4; off = s->nodes4_offset(); break;
         case EOS_DBG_XFORMS: b = &s->xf; need = 16 * kXfRows * (size_t)s->n_xf; break;
         default: return fail(EOS_ERR_INVALID, "eos_debug_read: unknown array");
     }
@@ -565,6 +565,7 @@ eos_status eos_debug_read(const eos_scene* s, int32_t what, void* dst, int64_t b
     if ((size_t)bytes < need) return fail(EOS_ERR_INVALID, "eos_debug_read: destination too small");
     if (need == 0) return EOS_OK;
     EOS_HIP(hipSetDevice(s->device));
+    if (what == EOS_DBG_NODES) EOS_TRY(make_binary_nodes(const_cast<eos_scene*>(s)));
     EOS_HIP(hipMemcpyAsync(dst, b->as<char>() + off, need, hipMemcpyDeviceToHost, s->stream));
     EOS_HIP(hipStreamSynchronize(s->stream));
     return EOS_OK;

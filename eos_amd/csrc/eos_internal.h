@@ -190,17 +190,18 @@ struct eos_scene {
     eos::DevBuf verts, normals, matidx;
     eos::DevBuf mats, lights;
     // LBVH and sorted layouts
-    // tree: the 4-wide nodes, then the triangle geometry records, in one allocation:
+    // tree: the triangle geometry records, then the 4-wide nodes, in one allocation:
     // the traversal addresses both from one base with 32-bit byte offsets (a tree
     // past 4 GiB, about 45 million triangles, takes kernels with 64-bit addresses)
     eos::DevBuf nodes, tree, shade;
-    size_t tree_bytes() const { return 128 * (size_t)n_nodes4 + 48 * (size_t)n_tri; }
-    bool tree_big() const { return tree_bytes() > (size_t)UINT32_MAX; }
-    eos::Node4* nodes4() const { return tree.as<eos::Node4>(); }
-    float4* geo() const { return reinterpret_cast<float4*>(tree.as<char>() + 128 * (size_t)n_nodes4); }
-    eos::DevBuf codes, codes_sorted, perm, kchild, kparent, first_last, ibox, lbox, flags, cbounds;
+    size_t nodes4_offset() const { return (48 * (size_t)n_tri + 127) & ~(size_t)127; }
+    size_t tree_bytes(size_t nodes) const { return nodes4_offset() + 128 * nodes; }
+    bool tree_big() const { return tree_bytes((size_t)n_nodes4) > (size_t)UINT32_MAX; }
+    eos::Node4* nodes4() const { return reinterpret_cast<eos::Node4*>(tree.as<char>() + nodes4_offset()); }
+    float4* geo() const { return tree.as<float4>(); }
+    eos::DevBuf codes, codes_sorted, perm, kchild, kparent, first_last, ibox, lbox, cbounds;
     eos::DevBuf sort_tmp_k, sort_tmp_v, sort_hist, bounds_part;
-    eos::DevBuf flags4, scan_tmp;
+    eos::DevBuf pyramid, masks4;
     // per-triangle transformations: xf [n_xf][kXfRows] float4, xf_index [N]
     // (original order, -1 = none), world-space vertices for the build
     eos::DevBuf xf, xf_index, wverts;
@@ -214,6 +215,7 @@ struct eos_scene {
     int width = 4;
     int leaf_max = 1;
     bool built = false;
+    bool nodes_valid = false;     // the binary nodes are made (builds of width 4 make them when they are read)
     bool batch_built = false;     // built by eos_build_lbvh_batch: the build's intermediate arrays are not kept
     eos::LaunchCfg cfg;
     int num_cu = 256;
@@ -240,6 +242,8 @@ namespace eos {
 // Implemented in lbvh.hip
 eos_status build_lbvh(eos_scene* s, int leaf_max, int width, eos_build_stats* st);
 eos_status build_lbvh_batch(eos_scene* const* scenes, int n, int leaf_max, int width, eos_build_stats* st);
+// The binary nodes of a scene built with width 4, for eos_debug_read.
+eos_status make_binary_nodes(eos_scene* s);
 // Implemented in render.hip
 // Rows [row0, row1) of the camera's frame (row1 < 0: to the last row).
 eos_status render(eos_scene* s, const eos_camera* cam, const eos_render_opts* o, uint8_t* rgba,

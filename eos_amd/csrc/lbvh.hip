@@ -5,10 +5,12 @@
 // (src/morton.h:30-48).  This file builds a Karras (2012) LBVH on the GPU:
 //   1. centroid bounds (two-level reduction, deterministic)
 //   2. 30-bit Morton codes (EncodeMorton3 bit layout: z above y above x)
-//   3. stable LSD radix sort of (code, index), 4 passes of 8 bits
+//   3. stable LSD radix sort of (code, index), 3 passes of 10 bits
 //   4. Karras hierarchy, one thread per internal node
-//   5. bottom-up AABB refit with per-node arrival counters
-//   6. 64-byte traversal nodes and 48-byte triangle records in leaf order
+//   5. boxes of aligned runs of 2^k leaves; a node covers consecutive leaves, so
+//      its box is the union of a few such runs
+//   6. 128-byte 4-wide nodes (64-byte binary nodes for width 2) and 48-byte
+//      triangle records in leaf order
 // Every step is integer or exact float min/max work, so the result is
 // bit-identical to the CPU restatement of the same algorithm.
 #include <hip/hip_runtime.h>
@@ -23,11 +25,9 @@
 namespace eos {
 namespace {
 
-constexpr int kSortThreads = 256;
-constexpr int kSortChunks = 16;                      // keys per block = 4096
-constexpr int kSortTile = kSortThreads * kSortChunks;
-constexpr int kWaves = kSortThreads / 64;
-constexpr int kRefitPasses = 64;                     // >= height of a Karras tree over 30-bit codes + index
+constexpr int kDigitBits = 10, kDigits = 1 << kDigitBits;
+constexpr int kSortWaves = 16, kSortThreads = 64 * kSortWaves;
+constexpr int kSortBlocks = 256;                     // at most: a workgroup per CU
 
 __device__ __forceinline__ uint32_t part1by2(uint32_t x) {
     x &= 0x000003ffu;
@@ -45,12 +45,45 @@ __device__ __forceinline__ void centroid(const float* __restrict__ v, size_t i, 
     for (int k = 0; k < 3; ++k) c[k] = ((t[k] + t[3 + k]) + t[6 + k]) / 3.0f;
 }
 
+// World-space vertices of a transformed triangle (M * (v, 1), glm's order of
+// operations; the rows of M are kXfM..kXfM+2 of its record), the input vertices
+// for the rest.  Keys and boxes of the build come from these; the triangle
+// records keep the local vertices, as rays meet triangles in local space.
+__device__ __forceinline__ void world_vertices(const float* __restrict__ t, int x, const float4* __restrict__ xf,
+                                               int n_xf, float w[9]) {
+    if (x < 0 || x >= n_xf) {
+#pragma unroll
+        for (int k = 0; k < 9; ++k) w[k] = t[k];
+        return;
+    }
+    const float4 r[3] = {xf[kXfRows * (size_t)x + kXfM], xf[kXfRows * (size_t)x + kXfM + 1],
+                         xf[kXfRows * (size_t)x + kXfM + 2]};
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+            w[3 * c + k] = (r[k].x * t[3 * c] + r[k].y * t[3 * c + 1]) + (r[k].z * t[3 * c + 2] + r[k].w * 1.0f);
+}
+
+// Centroid bounds of each workgroup's triangles.  XF: also writes the world-space
+// vertices of scenes with transformations.
+template <bool XF>
 __global__ __launch_bounds__(256) void k_cbounds_partial(const float* __restrict__ verts, int n,
+                                                         const int32_t* __restrict__ xi, const float4* __restrict__ xf,
+                                                         int n_xf, float* __restrict__ wverts,
                                                          float* __restrict__ part) {
     float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         float c[3];
-        centroid(verts, (size_t)i, c);
+        if (XF) {
+            float w[9];
+            world_vertices(verts + 9 * (size_t)i, xi[i], xf, n_xf, w);
+#pragma unroll
+            for (int k = 0; k < 9; ++k) wverts[9 * (size_t)i + k] = w[k];
+            centroid(w, 0, c);
+        } else {
+            centroid(verts, (size_t)i, c);
+        }
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
             lo[k] = fminf(lo[k], c[k]);
@@ -77,14 +110,20 @@ __global__ __launch_bounds__(256) void k_cbounds_partial(const float* __restrict
     if (threadIdx.x < 6) part[6 * blockIdx.x + threadIdx.x] = s[threadIdx.x][0];
 }
 
-__global__ __launch_bounds__(64) void k_cbounds_final(const float* __restrict__ part, int nparts,
-                                                      float* __restrict__ cb) {
-    // 6 lanes each reduce one component over all partials (min and max are exact).
-    int k = threadIdx.x;
-    if (k >= 6) return;
+// One wave per component over all partials (min and max are exact, so the order
+// does not matter; one lane per component walking them one after another took
+// 98 us at 1M triangles), and the build's error counters set to zero.
+__global__ __launch_bounds__(384) void k_cbounds_final(const float* __restrict__ part, int nparts,
+                                                       float* __restrict__ cb, int32_t* __restrict__ err) {
+    const int k = threadIdx.x >> 6, lane = threadIdx.x & 63;
     float r = k < 3 ? INFINITY : -INFINITY;
-    for (int b = 0; b < nparts; ++b) r = k < 3 ? fminf(r, part[6 * b + k]) : fmaxf(r, part[6 * b + k]);
-    cb[k] = r;
+    for (int b = lane; b < nparts; b += 64) r = k < 3 ? fminf(r, part[6 * b + k]) : fmaxf(r, part[6 * b + k]);
+    for (int off = 32; off > 0; off >>= 1) {
+        const float o = __shfl_xor(r, off);
+        r = k < 3 ? fminf(r, o) : fmaxf(r, o);
+    }
+    if (lane == 0) cb[k] = r;
+    if (threadIdx.x < 4) err[threadIdx.x] = 0;
 }
 
 __device__ __forceinline__ uint32_t quant10(float c, float lo, float hi) {
@@ -96,8 +135,7 @@ __device__ __forceinline__ uint32_t quant10(float c, float lo, float hi) {
 }
 
 __global__ __launch_bounds__(256) void k_morton(const float* __restrict__ verts, int n, const float* __restrict__ cb,
-                                                uint32_t* __restrict__ codes, uint32_t* __restrict__ keys,
-                                                int32_t* __restrict__ vals) {
+                                                uint32_t* __restrict__ codes) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     float c[3];
@@ -105,78 +143,159 @@ __global__ __launch_bounds__(256) void k_morton(const float* __restrict__ verts,
     uint32_t x = quant10(c[0], cb[0], cb[3]);
     uint32_t y = quant10(c[1], cb[1], cb[4]);
     uint32_t z = quant10(c[2], cb[2], cb[5]);
-    uint32_t code = (part1by2(z) << 2) + (part1by2(y) << 1) + part1by2(x);
-    codes[i] = code;
-    keys[i] = code;
-    vals[i] = i;
+    codes[i] = (part1by2(z) << 2) + (part1by2(y) << 1) + part1by2(x);
 }
 
-// ---- LSD radix sort, 8-bit digits -------------------------------------------
+// ---- LSD radix sort, 10-bit digits: three launches per pass --------------------
+// At most one workgroup of 16 waves per CU; each wave owns `seg` consecutive keys
+// (a multiple of 64) and counts and ranks them in its own row of LDS counters, so
+// the only barriers are around the counters, not between rounds of 256 keys.
+// 1M keys: four 8-bit passes of five launches 156 us, three passes like this 92.
+struct SortShape {
+    int blocks, seg;
+};
+inline SortShape sort_shape(size_t n) {
+    const size_t waves = (size_t)kSortBlocks * kSortWaves;
+    const size_t seg = ((n + waves - 1) / waves + 63) / 64 * 64;
+    return {(int)((n + seg * kSortWaves - 1) / (seg * kSortWaves)), (int)seg};
+}
+inline size_t sort_hist_bytes(const SortShape& sh) { return 4 * (size_t)kDigits * (size_t)(sh.blocks + 1); }
+
+// Digit counts of each workgroup, digit-major.
 __global__ __launch_bounds__(kSortThreads) void k_radix_hist(const uint32_t* __restrict__ keys, int n, int shift,
-                                                             uint32_t* __restrict__ hist, int nblocks) {
-    __shared__ uint32_t h[256];
+                                                             int seg, uint32_t* __restrict__ hist, int nblocks) {
+    __shared__ uint32_t h[kDigits];
     h[threadIdx.x] = 0;
     __syncthreads();
-    const int base = blockIdx.x * kSortTile;
-    const int end = min(n, base + kSortTile);
-    for (int i = base + threadIdx.x; i < end; i += kSortThreads) atomicAdd(&h[(keys[i] >> shift) & 255u], 1u);
+    const long long base = (long long)blockIdx.x * seg * kSortWaves;
+    const long long end = min((long long)n, base + (long long)seg * kSortWaves);
+    for (long long i = base + threadIdx.x; i < end; i += kSortThreads)
+        atomicAdd(&h[(keys[i] >> shift) & (kDigits - 1)], 1u);
     __syncthreads();
-    hist[threadIdx.x * nblocks + blockIdx.x] = h[threadIdx.x];
+    hist[(size_t)threadIdx.x * nblocks + blockIdx.x] = h[threadIdx.x];
+}
+static_assert(kDigits == kSortThreads, "a thread per digit");
+
+// A wave per digit: its counts become the exclusive prefix over the workgroups
+// (at most 256, four per lane), and its total.
+__global__ __launch_bounds__(256) void k_radix_scan(uint32_t* __restrict__ hist, int nblocks,
+                                                    uint32_t* __restrict__ totals) {
+    const int d = blockIdx.x * 4 + (int)(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    uint32_t* row = hist + (size_t)d * nblocks;
+    uint32_t v[4], t = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const int b = 4 * lane + k;
+        v[k] = b < nblocks ? row[b] : 0u;
+        t += v[k];
+    }
+    uint32_t x = t;
+    for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t y = __shfl_up(x, off);
+        if (lane >= off) x += y;
+    }
+    uint32_t run = x - t;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const int b = 4 * lane + k;
+        if (b < nblocks) row[b] = run;
+        run += v[k];
+    }
+    if (lane == 63) totals[d] = x;
+}
+static_assert(kSortBlocks <= 256, "four workgroups' counts per lane");
+
+// Exclusive scan of one value per thread over a workgroup of 1024 threads.
+__device__ __forceinline__ uint32_t block_scan_1024(uint32_t v, uint32_t* s_wave /* [16] */, uint32_t* total) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    uint32_t x = v;
+    for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t y = __shfl_up(x, off);
+        if (lane >= off) x += y;
+    }
+    if (lane == 63) s_wave[w] = x;
+    __syncthreads();
+    uint32_t before = 0, all = 0;
+    for (int k = 0; k < 16; ++k) {
+        before += k < w ? s_wave[k] : 0u;
+        all += s_wave[k];
+    }
+    if (total) *total = all;
+    return before + x - v;
 }
 
-// The digit-major histogram is scanned with the multi-block scan below.
-
-// Stable scatter: keys are taken in order, 256 per step; lanes holding the same
-// digit are matched with eight ballots, ranked by lane, and waves are ordered
-// by a per-digit prefix over the block's waves.
+// Stable scatter.  Each wave counts its keys' digits; a prefix over the digits,
+// the workgroups and the waves turns the counters into destinations; then each
+// wave walks its keys again in order, 64 at a time: lanes holding the same digit
+// are matched with ten ballots and ranked by lane.  vin null: the values are the
+// keys' indices.
 __global__ __launch_bounds__(kSortThreads) void k_radix_scatter(const uint32_t* __restrict__ kin,
                                                                 const int32_t* __restrict__ vin,
                                                                 uint32_t* __restrict__ kout, int32_t* __restrict__ vout,
-                                                                int n, int shift, const uint32_t* __restrict__ hist,
-                                                                int nblocks) {
-    __shared__ uint32_t running[256];
-    __shared__ uint32_t wcount[kWaves][256];
-    __shared__ uint32_t woff[kWaves][256];
-    const int tid = threadIdx.x;
-    const int wave = tid >> 6, lane = tid & 63;
-    running[tid] = hist[tid * nblocks + blockIdx.x];
-    const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-    const int base = blockIdx.x * kSortTile;
-    for (int ch = 0; ch < kSortChunks; ++ch) {
-        const int i = base + ch * kSortThreads + tid;
-        const bool valid = i < n;
-        uint32_t key = valid ? kin[i] : 0u;
-        int32_t val = valid ? vin[i] : 0;
-        uint32_t d = (key >> shift) & 255u;
+                                                                int n, int shift, int seg,
+                                                                const uint32_t* __restrict__ hist, int nblocks,
+                                                                const uint32_t* __restrict__ totals) {
+    __shared__ uint32_t cnt[kSortWaves][kDigits];
+    __shared__ uint32_t s_wave[16];
+    const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) wcount[wave][lane * 4 + j] = 0;
+    for (int k = 0; k < kSortWaves; ++k) cnt[k][tid] = 0;
+    __syncthreads();
+    const long long base = ((long long)blockIdx.x * kSortWaves + w) * seg;
+    const long long end = min((long long)n, base + seg);
+    for (long long i = base + lane; i < end; i += 64) atomicAdd(&cnt[w][(kin[i] >> shift) & (kDigits - 1)], 1u);
+    uint32_t run = block_scan_1024(totals[tid], s_wave, nullptr);   // its barrier ends the counting too
+    run += hist[(size_t)tid * nblocks + blockIdx.x];
+#pragma unroll
+    for (int k = 0; k < kSortWaves; ++k) {
+        const uint32_t c = cnt[k][tid];
+        cnt[k][tid] = run;
+        run += c;
+    }
+    __syncthreads();
+    volatile uint32_t* mine = cnt[w];
+    const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+    uint32_t key = 0;
+    int32_t val = 0;
+    auto load = [&](long long i) {
+        if (i < end) {
+            key = kin[i];
+            val = vin ? vin[i] : (int32_t)i;
+        }
+    };
+    load(base + lane);
+    for (long long i0 = base; i0 < end; i0 += 64) {
+        const bool valid = i0 + lane < end;
+        const uint32_t k = key;
+        const int32_t v = val;
+        load(i0 + 64 + lane);
+        const uint32_t d = (k >> shift) & (kDigits - 1);
         uint64_t peers = __ballot(valid);
 #pragma unroll
-        for (int bit = 0; bit < 8; ++bit) {
-            uint64_t b = __ballot((d >> bit) & 1u);
+        for (int bit = 0; bit < kDigitBits; ++bit) {
+            const uint64_t b = __ballot((d >> bit) & 1u);
             peers &= ((d >> bit) & 1u) ? b : ~b;
         }
         const uint32_t rank = __popcll(peers & lt);
-        __syncthreads();
-        if (valid && rank == 0) wcount[wave][d] = __popcll(peers);
-        __syncthreads();
-        {
-            uint32_t acc = running[tid];
-#pragma unroll
-            for (int w = 0; w < kWaves; ++w) {
-                woff[w][tid] = acc;
-                acc += wcount[w][tid];
-            }
-            running[tid] = acc;
-        }
-        __syncthreads();
+        const uint32_t off = mine[d];
+        __builtin_amdgcn_wave_barrier();
+        if (valid && rank == 0) mine[d] = off + __popcll(peers);
+        __builtin_amdgcn_wave_barrier();
         if (valid) {
-            uint32_t dst = woff[wave][d] + rank;
-            kout[dst] = key;
-            vout[dst] = val;
+            kout[off + rank] = k;
+            vout[off + rank] = v;
         }
-        __syncthreads();
     }
+}
+
+// One pass over n keys (hist: sort_hist_bytes).
+void radix_pass(hipStream_t S, const SortShape& sh, const uint32_t* kin, const int32_t* vin, uint32_t* kout,
+                int32_t* vout, int n, int shift, uint32_t* hist) {
+    uint32_t* totals = hist + (size_t)kDigits * sh.blocks;
+    hipLaunchKernelGGL(k_radix_hist, dim3(sh.blocks), dim3(kSortThreads), 0, S, kin, n, shift, sh.seg, hist, sh.blocks);
+    hipLaunchKernelGGL(k_radix_scan, dim3(kDigits / 4), dim3(256), 0, S, hist, sh.blocks, totals);
+    hipLaunchKernelGGL(k_radix_scatter, dim3(sh.blocks), dim3(kSortThreads), 0, S, kin, vin, kout, vout, n, shift,
+                       sh.seg, hist, sh.blocks, totals);
 }
 
 // ---- Karras hierarchy --------------------------------------------------------
@@ -190,6 +309,7 @@ __device__ __forceinline__ int delta(const uint32_t* __restrict__ k, int n, int 
 __global__ __launch_bounds__(256) void k_karras(const uint32_t* __restrict__ k, int n, int2* __restrict__ kchild,
                                                 int32_t* __restrict__ kparent, int2* __restrict__ fl) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i == 0) kparent[0] = -1;   // the root, or the only leaf
     if (i >= n - 1) return;
     const int d = (delta(k, n, i, i + 1) - delta(k, n, i, i - 1)) >= 0 ? 1 : -1;
     const int dmin = delta(k, n, i, i - d);
@@ -216,57 +336,129 @@ __global__ __launch_bounds__(256) void k_karras(const uint32_t* __restrict__ k, 
     kparent[right >= 0 ? right : (n - 1 + ~right)] = i;
 }
 
-__global__ void k_fill_i32(int32_t* __restrict__ p, int n, int32_t v) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = v;
-}
-
-__global__ void k_copy_i32(const int32_t* __restrict__ src, int32_t* __restrict__ dst, int n) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) dst[i] = src[i];
-}
-
-// Leaf boxes: exact min/max of the three vertices, one thread per sorted slot.
-__global__ __launch_bounds__(256) void k_leaf_boxes(const float* __restrict__ verts, const int32_t* __restrict__ perm,
-                                                    int n, float* __restrict__ lbox) {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= n) return;
-    const float* t = verts + 9 * (size_t)perm[s];
+// ---- boxes ------------------------------------------------------------------
+// A box is six floats: lo.xyz, hi.xyz.  Level k >= 1 of the pyramid holds the
+// boxes of the runs of 2^k leaves starting at multiples of 2^k, at entry
+// top - (top >> (k - 1)) on, top = the leaf count rounded up to a power of two;
+// level 0 is lbox.  (Boxing the tree level by level, each pass over every node
+// still open, took 64 launches, 0.74 ms of a 1.4 ms build of 1M triangles.)
+struct Box6 {
+    float v[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
+    __device__ __forceinline__ void add(const Box6& o) {
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        lbox[6 * (size_t)s + k] = fminf(fminf(t[k], t[3 + k]), t[6 + k]);
-        lbox[6 * (size_t)s + 3 + k] = fmaxf(fmaxf(t[k], t[3 + k]), t[6 + k]);
-    }
-}
-
-// One level-synchronous refit pass over the internal nodes.  done[i] is the
-// pass that boxed node i (0: not yet).  A node is boxed once both children are
-// leaves or were boxed in an EARLIER pass, so every box it reads was written by
-// an earlier kernel: no cross-workgroup ordering inside a launch is needed
-// (device-scope release/acquire per climbing thread costs L2 writebacks on a
-// multi-die part).  Passes = tree height; min/max are exact, so the result
-// does not depend on the schedule.  Once the root (node 0) is boxed every node
-// is, and the remaining passes return at once.
-__global__ __launch_bounds__(256) void k_refit_pass(const int2* __restrict__ kchild, int m, int pass,
-                                                    const float* __restrict__ lbox, float* __restrict__ ibox,
-                                                    int32_t* __restrict__ done) {
-    if (done[0] != 0) return;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < m && done[i] == 0) {
-        const int2 c = kchild[i];
-        const int d0 = c.x >= 0 ? done[c.x] : -1, d1 = c.y >= 0 ? done[c.y] : -1;
-        const bool r0 = c.x < 0 || (d0 > 0 && d0 < pass), r1 = c.y < 0 || (d1 > 0 && d1 < pass);
-        if (r0 && r1) {
-            const float* b0 = c.x >= 0 ? ibox + 6 * (size_t)c.x : lbox + 6 * (size_t)~c.x;
-            const float* b1 = c.y >= 0 ? ibox + 6 * (size_t)c.y : lbox + 6 * (size_t)~c.y;
-#pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                ibox[6 * (size_t)i + k] = fminf(b0[k], b1[k]);
-                ibox[6 * (size_t)i + 3 + k] = fmaxf(b0[3 + k], b1[3 + k]);
-            }
-            done[i] = pass;
+        for (int k = 0; k < 3; ++k) {
+            v[k] = fminf(v[k], o.v[k]);
+            v[3 + k] = fmaxf(v[3 + k], o.v[3 + k]);
         }
     }
+    __device__ __forceinline__ static Box6 load(const float* __restrict__ p, size_t i) {
+        Box6 b;
+#pragma unroll
+        for (int k = 0; k < 6; ++k) b.v[k] = p[6 * i + k];
+        return b;
+    }
+    __device__ __forceinline__ void store(float* __restrict__ p, size_t i) const {
+#pragma unroll
+        for (int k = 0; k < 6; ++k) p[6 * i + k] = v[k];
+    }
+};
+inline size_t pyramid_top(size_t n) {
+    size_t t = 1;
+    while (t < n) t *= 2;
+    return t;
+}
+__device__ __forceinline__ size_t pyramid_at(size_t top, int level, size_t i) { return top - (top >> (level - 1)) + i; }
+constexpr int kBoxBlock = 1024;   // leaves per workgroup of k_leaf_boxes (levels 1..10)
+
+// Leaf boxes (exact min/max of the three vertices of the sorted slots) and the
+// first ten levels of the pyramid: four leaves per lane, then lane shuffles, then
+// the four waves.
+__global__ __launch_bounds__(256) void k_leaf_boxes(const float* __restrict__ verts, const int32_t* __restrict__ perm,
+                                                    int n, float* __restrict__ lbox, float* __restrict__ pyr,
+                                                    size_t top) {
+    const size_t quad = (size_t)blockIdx.x * 256 + threadIdx.x;
+    Box6 b[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const size_t s = 4 * quad + q;
+        if (s < (size_t)n) {
+            const float* t = verts + 9 * (size_t)perm[s];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                b[q].v[k] = fminf(fminf(t[k], t[3 + k]), t[6 + k]);
+                b[q].v[3 + k] = fmaxf(fmaxf(t[k], t[3 + k]), t[6 + k]);
+            }
+            b[q].store(lbox, s);
+        }
+    }
+    b[0].add(b[1]);
+    b[2].add(b[3]);
+    if (4 * quad < (size_t)n) b[0].store(pyr, pyramid_at(top, 1, 2 * quad));
+    if (4 * quad + 2 < (size_t)n) b[2].store(pyr, pyramid_at(top, 1, 2 * quad + 1));
+    b[0].add(b[2]);
+    if (n > 2 && 4 * quad < (size_t)n) b[0].store(pyr, pyramid_at(top, 2, quad));
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    for (int level = 3; level <= 8; ++level) {
+        const int off = 1 << (level - 3);
+        Box6 o;
+#pragma unroll
+        for (int k = 0; k < 6; ++k) o.v[k] = __shfl_down(b[0].v[k], off);
+        b[0].add(o);   // right for the lanes that the next level reads
+        if ((lane & (2 * off - 1)) == 0 && (size_t)n > ((size_t)1 << (level - 1)) && 4 * quad < (size_t)n)
+            b[0].store(pyr, pyramid_at(top, level, quad >> (level - 2)));
+    }
+    __shared__ float s_box[6][4];
+    if (lane == 0)
+#pragma unroll
+        for (int k = 0; k < 6; ++k) s_box[k][w] = b[0].v[k];
+    __syncthreads();
+    if (threadIdx.x < 2) {
+        // level 9: one pair of waves per thread; level 10 by thread 0
+        Box6 r[2];
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            Box6 x, y;
+#pragma unroll
+            for (int k = 0; k < 6; ++k) {
+                x.v[k] = s_box[k][2 * q];
+                y.v[k] = s_box[k][2 * q + 1];
+            }
+            x.add(y);
+            r[q] = x;
+        }
+        const size_t first = (size_t)blockIdx.x * kBoxBlock + 512 * threadIdx.x;
+        if (n > 256 && first < (size_t)n) (threadIdx.x == 0 ? r[0] : r[1]).store(pyr, pyramid_at(top, 9, first >> 9));
+        r[0].add(r[1]);
+        if (threadIdx.x == 0 && n > 512) r[0].store(pyr, pyramid_at(top, 10, blockIdx.x));
+    }
+}
+
+// The levels above, in one workgroup (the eleventh has a box per 2,048 leaves).
+__global__ __launch_bounds__(1024) void k_pyramid_top(int n, float* pyr, size_t top) {
+    size_t below = ((size_t)n + 1023) / 1024;
+    for (int level = 11; below > 1; ++level) {
+        const size_t cnt = (below + 1) / 2;
+        for (size_t j = threadIdx.x; j < cnt; j += 1024) {
+            Box6 b = Box6::load(pyr, pyramid_at(top, level - 1, 2 * j));
+            if (2 * j + 1 < below) b.add(Box6::load(pyr, pyramid_at(top, level - 1, 2 * j + 1)));
+            b.store(pyr, pyramid_at(top, level, j));
+        }
+        __syncthreads();   // this workgroup's next level reads what it wrote
+        below = cnt;
+    }
+}
+
+// The box of leaves [l, r]: the fewest aligned runs that make it up.
+__device__ __forceinline__ Box6 range_box(const float* __restrict__ lbox, const float* __restrict__ pyr, size_t top,
+                                          int l, int r) {
+    Box6 b;
+    for (int i = l; i <= r;) {
+        int k = 31 - __clz(r - i + 1);
+        if (i != 0) k = min(k, __ffs(i) - 1);
+        b.add(k == 0 ? Box6::load(lbox, (size_t)i) : Box6::load(pyr, pyramid_at(top, k, (size_t)(i >> k))));
+        i += 1 << k;
+    }
+    return b;
 }
 
 __device__ __forceinline__ float inflate_pad(float lo, float hi, float eps) {
@@ -316,33 +508,6 @@ __global__ __launch_bounds__(256) void k_nodes(const int2* __restrict__ kchild, 
     nodes[i] = nd;
 }
 
-// World-space vertices of transformed triangles (M * (v, 1), glm's order of
-// operations; the rows of M are kXfM..kXfM+2 of the triangle's record), the
-// input vertices for the rest.  Keys and boxes of the build come from these;
-// the triangle records keep the local vertices, as rays meet triangles in
-// local space.
-__global__ __launch_bounds__(256) void k_world_verts(const float* __restrict__ verts, const int32_t* __restrict__ xi,
-                                                     int n, const float4* __restrict__ xf, int n_xf,
-                                                     float* __restrict__ out) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float* t = verts + 9 * (size_t)i;
-    float* w = out + 9 * (size_t)i;
-    const int x = xi[i];
-    if (x < 0 || x >= n_xf) {
-#pragma unroll
-        for (int k = 0; k < 9; ++k) w[k] = t[k];
-        return;
-    }
-    const float4 r[3] = {xf[kXfRows * (size_t)x + kXfM], xf[kXfRows * (size_t)x + kXfM + 1],
-                         xf[kXfRows * (size_t)x + kXfM + 2]};
-#pragma unroll
-    for (int c = 0; c < 3; ++c)
-#pragma unroll
-        for (int k = 0; k < 3; ++k)
-            w[3 * c + k] = (r[k].x * t[3 * c] + r[k].y * t[3 * c + 1]) + (r[k].z * t[3 * c + 2] + r[k].w * 1.0f);
-}
-
 // Triangle records in leaf order: geo = (v1, e1, e2, original index,
 // transformation index), shade = (n1 material, n2 transformation index, n3).
 __global__ __launch_bounds__(256) void k_tris(const float* __restrict__ verts, const float* __restrict__ normals,
@@ -376,88 +541,86 @@ __global__ __launch_bounds__(256) void k_tris(const float* __restrict__ verts, c
     shade[3 * (size_t)s + 2] = make_float4(nn[6], nn[7], nn[8], 0.0f);
 }
 
-// ---- exclusive scan of int32 (three phases: blocks of 1024, block sums, add) --
-constexpr int kScanBlock = 1024;
-
-__global__ __launch_bounds__(256) void k_scan_blocks(const int32_t* __restrict__ in, int32_t* __restrict__ out, int n,
-                                                     int32_t* __restrict__ sums) {
-    __shared__ int32_t s[256];
-    const int base = blockIdx.x * kScanBlock + threadIdx.x * 4;
-    int32_t v[4], t = 0;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        v[k] = base + k < n ? in[base + k] : 0;
-        t += v[k];
-    }
-    s[threadIdx.x] = t;
-    __syncthreads();
-    for (int off = 1; off < 256; off <<= 1) {
-        int32_t x = threadIdx.x >= (unsigned)off ? s[threadIdx.x - off] : 0;
-        __syncthreads();
-        s[threadIdx.x] += x;
-        __syncthreads();
-    }
-    int32_t run = s[threadIdx.x] - t;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        if (base + k < n) out[base + k] = run;
-        run += v[k];
-    }
-    if (threadIdx.x == 255) sums[blockIdx.x] = s[255];
-}
-
-__global__ __launch_bounds__(1024) void k_scan_sums(int32_t* __restrict__ sums, int nb) {
-    __shared__ int32_t s[1024];
-    __shared__ int32_t carry;
-    if (threadIdx.x == 0) carry = 0;
-    __syncthreads();
-    for (int b0 = 0; b0 < nb; b0 += 1024) {
-        const int i = b0 + threadIdx.x;
-        const int32_t v = i < nb ? sums[i] : 0;
-        s[threadIdx.x] = v;
-        __syncthreads();
-        for (int off = 1; off < 1024; off <<= 1) {
-            int32_t x = threadIdx.x >= (unsigned)off ? s[threadIdx.x - off] : 0;
-            __syncthreads();
-            s[threadIdx.x] += x;
-            __syncthreads();
-        }
-        if (i < nb) sums[i] = carry + s[threadIdx.x] - v;
-        __syncthreads();
-        if (threadIdx.x == 1023) carry += s[1023];
-        __syncthreads();
-    }
-}
-
-__global__ __launch_bounds__(256) void k_scan_add(int32_t* __restrict__ out, int n, const int32_t* __restrict__ sums) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i < n) out[i] += sums[i / kScanBlock];
-}
-
 // ---- 4-wide collapse -----------------------------------------------------------
 // A 4-wide node stands for every binary node that stays internal (range larger
-// than leaf_max) at even depth; nodes are numbered in binary index order.
-__global__ __launch_bounds__(256) void k_flags4(const int32_t* __restrict__ kparent, const int2* __restrict__ fl, int n,
-                                                int leaf_max, int32_t* __restrict__ flags) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n - 1) return;
-    const int2 r = fl[i];
-    int f = 0;
-    if (r.y - r.x + 1 > leaf_max) {
-        int depth = 0;
-        for (int p = kparent[i]; p >= 0 && depth < 128; p = kparent[p]) ++depth;
-        f = (depth & 1) == 0;
+// than leaf_max) at even depth; nodes are numbered in binary index order.  The
+// nodes that stand are kept as one bit each, 64 per word, and a count per 256,
+// which a scan turns into the first number of each 256.
+constexpr int kNodeBlock = 256;
+constexpr int kMaskWords = kNodeBlock / 64;
+
+// Every lane of the workgroup calls it: node's bit and the workgroup's count.
+__device__ __forceinline__ void keep_flags(bool stands, uint64_t* __restrict__ masks, int32_t* __restrict__ counts) {
+    __shared__ int32_t s_n[kMaskWords];
+    const uint64_t m = __ballot(stands);
+    const int w = threadIdx.x >> 6;
+    if ((threadIdx.x & 63) == 0) {
+        masks[(size_t)blockIdx.x * kMaskWords + w] = m;
+        s_n[w] = __popcll(m);
     }
-    flags[i] = f;
+    __syncthreads();
+    if (threadIdx.x == 0) counts[blockIdx.x] = s_n[0] + s_n[1] + s_n[2] + s_n[3];
+}
+static_assert(kMaskWords == 4, "four waves per workgroup");
+
+// The number of the nodes that stand before node g.
+__device__ __forceinline__ int number_of(const uint64_t* __restrict__ masks, const int32_t* __restrict__ first, int g) {
+    const uint64_t* m = masks + (size_t)(g / kNodeBlock) * kMaskWords;
+    const int w = (g / 64) % kMaskWords;
+    int c = first[g / kNodeBlock] + __popcll(m[w] & ((1ull << (g & 63)) - 1));
+    for (int k = 0; k < w; ++k) c += __popcll(m[k]);
+    return c;
+}
+__device__ __forceinline__ bool stands(const uint64_t* __restrict__ masks, int g) {
+    return (masks[(size_t)(g / kNodeBlock) * kMaskWords + (g / 64) % kMaskWords] >> (g & 63)) & 1ull;
+}
+
+// Exclusive scan of the counts in place (one workgroup, a stretch per thread) and
+// their sum.
+__global__ __launch_bounds__(1024) void k_scan_counts(int32_t* __restrict__ c, int nb, int32_t* __restrict__ total) {
+    __shared__ uint32_t s_wave[16];
+    const int per = (nb + 1023) / 1024;
+    const int b0 = min(nb, (int)threadIdx.x * per), b1 = min(nb, b0 + per);
+    uint32_t t = 0;
+    for (int b = b0; b < b1; ++b) t += (uint32_t)c[b];
+    uint32_t all = 0;
+    uint32_t run = block_scan_1024(t, s_wave, &all);
+    for (int b = b0; b < b1; ++b) {
+        const uint32_t v = (uint32_t)c[b];
+        c[b] = (int32_t)run;
+        run += v;
+    }
+    if (threadIdx.x == 0) *total = (int32_t)all;
+}
+
+// Boxes of the internal nodes, and which of them stand as 4-wide nodes.
+__global__ __launch_bounds__(kNodeBlock) void k_node_boxes(const int32_t* __restrict__ kparent,
+                                                           const int2* __restrict__ fl, int n, int leaf_max,
+                                                           const float* __restrict__ lbox,
+                                                           const float* __restrict__ pyr, size_t top,
+                                                           float* __restrict__ ibox, uint64_t* __restrict__ masks,
+                                                           int32_t* __restrict__ counts) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    bool f = false;
+    if (i < n - 1) {
+        const int2 r = fl[i];
+        range_box(lbox, pyr, top, r.x, r.y).store(ibox, (size_t)i);
+        if (r.y - r.x + 1 > leaf_max) {
+            int depth = 0;
+            for (int p = kparent[i]; p >= 0 && depth < 128; p = kparent[p]) ++depth;
+            f = (depth & 1) == 0;
+        }
+    }
+    keep_flags(f, masks, counts);
 }
 
 __global__ __launch_bounds__(256) void k_nodes4(const int2* __restrict__ kchild, const int2* __restrict__ fl,
                                                 const float* __restrict__ ibox, const float* __restrict__ lbox,
-                                                const float* __restrict__ cb, const int32_t* __restrict__ flags,
-                                                const int32_t* __restrict__ idx, int n, int leaf_max,
+                                                const float* __restrict__ cb, const uint64_t* __restrict__ masks,
+                                                const int32_t* __restrict__ first, int n, int leaf_max,
                                                 Node4* __restrict__ nodes4) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n - 1 || !flags[i]) return;
+    if (i >= n - 1 || !stands(masks, i)) return;
     float eps = 0.0f;
 #pragma unroll
     for (int k = 0; k < 6; ++k) eps = fmaxf(eps, fabsf(cb[k]));
@@ -501,7 +664,7 @@ __global__ __launch_bounds__(256) void k_nodes4(const int2* __restrict__ kchild,
                 ref[k] = leaf_ref(~g, 1);
             } else {
                 const int2 r = fl[g];
-                ref[k] = (r.y - r.x + 1 <= leaf_max) ? leaf_ref(r.x, r.y - r.x + 1) : idx[g];
+                ref[k] = (r.y - r.x + 1 <= leaf_max) ? leaf_ref(r.x, r.y - r.x + 1) : number_of(masks, first, g);
             }
         }
     }
@@ -514,7 +677,7 @@ __global__ __launch_bounds__(256) void k_nodes4(const int2* __restrict__ kchild,
     nd.hiz = make_float4(hi[2][0], hi[2][1], hi[2][2], hi[2][3]);
     nd.ref = make_int4(ref[0], ref[1], ref[2], ref[3]);
     nd.pad = make_int4(0, 0, 0, 0);
-    nodes4[idx[i]] = nd;
+    nodes4[number_of(masks, first, i)] = nd;
 }
 
 inline unsigned blocks(size_t n, unsigned t) { return (unsigned)((n + t - 1) / t); }
@@ -526,132 +689,102 @@ eos_status build_lbvh(eos_scene* s, int leaf_max, int width, eos_build_stats* st
     hipStream_t S = s->stream;
     s->built = false;
     s->batch_built = false;
+    s->nodes_valid = false;
     s->fb.rec_valid = 0;
     s->leaf_max = leaf_max;
     s->width = width;
     s->n_nodes4 = 0;
     const size_t un = (size_t)n, m = n > 0 ? un - 1 : 0;
-    const int nblocks = n > 0 ? (int)blocks(un, kSortTile) : 1;
+    const SortShape sh = sort_shape(std::max<size_t>(un, 1));
     const int nparts = n > 0 ? (int)std::min<size_t>(blocks(un, 256), 1024) : 1;
+    const size_t nblk = blocks(std::max<size_t>(m, 1), kNodeBlock);
+    const size_t top = pyramid_top(std::max<size_t>(un, 1));
     EOS_TRY(s->codes.ensure(4 * un));
     EOS_TRY(s->codes_sorted.ensure(4 * un));
     EOS_TRY(s->perm.ensure(4 * un));
     EOS_TRY(s->sort_tmp_k.ensure(4 * un));
     EOS_TRY(s->sort_tmp_v.ensure(4 * un));
-    EOS_TRY(s->sort_hist.ensure(2 * 4 * 256 * (size_t)nblocks));
-    EOS_TRY(s->scan_tmp.ensure(4 * blocks(256 * (size_t)nblocks, kScanBlock) + 4 * blocks(un, kScanBlock) + 8));
+    EOS_TRY(s->sort_hist.ensure(sort_hist_bytes(sh)));
     EOS_TRY(s->kchild.ensure(8 * m));
     EOS_TRY(s->kparent.ensure(4 * (2 * un)));
     EOS_TRY(s->first_last.ensure(8 * m));
     EOS_TRY(s->ibox.ensure(24 * m));
     EOS_TRY(s->lbox.ensure(24 * un));
-    EOS_TRY(s->flags.ensure(4 * m + 4));
+    EOS_TRY(s->pyramid.ensure(24 * top));
+    EOS_TRY(s->masks4.ensure(8 * kMaskWords * nblk + 4 * nblk));
     EOS_TRY(s->cbounds.ensure(64));
     EOS_TRY(s->bounds_part.ensure(24 * (size_t)nparts));
-    EOS_TRY(s->nodes.ensure(64 * m));
     EOS_TRY(s->shade.ensure(48 * un));
+    // Room for the 4-wide nodes before their number is known: at most one per
+    // internal node, and fewer than half a node per triangle when leaf_max >= 3.
+    // (A standing node has k standing children among its two to four slots; with
+    // none it holds at least four triangles, with one it has two other slots, with
+    // two at least one unless it has four.  Counting nodes by their children,
+    // S = 1 + S1 + 2 S2 + 3 S3 + 4 S4 and n >= 4 (1 + S2 + 2 S3 + 3 S4) + 2 S1.)
+    const bool four = n > leaf_max;
+    EOS_TRY(s->tree.ensure(s->tree_bytes(four ? (leaf_max >= 3 ? un / 2 : un) : 0)));
     EOS_HIP(hipEventRecord(s->ev[0], S));
-    int32_t* err = s->cbounds.as<int32_t>() + 8;
-    int32_t* root_pass = err + 1;   // refit pass that boxed the root (0: none); err[2]: bad transformation indices
-    hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, S, err, 3, 0);
+    float* cb = s->cbounds.as<float>();
+    int32_t* err = s->cbounds.as<int32_t>() + 8;   // [0] materials, [1] 4-wide nodes, [2] transformations out of range
     const bool xf = s->n_xf > 0;
+    int32_t herr[4] = {0, 0, 0, 0};
     if (n > 0) {
         const float* V = s->verts.as<float>();   // keys and boxes: world space
         if (xf) {
             EOS_TRY(s->wverts.ensure(36 * un));
-            hipLaunchKernelGGL(k_world_verts, dim3(blocks(un, 256)), dim3(256), 0, S, V,
-                               s->xf_index.as<const int32_t>(), n, s->xf.as<const float4>(), s->n_xf,
-                               s->wverts.as<float>());
+            hipLaunchKernelGGL(k_cbounds_partial<true>, dim3(nparts), dim3(256), 0, S, V, n,
+                               s->xf_index.as<const int32_t>(), s->xf.as<const float4>(), s->n_xf,
+                               s->wverts.as<float>(), s->bounds_part.as<float>());
             V = s->wverts.as<const float>();
+        } else {
+            hipLaunchKernelGGL(k_cbounds_partial<false>, dim3(nparts), dim3(256), 0, S, V, n, nullptr, nullptr, 0,
+                               nullptr, s->bounds_part.as<float>());
         }
-        float* cb = s->cbounds.as<float>();
-        hipLaunchKernelGGL(k_cbounds_partial, dim3(nparts), dim3(256), 0, S, V, n, s->bounds_part.as<float>());
-        hipLaunchKernelGGL(k_cbounds_final, dim3(1), dim3(64), 0, S, s->bounds_part.as<const float>(), nparts, cb);
-        uint32_t* kA = s->codes_sorted.as<uint32_t>();
-        int32_t* vA = s->perm.as<int32_t>();
-        uint32_t* kB = s->sort_tmp_k.as<uint32_t>();
-        int32_t* vB = s->sort_tmp_v.as<int32_t>();
-        hipLaunchKernelGGL(k_morton, dim3(blocks(un, 256)), dim3(256), 0, S, V, n, cb, s->codes.as<uint32_t>(), kA, vA);
+        hipLaunchKernelGGL(k_cbounds_final, dim3(1), dim3(384), 0, S, s->bounds_part.as<const float>(), nparts, cb, err);
+        uint32_t* codes = s->codes.as<uint32_t>();
+        hipLaunchKernelGGL(k_morton, dim3(blocks(un, 256)), dim3(256), 0, S, V, n, cb, codes);
+        uint32_t *kA = s->codes_sorted.as<uint32_t>(), *kB = s->sort_tmp_k.as<uint32_t>();
+        int32_t *vA = s->perm.as<int32_t>(), *vB = s->sort_tmp_v.as<int32_t>();
         uint32_t* H = s->sort_hist.as<uint32_t>();
-        uint32_t* H2 = H + 256 * (size_t)nblocks;
-        const int htot = 256 * nblocks, hb = (int)blocks((size_t)htot, kScanBlock);
-        int32_t* hsums = s->scan_tmp.as<int32_t>();
-        for (int pass = 0; pass < 4; ++pass) {
-            const int shift = 8 * pass;
-            const uint32_t* ki = (pass & 1) ? kB : kA;
-            const int32_t* vi = (pass & 1) ? vB : vA;
-            uint32_t* ko = (pass & 1) ? kA : kB;
-            int32_t* vo = (pass & 1) ? vA : vB;
-            hipLaunchKernelGGL(k_radix_hist, dim3(nblocks), dim3(kSortThreads), 0, S, ki, n, shift, H, nblocks);
-            // exclusive scan of the digit-major histogram into H2 (counts < 2^31)
-            hipLaunchKernelGGL(k_scan_blocks, dim3(hb), dim3(256), 0, S, reinterpret_cast<const int32_t*>(H),
-                               reinterpret_cast<int32_t*>(H2), htot, hsums);
-            hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(1024), 0, S, hsums, hb);
-            hipLaunchKernelGGL(k_scan_add, dim3(blocks(htot, 256)), dim3(256), 0, S, reinterpret_cast<int32_t*>(H2),
-                               htot, hsums);
-            hipLaunchKernelGGL(k_radix_scatter, dim3(nblocks), dim3(kSortThreads), 0, S, ki, vi, ko, vo, n, shift, H2,
-                               nblocks);
-        }
-        hipLaunchKernelGGL(k_fill_i32, dim3(blocks(2 * un, 256)), dim3(256), 0, S, s->kparent.as<int32_t>(),
-                           (int)(2 * un - 1), -1);
-        if (n > 1) {
-            hipLaunchKernelGGL(k_karras, dim3(blocks(m, 256)), dim3(256), 0, S, kA, n, s->kchild.as<int2>(),
-                               s->kparent.as<int32_t>(), s->first_last.as<int2>());
-            hipLaunchKernelGGL(k_fill_i32, dim3(blocks(m, 256)), dim3(256), 0, S, s->flags.as<int32_t>(), (int)m, 0);
-        }
-        hipLaunchKernelGGL(k_leaf_boxes, dim3(blocks(un, 256)), dim3(256), 0, S, V, vA, n, s->lbox.as<float>());
-        if (n > 1) {
-            for (int pass = 1; pass <= kRefitPasses; ++pass)
-                hipLaunchKernelGGL(k_refit_pass, dim3(blocks(m, 256)), dim3(256), 0, S, s->kchild.as<const int2>(),
-                                   (int)m, pass, s->lbox.as<const float>(), s->ibox.as<float>(),
-                                   s->flags.as<int32_t>());
-            // the root's pass number, 0 if the passes did not reach it
-            hipLaunchKernelGGL(k_copy_i32, dim3(1), dim3(64), 0, S, s->flags.as<const int32_t>(), root_pass, 1);
-        }
+        radix_pass(S, sh, codes, nullptr, kA, vA, n, 0, H);
+        radix_pass(S, sh, kA, vA, kB, vB, n, kDigitBits, H);
+        radix_pass(S, sh, kB, vB, kA, vA, n, 2 * kDigitBits, H);
+        hipLaunchKernelGGL(k_karras, dim3(blocks(un, 256)), dim3(256), 0, S, kA, n, s->kchild.as<int2>(),
+                           s->kparent.as<int32_t>(), s->first_last.as<int2>());
+        hipLaunchKernelGGL(k_leaf_boxes, dim3(blocks(un, kBoxBlock)), dim3(256), 0, S, V, vA, n, s->lbox.as<float>(),
+                           s->pyramid.as<float>(), top);
+        if (n > kBoxBlock) hipLaunchKernelGGL(k_pyramid_top, dim3(1), dim3(1024), 0, S, n, s->pyramid.as<float>(), top);
+        uint64_t* masks = s->masks4.as<uint64_t>();
+        int32_t* counts = reinterpret_cast<int32_t*>(masks + kMaskWords * nblk);
         if (n > 1)
-            hipLaunchKernelGGL(k_nodes, dim3(blocks(m, 256)), dim3(256), 0, S, s->kchild.as<const int2>(),
-                               s->first_last.as<const int2>(), s->ibox.as<const float>(), s->lbox.as<const float>(),
-                               cb, n, leaf_max, s->nodes.as<Node>());
-        if (n > leaf_max) {
-            // 4-wide collapse: flags, their exclusive scan (node numbers), node count, nodes
-            const int nb = (int)blocks(m, kScanBlock);
-            EOS_TRY(s->flags4.ensure(8 * m + 8));
-            EOS_TRY(s->scan_tmp.ensure(4 * (size_t)nb + 4));
-            int32_t* flags = s->flags4.as<int32_t>();
-            int32_t* idx = flags + m;
-            hipLaunchKernelGGL(k_flags4, dim3(blocks(m, 256)), dim3(256), 0, S, s->kparent.as<const int32_t>(),
-                               s->first_last.as<const int2>(), n, leaf_max, flags);
-            hipLaunchKernelGGL(k_scan_blocks, dim3(nb), dim3(256), 0, S, flags, idx, (int)m, s->scan_tmp.as<int32_t>());
-            hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(1024), 0, S, s->scan_tmp.as<int32_t>(), nb);
-            hipLaunchKernelGGL(k_scan_add, dim3(blocks(m, 256)), dim3(256), 0, S, idx, (int)m,
-                               s->scan_tmp.as<const int32_t>());
-            int32_t tail[2] = {0, 0};
-            EOS_HIP(hipMemcpyAsync(&tail[0], flags + (m - 1), 4, hipMemcpyDeviceToHost, S));
-            EOS_HIP(hipMemcpyAsync(&tail[1], idx + (m - 1), 4, hipMemcpyDeviceToHost, S));
-            EOS_HIP(hipStreamSynchronize(S));
-            s->n_nodes4 = tail[0] + tail[1];
-            EOS_TRY(s->tree.ensure(s->tree_bytes()));
+            hipLaunchKernelGGL(k_node_boxes, dim3((unsigned)nblk), dim3(kNodeBlock), 0, S,
+                               s->kparent.as<const int32_t>(), s->first_last.as<const int2>(), n, leaf_max,
+                               s->lbox.as<const float>(), s->pyramid.as<const float>(), top, s->ibox.as<float>(), masks,
+                               counts);
+        if (four) hipLaunchKernelGGL(k_scan_counts, dim3(1), dim3(1024), 0, S, counts, (int)nblk, err + 1);
+        if (four)
             hipLaunchKernelGGL(k_nodes4, dim3(blocks(m, 256)), dim3(256), 0, S, s->kchild.as<const int2>(),
                                s->first_last.as<const int2>(), s->ibox.as<const float>(), s->lbox.as<const float>(),
-                               cb, flags, idx, n, leaf_max, s->nodes4());
-        }
-        EOS_TRY(s->tree.ensure(s->tree_bytes()));
+                               cb, masks, counts, n, leaf_max, s->nodes4());
         hipLaunchKernelGGL(k_tris, dim3(blocks(un, 256)), dim3(256), 0, S, s->verts.as<const float>(),
                            s->normals.as<const float>(), s->matidx.as<const int32_t>(), vA, n, s->n_mat,
-                           xf ? s->xf_index.as<const int32_t>() : nullptr, s->n_xf, s->geo(),
-                           s->shade.as<float4>(), err);
+                           xf ? s->xf_index.as<const int32_t>() : nullptr, s->n_xf, s->geo(), s->shade.as<float4>(),
+                           err);
+        if (width == 2) EOS_TRY(make_binary_nodes(s));
+        EOS_HIP(hipEventRecord(s->ev[1], S));
+        EOS_HIP(hipMemcpyAsync(herr, err, sizeof herr, hipMemcpyDeviceToHost, S));
+        EOS_HIP(hipStreamSynchronize(S));
+        s->n_nodes4 = four ? herr[1] : 0;
+    } else {
+        EOS_HIP(hipEventRecord(s->ev[1], S));
+        EOS_HIP(hipStreamSynchronize(S));
     }
     EOS_HIP(hipGetLastError());
-    EOS_HIP(hipEventRecord(s->ev[1], S));
-    int32_t herr[3] = {0, 0, 0};
-    EOS_HIP(hipMemcpyAsync(herr, err, 12, hipMemcpyDeviceToHost, S));
-    EOS_HIP(hipStreamSynchronize(S));
     if (herr[0] != 0)
         return fail(EOS_ERR_INVALID, "eos_build_lbvh: " + std::to_string(herr[0]) + " material indices out of range");
     if (herr[2] != 0)
         return fail(EOS_ERR_INVALID,
                     "eos_build_lbvh: " + std::to_string(herr[2]) + " transformation indices out of range");
-    if (n > 1 && herr[1] == 0) return fail(EOS_ERR_STATE, "eos_build_lbvh: refit did not reach the root");
     float ms = 0.0f;
     EOS_HIP(hipEventElapsedTime(&ms, s->ev[0], s->ev[1]));
     if (n == 0) s->root = kDone;
@@ -671,13 +804,25 @@ eos_status build_lbvh(eos_scene* s, int leaf_max, int width, eos_build_stats* st
     return EOS_OK;
 }
 
+eos_status make_binary_nodes(eos_scene* s) {
+    const size_t m = s->n_tri > 1 ? (size_t)s->n_tri - 1 : 0;
+    if (s->nodes_valid || m == 0) return EOS_OK;
+    EOS_TRY(s->nodes.ensure(64 * m));
+    hipLaunchKernelGGL(k_nodes, dim3(blocks(m, 256)), dim3(256), 0, s->stream, s->kchild.as<const int2>(),
+                       s->first_last.as<const int2>(), s->ibox.as<const float>(), s->lbox.as<const float>(),
+                       s->cbounds.as<const float>(), s->n_tri, s->leaf_max, s->nodes.as<Node>());
+    EOS_HIP(hipGetLastError());
+    s->nodes_valid = true;
+    return EOS_OK;
+}
+
 }  // namespace eos
 
 // ---- many scenes in one launch sequence ---------------------------------------
 // The scenes' triangles are concatenated (scene s at global slots
 // [tri_off, tri_off + n)); every stage is one launch over all of them.  Each
 // scene keeps its own centroid bounds, Morton codes and Karras tree: the sort
-// orders (scene, code, index) -- four passes over the codes, then a stable pass
+// orders (scene, code, index) -- three passes over the codes, then a stable pass
 // over the scene index -- and the Karras kernel builds scene s's tree from the
 // keys of its own segment with its own local indices, so every per-scene array
 // is the one eos_build_lbvh_ex gives that scene alone, bit for bit.  Internal
@@ -720,28 +865,17 @@ __device__ __forceinline__ int seg_of(const int* __restrict__ off, int nseg, int
     return lo;
 }
 
-// World-space vertices, k_world_verts's arithmetic, into one concatenated array.
+// World-space vertices into one concatenated array.
 __global__ __launch_bounds__(256) void k_bworld(const BuildSeg* __restrict__ seg, const int* __restrict__ seg_tri,
                                                 int nseg, int N, float* __restrict__ out) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= N) return;
     const BuildSeg& S = seg[seg_of(seg_tri, nseg, i)];
     const int li = i - S.tri_off;
-    const float* t = S.verts + 9 * (size_t)li;
-    float* w = out + 9 * (size_t)i;
-    const int x = S.xi ? S.xi[li] : -1;
-    if (x < 0 || x >= S.n_xf) {
+    float w[9];
+    world_vertices(S.verts + 9 * (size_t)li, S.xi ? S.xi[li] : -1, S.xf, S.n_xf, w);
 #pragma unroll
-        for (int k = 0; k < 9; ++k) w[k] = t[k];
-        return;
-    }
-    const float4 r[3] = {S.xf[kXfRows * (size_t)x + kXfM], S.xf[kXfRows * (size_t)x + kXfM + 1],
-                         S.xf[kXfRows * (size_t)x + kXfM + 2]};
-#pragma unroll
-    for (int c = 0; c < 3; ++c)
-#pragma unroll
-        for (int k = 0; k < 3; ++k)
-            w[3 * c + k] = (r[k].x * t[3 * c] + r[k].y * t[3 * c + 1]) + (r[k].z * t[3 * c + 2] + r[k].w * 1.0f);
+    for (int k = 0; k < 9; ++k) out[9 * (size_t)i + k] = w[k];
 }
 
 // Partial centroid bounds: block b covers kBoundsChunk triangles of one scene.
@@ -783,8 +917,9 @@ __global__ __launch_bounds__(256) void k_bcb_partial(const float* __restrict__ W
 
 // One thread per (scene, component): min or max over the scene's partials.
 __global__ void k_bcb_final(const float* __restrict__ part, const BuildSeg* __restrict__ seg, int nseg,
-                            float* __restrict__ cb) {
+                            float* __restrict__ cb, int32_t* __restrict__ err) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t < 4) err[t] = 0;
     if (t >= 6 * nseg) return;
     const int sidx = t / 6, k = t - 6 * sidx;
     const BuildSeg& S = seg[sidx];
@@ -798,8 +933,7 @@ __global__ void k_bcb_final(const float* __restrict__ part, const BuildSeg* __re
 }
 
 __global__ __launch_bounds__(256) void k_bmorton(const float* __restrict__ W, const int* __restrict__ seg_tri, int nseg,
-                                                 int N, const float* __restrict__ cb, uint32_t* __restrict__ codes,
-                                                 uint32_t* __restrict__ keys, int32_t* __restrict__ vals) {
+                                                 int N, const float* __restrict__ cb, uint32_t* __restrict__ codes) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= N) return;
     const float* c6 = cb + 6 * seg_of(seg_tri, nseg, i);
@@ -808,10 +942,7 @@ __global__ __launch_bounds__(256) void k_bmorton(const float* __restrict__ W, co
     const uint32_t x = quant10(c[0], c6[0], c6[3]);
     const uint32_t y = quant10(c[1], c6[1], c6[4]);
     const uint32_t z = quant10(c[2], c6[2], c6[5]);
-    const uint32_t code = (part1by2(z) << 2) + (part1by2(y) << 1) + part1by2(x);
-    codes[i] = code;
-    keys[i] = code;
-    vals[i] = i;
+    codes[i] = (part1by2(z) << 2) + (part1by2(y) << 1) + part1by2(x);
 }
 
 // Sort keys of the scene pass: the scene of each element.
@@ -847,6 +978,7 @@ __global__ __launch_bounds__(256) void k_bkarras(const uint32_t* __restrict__ so
     const int sidx = seg_of(seg_tri, nseg, gi);
     const BuildSeg& S = seg[sidx];
     const int n = S.n, i = gi - S.tri_off;
+    if (i == 0) kparent[2 * (size_t)S.tri_off - sidx] = -1;
     if (i >= n - 1) return;
     const uint32_t* k = sorted + S.tri_off;
     const int d = (delta(k, n, i, i + 1) - delta(k, n, i, i - 1)) >= 0 ? 1 : -1;
@@ -873,47 +1005,6 @@ __global__ __launch_bounds__(256) void k_bkarras(const uint32_t* __restrict__ so
     int32_t* kp = kparent + (2 * (size_t)S.tri_off - sidx);
     kp[left >= 0 ? left : (n - 1 + ~left)] = i;
     kp[right >= 0 ? right : (n - 1 + ~right)] = i;
-}
-
-// k_refit_pass over every scene's internal nodes; a scene's root boxed counts
-// in *roots, and once every root is boxed the remaining passes return at once.
-__global__ __launch_bounds__(256) void k_brefit_pass(const int2* __restrict__ kchild, const BuildSeg* __restrict__ seg,
-                                                     const int* __restrict__ seg_node, int nseg, int M, int pass,
-                                                     const float* __restrict__ lbox, float* __restrict__ ibox,
-                                                     int32_t* __restrict__ done, int n_roots,
-                                                     int32_t* __restrict__ roots) {
-    if (*roots >= n_roots) return;
-    const int gi = blockIdx.x * blockDim.x + threadIdx.x;
-    if (gi >= M || done[gi] != 0) return;
-    const BuildSeg& S = seg[seg_of(seg_node, nseg, gi)];
-    const int2 c = kchild[gi];
-    const int g0 = S.node_off + c.x, g1 = S.node_off + c.y;
-    const int d0 = c.x >= 0 ? done[g0] : -1, d1 = c.y >= 0 ? done[g1] : -1;
-    const bool r0 = c.x < 0 || (d0 > 0 && d0 < pass), r1 = c.y < 0 || (d1 > 0 && d1 < pass);
-    if (r0 && r1) {
-        const float* b0 = c.x >= 0 ? ibox + 6 * (size_t)g0 : lbox + 6 * (size_t)(S.tri_off + ~c.x);
-        const float* b1 = c.y >= 0 ? ibox + 6 * (size_t)g1 : lbox + 6 * (size_t)(S.tri_off + ~c.y);
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            ibox[6 * (size_t)gi + k] = fminf(b0[k], b1[k]);
-            ibox[6 * (size_t)gi + 3 + k] = fmaxf(b0[3 + k], b1[3 + k]);
-        }
-        done[gi] = pass;
-        if (gi == S.node_off) atomicAdd(roots, 1);
-    }
-}
-
-// Leaf boxes of the concatenated sorted slots (k_leaf_boxes over the world vertices).
-__global__ __launch_bounds__(256) void k_bleaf_boxes(const float* __restrict__ W, const int32_t* __restrict__ vals,
-                                                     int N, float* __restrict__ lbox) {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= N) return;
-    const float* t = W + 9 * (size_t)vals[s];
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        lbox[6 * (size_t)s + k] = fminf(fminf(t[k], t[3 + k]), t[6 + k]);
-        lbox[6 * (size_t)s + 3 + k] = fmaxf(fmaxf(t[k], t[3 + k]), t[6 + k]);
-    }
 }
 
 // k_nodes per scene, into the scene's node array.
@@ -989,36 +1080,44 @@ __global__ __launch_bounds__(256) void k_btris(const int32_t* __restrict__ vals,
     S.shade[3 * (size_t)s + 2] = make_float4(nn[6], nn[7], nn[8], 0.0f);
 }
 
-// k_flags4 per scene (scenes of at most leaf_max triangles have no 4-wide nodes).
-__global__ __launch_bounds__(256) void k_bflags4(const int32_t* __restrict__ kparent, const int2* __restrict__ fl,
-                                                 const BuildSeg* __restrict__ seg, const int* __restrict__ seg_node,
-                                                 int nseg, int M, int leaf_max, int32_t* __restrict__ flags) {
+// k_node_boxes over every scene's nodes (scenes of at most leaf_max triangles have
+// no 4-wide nodes); the leaves are the concatenated sorted slots.
+__global__ __launch_bounds__(kNodeBlock) void k_bnode_boxes(const int32_t* __restrict__ kparent,
+                                                            const int2* __restrict__ fl,
+                                                            const BuildSeg* __restrict__ seg,
+                                                            const int* __restrict__ seg_node, int nseg, int M,
+                                                            int leaf_max, const float* __restrict__ lbox,
+                                                            const float* __restrict__ pyr, size_t top,
+                                                            float* __restrict__ ibox, uint64_t* __restrict__ masks,
+                                                            int32_t* __restrict__ counts) {
     const int gi = blockIdx.x * blockDim.x + threadIdx.x;
-    if (gi >= M) return;
-    const int sidx = seg_of(seg_node, nseg, gi);
-    const BuildSeg& S = seg[sidx];
-    const int2 r = fl[gi];
-    int f = 0;
-    if (S.n > leaf_max && r.y - r.x + 1 > leaf_max) {
-        const int32_t* kp = kparent + (2 * (size_t)S.tri_off - sidx);
-        int depth = 0;
-        for (int p = kp[gi - S.node_off]; p >= 0 && depth < 128; p = kp[p]) ++depth;
-        f = (depth & 1) == 0;
+    bool f = false;
+    if (gi < M) {
+        const int sidx = seg_of(seg_node, nseg, gi);
+        const BuildSeg& S = seg[sidx];
+        const int2 r = fl[gi];
+        range_box(lbox, pyr, top, S.tri_off + r.x, S.tri_off + r.y).store(ibox, (size_t)gi);
+        if (S.n > leaf_max && r.y - r.x + 1 > leaf_max) {
+            const int32_t* kp = kparent + (2 * (size_t)S.tri_off - sidx);
+            int depth = 0;
+            for (int p = kp[gi - S.node_off]; p >= 0 && depth < 128; p = kp[p]) ++depth;
+            f = (depth & 1) == 0;
+        }
     }
-    flags[gi] = f;
+    keep_flags(f, masks, counts);
 }
 
 // Per scene: 4-wide node count and global number of its first node.
-__global__ void k_bcount4(const int32_t* __restrict__ flags, const int32_t* __restrict__ idx,
+__global__ void k_bcount4(const uint64_t* __restrict__ masks, const int32_t* __restrict__ first,
                           const BuildSeg* __restrict__ seg, int nseg, int32_t* __restrict__ out) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= nseg) return;
     const BuildSeg& S = seg[t];
     int count = 0, base = 0;
     if (S.n > 1) {
-        const int first = S.node_off, last = S.node_off + S.n - 2;
-        base = idx[first];
-        count = idx[last] + flags[last] - base;
+        const int last = S.node_off + S.n - 2;
+        base = number_of(masks, first, S.node_off);
+        count = number_of(masks, first, last) + (stands(masks, last) ? 1 : 0) - base;
     }
     out[2 * t] = count;
     out[2 * t + 1] = base;
@@ -1027,11 +1126,11 @@ __global__ void k_bcount4(const int32_t* __restrict__ flags, const int32_t* __re
 // k_nodes4 per scene, numbered within the scene.
 __global__ __launch_bounds__(256) void k_bnodes4(const int2* __restrict__ kchild, const int2* __restrict__ fl,
                                                  const float* __restrict__ ibox, const float* __restrict__ lbox,
-                                                 const float* __restrict__ cbs, const int32_t* __restrict__ flags,
-                                                 const int32_t* __restrict__ idx, const BuildSeg* __restrict__ seg,
+                                                 const float* __restrict__ cbs, const uint64_t* __restrict__ masks,
+                                                 const int32_t* __restrict__ first, const BuildSeg* __restrict__ seg,
                                                  const int* __restrict__ seg_node, int nseg, int M, int leaf_max) {
     const int gi = blockIdx.x * blockDim.x + threadIdx.x;
-    if (gi >= M || !flags[gi]) return;
+    if (gi >= M || !stands(masks, gi)) return;
     const int sidx = seg_of(seg_node, nseg, gi);
     const BuildSeg& S = seg[sidx];
     const float* cb = cbs + 6 * sidx;
@@ -1078,7 +1177,7 @@ __global__ __launch_bounds__(256) void k_bnodes4(const int2* __restrict__ kchild
                 ref[k] = leaf_ref(~g, 1);
             } else {
                 const int2 r = fl[S.node_off + g];
-                ref[k] = (r.y - r.x + 1 <= leaf_max) ? leaf_ref(r.x, r.y - r.x + 1) : idx[S.node_off + g] - S.base4;
+                ref[k] = (r.y - r.x + 1 <= leaf_max) ? leaf_ref(r.x, r.y - r.x + 1) : number_of(masks, first, S.node_off + g) - S.base4;
             }
         }
     }
@@ -1091,13 +1190,13 @@ __global__ __launch_bounds__(256) void k_bnodes4(const int2* __restrict__ kchild
     nd.hiz = make_float4(hi[2][0], hi[2][1], hi[2][2], hi[2][3]);
     nd.ref = make_int4(ref[0], ref[1], ref[2], ref[3]);
     nd.pad = make_int4(0, 0, 0, 0);
-    S.nodes4[idx[gi] - S.base4] = nd;
+    S.nodes4[number_of(masks, first, gi) - S.base4] = nd;
 }
 
 // Scratch of the batched build (per process; calls must not overlap).
 struct BatchBuild {
-    DevBuf table, offs, W, part, cb, codes, kA, vA, kB, vB, sorted, hist, scan, kchild, kparent, fl, lbox, ibox,
-        done, flags4, counts, misc;
+    DevBuf table, offs, W, part, cb, codes, kA, vA, kB, vB, sorted, hist, kchild, kparent, fl, lbox, ibox,
+        pyramid, masks4, counts, misc;
     hipEvent_t ev[2] = {nullptr, nullptr};
 };
 BatchBuild g_bbuild;
@@ -1115,7 +1214,7 @@ eos_status build_lbvh_batch(eos_scene* const* scenes, int n_scenes, int leaf_max
     std::vector<BuildSeg> segs;
     std::vector<int> seg_scene, seg_tri, seg_node, seg_blk;
     size_t N = 0;
-    int nblk = 0, n_roots = 0;
+    int nblk = 0;
     for (int i = 0; i < n_scenes; ++i) {
         eos_scene* s = scenes[i];
         s->built = false;
@@ -1124,6 +1223,7 @@ eos_status build_lbvh_batch(eos_scene* const* scenes, int n_scenes, int leaf_max
         s->width = width;
         s->n_nodes4 = 0;
         s->batch_built = true;
+        s->nodes_valid = true;
         const size_t un = (size_t)s->n_tri;
         if (un == 0) continue;
         if (N + un > (size_t)INT_MAX / 2)
@@ -1156,7 +1256,6 @@ eos_status build_lbvh_batch(eos_scene* const* scenes, int n_scenes, int leaf_max
         seg_node.push_back(g.node_off);
         seg_blk.push_back(g.blk_off);
         nblk += (int)((un + kBoundsChunk - 1) / kBoundsChunk);
-        n_roots += un > 1 ? 1 : 0;
         N += un;
     }
     const int nseg = (int)segs.size();
@@ -1169,7 +1268,8 @@ eos_status build_lbvh_batch(eos_scene* const* scenes, int n_scenes, int leaf_max
     if (nseg > 0) {
         const size_t M = N - (size_t)nseg;       // internal nodes of every scene
         const int Ni = (int)N, Mi = (int)M;
-        const int nblocks = (int)blocks(N, kSortTile);
+        const SortShape sh = sort_shape(N);
+        const size_t top = pyramid_top(N), mblk = blocks(std::max<size_t>(M, 1), kNodeBlock);
         EOS_TRY(B.table.ensure(sizeof(BuildSeg) * nseg));
         EOS_TRY(B.offs.ensure(4 * 3 * (size_t)nseg));
         EOS_TRY(B.W.ensure(36 * N));
@@ -1181,15 +1281,14 @@ eos_status build_lbvh_batch(eos_scene* const* scenes, int n_scenes, int leaf_max
         EOS_TRY(B.kB.ensure(4 * N));
         EOS_TRY(B.vB.ensure(4 * N));
         EOS_TRY(B.sorted.ensure(4 * N));
-        EOS_TRY(B.hist.ensure(2 * 4 * 256 * (size_t)nblocks));
-        EOS_TRY(B.scan.ensure(4 * blocks(256 * (size_t)nblocks, kScanBlock) + 4 * blocks(N, kScanBlock) + 8));
+        EOS_TRY(B.hist.ensure(sort_hist_bytes(sh)));
+        EOS_TRY(B.pyramid.ensure(24 * top));
+        EOS_TRY(B.masks4.ensure(8 * kMaskWords * mblk + 4 * mblk));
         EOS_TRY(B.kchild.ensure(8 * M + 8));
         EOS_TRY(B.kparent.ensure(4 * (2 * N)));
         EOS_TRY(B.fl.ensure(8 * M + 8));
         EOS_TRY(B.lbox.ensure(24 * N));
         EOS_TRY(B.ibox.ensure(24 * M + 24));
-        EOS_TRY(B.done.ensure(4 * M + 4));
-        EOS_TRY(B.flags4.ensure(8 * M + 8));
         EOS_TRY(B.counts.ensure(8 * (size_t)nseg));
         EOS_TRY(B.misc.ensure(64));
         std::vector<int> offs;
@@ -1202,75 +1301,54 @@ eos_status build_lbvh_batch(eos_scene* const* scenes, int n_scenes, int leaf_max
         const int* o_tri = B.offs.as<const int>();
         const int* o_node = o_tri + nseg;
         const int* o_blk = o_node + nseg;
-        int32_t* err = B.misc.as<int32_t>();           // [0] materials, [1] roots boxed, [2] transformations
-        hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, S, err, 4, 0);
+        int32_t* err = B.misc.as<int32_t>();           // [0] materials, [1] 4-wide nodes, [2] transformations
         float* W = B.W.as<float>();
         hipLaunchKernelGGL(k_bworld, dim3(blocks(N, 256)), dim3(256), 0, S, T, o_tri, nseg, Ni, W);
         hipLaunchKernelGGL(k_bcb_partial, dim3(nblk), dim3(256), 0, S, W, T, o_blk, nseg, B.part.as<float>());
         hipLaunchKernelGGL(k_bcb_final, dim3(blocks(6 * (size_t)nseg, 64)), dim3(64), 0, S, B.part.as<const float>(),
-                           T, nseg, B.cb.as<float>());
+                           T, nseg, B.cb.as<float>(), err);
         uint32_t* kA = B.kA.as<uint32_t>();
         int32_t* vA = B.vA.as<int32_t>();
         uint32_t* kB = B.kB.as<uint32_t>();
         int32_t* vB = B.vB.as<int32_t>();
+        uint32_t* codes = B.codes.as<uint32_t>();
         hipLaunchKernelGGL(k_bmorton, dim3(blocks(N, 256)), dim3(256), 0, S, W, o_tri, nseg, Ni, B.cb.as<const float>(),
-                           B.codes.as<uint32_t>(), kA, vA);
+                           codes);
+        // three passes over the codes, then one (two beyond 1,024 scenes) over the scene index
         uint32_t* H = B.hist.as<uint32_t>();
-        uint32_t* H2 = H + 256 * (size_t)nblocks;
-        const int htot = 256 * nblocks, hb = (int)blocks((size_t)htot, kScanBlock);
-        int32_t* hsums = B.scan.as<int32_t>();
-        // four passes over the codes, then one (two beyond 256 scenes) over the scene index
-        const int scene_passes = nseg > 256 ? 2 : 1;
-        for (int pass = 0; pass < 4 + scene_passes; ++pass) {
-            const int shift = pass < 4 ? 8 * pass : 8 * (pass - 4);
-            const uint32_t* ki = (pass & 1) ? kB : kA;
-            const int32_t* vi = (pass & 1) ? vB : vA;
-            uint32_t* ko = (pass & 1) ? kA : kB;
-            int32_t* vo = (pass & 1) ? vA : vB;
-            if (pass == 4)   // keys of the scene passes: each element's scene (its values move with it)
-                hipLaunchKernelGGL(k_bscene_keys, dim3(blocks(N, 256)), dim3(256), 0, S, vi, o_tri, nseg, Ni,
-                                   const_cast<uint32_t*>(ki));
-            hipLaunchKernelGGL(k_radix_hist, dim3(nblocks), dim3(kSortThreads), 0, S, ki, Ni, shift, H, nblocks);
-            hipLaunchKernelGGL(k_scan_blocks, dim3(hb), dim3(256), 0, S, reinterpret_cast<const int32_t*>(H),
-                               reinterpret_cast<int32_t*>(H2), htot, hsums);
-            hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(1024), 0, S, hsums, hb);
-            hipLaunchKernelGGL(k_scan_add, dim3(blocks(htot, 256)), dim3(256), 0, S, reinterpret_cast<int32_t*>(H2),
-                               htot, hsums);
-            hipLaunchKernelGGL(k_radix_scatter, dim3(nblocks), dim3(kSortThreads), 0, S, ki, vi, ko, vo, Ni, shift, H2,
-                               nblocks);
+        radix_pass(S, sh, codes, nullptr, kA, vA, Ni, 0, H);
+        radix_pass(S, sh, kA, vA, kB, vB, Ni, kDigitBits, H);
+        radix_pass(S, sh, kB, vB, kA, vA, Ni, 2 * kDigitBits, H);
+        hipLaunchKernelGGL(k_bscene_keys, dim3(blocks(N, 256)), dim3(256), 0, S, vA, o_tri, nseg, Ni, kA);
+        radix_pass(S, sh, kA, vA, kB, vB, Ni, 0, H);
+        const int32_t* vS = vB;
+        if (nseg > kDigits) {
+            radix_pass(S, sh, kB, vB, kA, vA, Ni, kDigitBits, H);
+            vS = vA;
         }
-        const int32_t* vS = ((4 + scene_passes) & 1) ? vB : vA;   // values after the last pass
         uint32_t* sorted = B.sorted.as<uint32_t>();
         hipLaunchKernelGGL(k_bgather, dim3(blocks(N, 256)), dim3(256), 0, S, vS, B.codes.as<const uint32_t>(), T, o_tri,
                            nseg, Ni, sorted);
         int32_t* kparent = B.kparent.as<int32_t>();
-        hipLaunchKernelGGL(k_fill_i32, dim3(blocks(2 * N, 256)), dim3(256), 0, S, kparent, (int)(2 * N), -1);
         int2* kchild = B.kchild.as<int2>();
         int2* fl = B.fl.as<int2>();
         hipLaunchKernelGGL(k_bkarras, dim3(blocks(N, 256)), dim3(256), 0, S, sorted, T, o_tri, nseg, Ni, kchild,
                            kparent, fl);
-        hipLaunchKernelGGL(k_bleaf_boxes, dim3(blocks(N, 256)), dim3(256), 0, S, W, vS, Ni, B.lbox.as<float>());
+        hipLaunchKernelGGL(k_leaf_boxes, dim3(blocks(N, kBoxBlock)), dim3(256), 0, S, W, vS, Ni, B.lbox.as<float>(),
+                           B.pyramid.as<float>(), top);
+        if (Ni > kBoxBlock)
+            hipLaunchKernelGGL(k_pyramid_top, dim3(1), dim3(1024), 0, S, Ni, B.pyramid.as<float>(), top);
+        uint64_t* masks = B.masks4.as<uint64_t>();
+        int32_t* first4 = reinterpret_cast<int32_t*>(masks + kMaskWords * mblk);
         if (M > 0) {
-            hipLaunchKernelGGL(k_fill_i32, dim3(blocks(M, 256)), dim3(256), 0, S, B.done.as<int32_t>(), Mi, 0);
-            for (int pass = 1; pass <= kRefitPasses; ++pass)
-                hipLaunchKernelGGL(k_brefit_pass, dim3(blocks(M, 256)), dim3(256), 0, S, kchild, T, o_node, nseg, Mi,
-                                   pass, B.lbox.as<const float>(), B.ibox.as<float>(), B.done.as<int32_t>(), n_roots,
-                                   err + 1);
+            hipLaunchKernelGGL(k_bnode_boxes, dim3((unsigned)mblk), dim3(kNodeBlock), 0, S, kparent, fl, T, o_node,
+                               nseg, Mi, leaf_max, B.lbox.as<const float>(), B.pyramid.as<const float>(), top,
+                               B.ibox.as<float>(), masks, first4);
             hipLaunchKernelGGL(k_bnodes, dim3(blocks(M, 256)), dim3(256), 0, S, kchild, fl, B.ibox.as<const float>(),
                                B.lbox.as<const float>(), B.cb.as<const float>(), T, o_node, nseg, Mi, leaf_max);
-        }
-        int32_t* flags = B.flags4.as<int32_t>();
-        int32_t* idx = flags + M + 1;
-        if (M > 0) {
-            // 4-wide collapse: flags, one exclusive scan over every scene's nodes, per-scene counts
-            const int nb = (int)blocks(M, kScanBlock);
-            EOS_TRY(B.scan.ensure(4 * (size_t)nb + 4));
-            hipLaunchKernelGGL(k_bflags4, dim3(blocks(M, 256)), dim3(256), 0, S, kparent, fl, T, o_node, nseg, Mi,
-                               leaf_max, flags);
-            hipLaunchKernelGGL(k_scan_blocks, dim3(nb), dim3(256), 0, S, flags, idx, Mi, B.scan.as<int32_t>());
-            hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(1024), 0, S, B.scan.as<int32_t>(), nb);
-            hipLaunchKernelGGL(k_scan_add, dim3(blocks(M, 256)), dim3(256), 0, S, idx, Mi, B.scan.as<const int32_t>());
-            hipLaunchKernelGGL(k_bcount4, dim3(blocks((size_t)nseg, 64)), dim3(64), 0, S, flags, idx, T, nseg,
+            // 4-wide collapse: one numbering over every scene's nodes, per-scene counts
+            hipLaunchKernelGGL(k_scan_counts, dim3(1), dim3(1024), 0, S, first4, (int)mblk, err + 1);
+            hipLaunchKernelGGL(k_bcount4, dim3(blocks((size_t)nseg, 64)), dim3(64), 0, S, masks, first4, T, nseg,
                                B.counts.as<int32_t>());
             EOS_HIP(hipMemcpyAsync(cnt4.data(), B.counts.ptr, 8 * (size_t)nseg, hipMemcpyDeviceToHost, S));
             EOS_HIP(hipStreamSynchronize(S));
@@ -1278,7 +1356,7 @@ eos_status build_lbvh_batch(eos_scene* const* scenes, int n_scenes, int leaf_max
         for (int k = 0; k < nseg; ++k) {
             eos_scene* s = scenes[seg_scene[k]];
             s->n_nodes4 = cnt4[2 * k];
-            EOS_TRY(s->tree.ensure(s->tree_bytes()));
+            EOS_TRY(s->tree.ensure(s->tree_bytes((size_t)s->n_nodes4)));
             segs[k].nodes4 = s->nodes4();
             segs[k].geo = s->geo();
             segs[k].base4 = cnt4[2 * k + 1];
@@ -1286,7 +1364,7 @@ eos_status build_lbvh_batch(eos_scene* const* scenes, int n_scenes, int leaf_max
         EOS_HIP(hipMemcpyAsync(B.table.ptr, segs.data(), sizeof(BuildSeg) * nseg, hipMemcpyHostToDevice, S));
         if (M > 0)
             hipLaunchKernelGGL(k_bnodes4, dim3(blocks(M, 256)), dim3(256), 0, S, kchild, fl, B.ibox.as<const float>(),
-                               B.lbox.as<const float>(), B.cb.as<const float>(), flags, idx, T, o_node, nseg, Mi,
+                               B.lbox.as<const float>(), B.cb.as<const float>(), masks, first4, T, o_node, nseg, Mi,
                                leaf_max);
         hipLaunchKernelGGL(k_btris, dim3(blocks(N, 256)), dim3(256), 0, S, vS, T, o_tri, nseg, Ni, err);
         EOS_HIP(hipGetLastError());
@@ -1299,7 +1377,6 @@ eos_status build_lbvh_batch(eos_scene* const* scenes, int n_scenes, int leaf_max
     if (herr[2] != 0)
         return fail(EOS_ERR_INVALID,
                     "eos_build_lbvh_batch: " + std::to_string(herr[2]) + " transformation indices out of range");
-    if (herr[1] != n_roots) return fail(EOS_ERR_STATE, "eos_build_lbvh_batch: refit did not reach every root");
     float ms = 0.0f;
     EOS_HIP(hipEventElapsedTime(&ms, B.ev[0], B.ev[1]));
     for (int i = 0; i < n_scenes; ++i) {

@@ -1164,9 +1164,9 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(XF ? 4 : 5))
         const Node4* __restrict__ nodes4 = a.sc.nodes4;
         const float4* __restrict__ geo = a.sc.geo;
         const float4* __restrict__ xf = a.sc.xf;
-        // the 4-wide nodes and the geometry records lie in one allocation
-        const char* const tree = reinterpret_cast<const char*>(a.sc.nodes4);
-        const uint32_t geo_off = (uint32_t)(reinterpret_cast<const char*>(a.sc.geo) - tree);
+        // the geometry records and the 4-wide nodes lie in one allocation
+        const char* const tree = reinterpret_cast<const char*>(a.sc.geo);
+        const uint32_t node_off = (uint32_t)(reinterpret_cast<const char*>(a.sc.nodes4) - tree);
         int item = -1;
         size_t out_idx = 0;
         Fetch f = fetch_start(a, n);
@@ -1312,7 +1312,7 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(XF ? 4 : 5))
                                                       : reinterpret_cast<const char*>(geo + 3 * (size_t)s0);
                                 fetch([p](int off) { return *reinterpret_cast<const float4*>(p + off); });
                             } else {
-                                const uint32_t b = inner ? (uint32_t)cur << 7 : geo_off + 48u * (uint32_t)s0;
+                                const uint32_t b = inner ? node_off + ((uint32_t)cur << 7) : 48u * (uint32_t)s0;
                                 fetch([tree, b](int off) {
                                     return *reinterpret_cast<const float4*>(tree + (uint32_t)(b + (uint32_t)off));
                                 });
