@@ -311,7 +311,7 @@ struct TraceArgs {
     int batch;               // most items a wave claims per fetch
     int coop;                // quad-cooperative walk: 0 never, 1..3 at most lanes/4, /2, /1 items, 4 always
     int group;               // group walk (16 lanes per ray) for launches of at most group x lanes/16 items (0: never)
-    int group_lanes;         // 64: launches of at most group x lanes/64 items walk each ray with a whole wave
+    int group_lanes;         // 64: launches of at most group x lanes/128 items walk each ray with a whole wave
     int steal;               // per-lane walk: idle lanes of a drained wave take pending subtrees of its rays
     int skip_dark;           // MODE_SHADOW: the set-up kernel wrote kVisDark where a light adds nothing to its
                              // surface, visible or not; those rays are not walked
@@ -1137,8 +1137,11 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(XF ? 4 : 5))
     }
     unsigned long long visits = 0, tests = 0;
     const long long lanes = (long long)gridDim.x * WG;
-    // a whole wave per ray for launches of a few thousand rays, else 16 lanes
-    const bool wide = GROUP && a.group_lanes == 64 && use_group(a.group, n, lanes, 64);
+    // a whole wave per ray while that leaves every other wave idle, else 16 lanes
+    // (a wave per ray up to all waves: 256 x 256 frame 291 us, up to half of them
+    // 262, a quarter 266; 5,000 rays queried 120 us by waves, 99 by 16 lanes; 1,000
+    // rays 83 and 88)
+    const bool wide = GROUP && a.group_lanes == 64 && use_group(a.group, 2 * (long long)n, lanes, 64);
     const bool grouped = GROUP && (wide || use_group(a.group, n, lanes, kGroupLanes));
     const bool coop = !grouped && WIDTH == 4 && use_coop(a.coop, n, lanes);
     // Waves beyond what the launch's items can occupy at once leave now: a

@@ -374,7 +374,7 @@ typedef struct eos_launch_config {
     int32_t scatter;          /* launches with at most scatter x lanes items claim them in a scattered
                                  order (item i * p mod n, p prime), so neighbouring rays -- often long
                                  together -- go to different waves; 0: never.  Results do not change */
-    int32_t group_lanes;      /* widest group walk: 64 (launches with at most group x lanes/64 items walk
+    int32_t group_lanes;      /* widest group walk: 64 (launches with at most group x lanes/128 items walk
                                  each ray with a whole wave, 16 nodes per step) or 16 (never wider) */
     int32_t cull;             /* 1: before a single scene's primary rays (4-wide tree) are traced, a tile
                                  test resolves the 8x8-pixel tiles whose rays all miss the root node's child
