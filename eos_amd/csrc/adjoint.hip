@@ -163,9 +163,11 @@ __global__ void k_zero_u64(unsigned long long* p, int n) {
 }
 
 // dst_m[M][7] += value of limbs i < 7M, dst_l[L][6] += the rest (unless the
-// records have to be traced again)
-__global__ void k_accumulate_out(const unsigned long long* g, const int* err, int M, int L, double* dm, double* dlg) {
+// records have to be traced again); the error word to pinned host memory
+__global__ void k_accumulate_out(const unsigned long long* g, const int* err, int32_t* err_out, int M, int L,
+                                 double* dm, double* dlg) {
     const int nacc = 7 * M + 6 * L;
+    if (blockIdx.x == 0 && threadIdx.x == 0) *err_out = *err;
     if (*err & kErrOpen) return;   // replayed again
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < nacc; i += gridDim.x * blockDim.x) {
         const double v = limb_value(g, nacc, i);
@@ -233,16 +235,18 @@ static eos_status adjoint_once(eos_scene* s, const eos_camera* cam, const eos_ad
     EOS_HIP(hipGetLastError());
     EOS_HIP(hipEventRecord(s->ev[1], S));
     int herr = 0;
-    EOS_HIP(hipMemcpyAsync(&herr, err, sizeof herr, hipMemcpyDeviceToHost, S));
+    EOS_TRY(s->ensure_host_small());
     if (o->memory == EOS_MEM_DEVICE) {
         hipLaunchKernelGGL(k_accumulate_out, dim3(std::max(1, std::min(64, (nacc + 255) / 256))), dim3(256), 0, S,
-                           g_dev.as<const unsigned long long>(), err, M, L, gm, gl);
+                           g_dev.as<const unsigned long long>(), err, s->host_small, M, L, gm, gl);
         EOS_HIP(hipStreamSynchronize(S));
+        herr = s->host_small[0];
         open = (herr & kErrOpen) != 0;
     } else {
-        std::vector<unsigned long long> h((size_t)std::max(3 * nacc, 1));
-        EOS_HIP(hipMemcpyAsync(h.data(), g_dev.ptr, 8 * 3 * (size_t)nacc, hipMemcpyDeviceToHost, S));
+        std::vector<unsigned long long> h((size_t)words);
+        EOS_HIP(hipMemcpyAsync(h.data(), g_dev.ptr, 8 * (size_t)words, hipMemcpyDeviceToHost, S));
         EOS_HIP(hipStreamSynchronize(S));
+        herr = (int)(uint32_t)h[3 * (size_t)nacc];
         open = (herr & kErrOpen) != 0;
         if (open) return EOS_OK;
         for (int i = 0; i < 7 * M; ++i) gm[i] += limb_value(h.data(), nacc, i);
@@ -254,13 +258,11 @@ static eos_status adjoint_once(eos_scene* s, const eos_camera* cam, const eos_ad
                                    "(a light on a surface?); the gradients are incomplete");
     float ms = 0.0f;
     EOS_HIP(hipEventElapsedTime(&ms, s->ev[0], s->ev[1]));
-    int hits[EOS_MAX_DEPTH + 1] = {0};
-    EOS_HIP(hipMemcpy(hits, ctr + CTR_HITS, sizeof(int) * (o->depth + 1), hipMemcpyDeviceToHost));
     if (st) {
         st->adjoint_ms = ms;
         st->retrace_ms = retrace_ms;
         st->records = 0;
-        for (int l = 0; l <= o->depth; ++l) st->records += hits[l];
+        for (int l = 0; l <= o->depth; ++l) st->records += fb.rec_hits[l];
     }
     return EOS_OK;
 }

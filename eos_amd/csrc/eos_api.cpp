@@ -97,6 +97,7 @@ static void free_scene(eos_scene* s) {
     for (hipEvent_t e : s->first_ev) (void)hipEventDestroy(e);
     s->first_ev.clear();
     if (s->host_ctr) (void)hipHostFree(s->host_ctr);
+    if (s->host_small) (void)hipHostFree(s->host_small);
     for (hipEvent_t& e : s->ev)
         if (e) (void)hipEventDestroy(e);
     for (hipEvent_t& e : s->sync)
@@ -155,6 +156,11 @@ static void inverse_glm(const float* m, float* out) {
 }
 
 }  // namespace eos
+
+eos_status eos_scene::ensure_host_small() {
+    if (!host_small) EOS_HIP(hipHostMalloc(reinterpret_cast<void**>(&host_small), 4 * kHostSmall, hipHostMallocDefault));
+    return EOS_OK;
+}
 
 using namespace eos;
 

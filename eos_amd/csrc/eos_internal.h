@@ -174,6 +174,7 @@ struct eos_frame_buffers {
     size_t npix = 0, n_ids = 0;
     int depth = -1, n_light = -1;
     int rec_valid = 0;      // records of the last frame kept (adjoint replay)
+    int rec_hits[EOS_MAX_DEPTH + 1] = {};   // hits per level of the last frame
     eos_camera rec_cam{};
 };
 
@@ -220,6 +221,8 @@ struct eos_scene {
     eos::LaunchCfg cfg;
     int num_cu = 256;
     eos_frame_buffers fb;
+    static constexpr int kHostSmall = 64;
+    eos_status ensure_host_small();
     hipEvent_t ev[96] = {};  // frame timing events
     // Further frame slots of eos_render_frames (kFrameSlots frames in flight;
     // slot 0 is fb / stream / stream2 / sync): frame buffers, two streams at
@@ -230,8 +233,11 @@ struct eos_scene {
     hipStream_t xstream[kFrameSlots - 1][2] = {};
     hipEvent_t xsync[kFrameSlots - 1][2] = {};
     hipEvent_t resolved[kFrameSlots] = {}, seq_start = nullptr, seq_ev[kFrameSlots] = {};
+    // pinned host memory that kernels write: the frames' counters (k_resolve), and
+    // small answers (adjoint and build error words, query error flag)
     void* host_ctr = nullptr;
     size_t host_ctr_bytes = 0;
+    int32_t* host_small = nullptr;   // [kHostSmall]
     std::vector<hipEvent_t> first_ev;   // frames in flight: timing events around each frame's primary launch
     // Ray queries (eos_trace_rays): staged rays and outputs for host memory,
     // hit records, fetch cursors and error flag, overflow stacks.

@@ -772,8 +772,10 @@ eos_status build_lbvh(eos_scene* s, int leaf_max, int width, eos_build_stats* st
                            err);
         if (width == 2) EOS_TRY(make_binary_nodes(s));
         EOS_HIP(hipEventRecord(s->ev[1], S));
-        EOS_HIP(hipMemcpyAsync(herr, err, sizeof herr, hipMemcpyDeviceToHost, S));
+        EOS_TRY(s->ensure_host_small());
+        EOS_HIP(hipMemcpyAsync(s->host_small, err, sizeof herr, hipMemcpyDeviceToHost, S));
         EOS_HIP(hipStreamSynchronize(S));
+        std::copy(s->host_small, s->host_small + 4, herr);
         s->n_nodes4 = four ? herr[1] : 0;
     } else {
         EOS_HIP(hipEventRecord(s->ev[1], S));

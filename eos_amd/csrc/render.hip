@@ -365,7 +365,20 @@ struct ResolveArgs {
     float4* acc;              // anti-aliasing: running sum of the pixel's samples
     int aa_mode;              // AA_NONE, AA_FIRST, AA_NEXT, AA_LAST
     float inv_n2;             // (1/n)^2, the final scale (AA_LAST)
+    const int* ctr;           // the frame's counters, complete by now,
+    int* ctr_out;             // and pinned host memory for them (null: not wanted)
 };
+
+// Counters of a frame as the host reads them: int counters, then the 64-bit
+// visit / test statistics (the device layout of the counter block's start).
+constexpr size_t kCounterBytes = 4 * CTR_COUNT + 8 * kStats;
+static_assert(kCounterBytes == 4 * 256, "a word per thread of a resolve workgroup");
+
+// The frame's last launch hands its counters to the host (two copies after it
+// cost a 256 x 256 frame 40 us).
+__device__ __forceinline__ void report(const ResolveArgs& a) {
+    if (blockIdx.x == 0 && a.ctr_out) a.ctr_out[threadIdx.x] = a.ctr[threadIdx.x];
+}
 
 // A pixel's final colour: quantised and written, or, with anti-aliasing
 // (src/RayTracer.cpp:214-242), one sample of n x n added in (q, p) order to a
@@ -396,6 +409,7 @@ __device__ __forceinline__ void pixel_out(const ResolveArgs& a, int p, float c0,
 
 // Chains of reflections: c_l = P_l + r_l * c_{l+1}, innermost first.
 __global__ __launch_bounds__(256) void k_resolve(ResolveArgs a) {
+    report(a);
     for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < a.npix; p += gridDim.x * blockDim.x) {
         const int nl = a.levels[p];
         float c0 = 0.0f, c1 = 0.0f, c2 = 0.0f;
@@ -450,6 +464,7 @@ __global__ __launch_bounds__(256) void k_resolve_tree(const int* count_ptr, floa
 
 // Ray trees: the pixel's colour is its primary hit's resolved colour.
 __global__ __launch_bounds__(256) void k_resolve_pixels(ResolveArgs a, const int32_t* pixhit, const float4* hitcol) {
+    report(a);
     for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < a.npix; p += gridDim.x * blockDim.x) {
         const int j = pixhit[p];
         float c0 = 0.0f, c1 = 0.0f, c2 = 0.0f;
@@ -493,6 +508,7 @@ struct CullArgs {
     int* live_ctr;
     int* culled_ctr;          // rays resolved here (pixels of the frame in resolved tiles)
     int scanned;              // k_cull_compact: block_live holds the scanned offsets (k_cull_scan ran)
+    int* counters;            // the frame's counters, zeroed here: kCounterInts of them
 };
 constexpr int kCullBlock = eos_frame_buffers::kTileBlock;   // tiles per workgroup of the tile test
 static_assert(kCullBlock == 256, "the tile test's kernels are written for four waves per workgroup");
@@ -518,6 +534,7 @@ constexpr int kCullSumBlocks = 4096;   // up to this many workgroups each sums t
 __global__ __launch_bounds__(256) void k_cull_tiles(CullArgs a) {
     using creal = EOS_CULL_REAL;
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    for (int i = t; i < kCounterInts; i += gridDim.x * blockDim.x) a.counters[i] = 0;
     bool traced = true;
     int culled = 0;
     if (t < a.n_tiles) {
@@ -787,6 +804,7 @@ struct Frame {
     uchar4* rgba = nullptr;
     float* rgb = nullptr;
     int32_t* hits = nullptr;
+    void* ctr_out = nullptr;   // pinned host memory for the frame's counters (kCounterBytes)
 };
 
 template <int MODE>
@@ -902,7 +920,6 @@ eos_status enqueue_frame(eos_frame_buffers& fb, const Frame& f, const FrameStrea
         if (E) (void)hipEventRecord(E[ev], st);
         return ev++;
     };
-    hipLaunchKernelGGL(k_zero_i32, dim3(16), dim3(256), 0, S, ctr, kCounterInts);
     // fetch cursors of launch slot k (closest level l: k = l; any hit from level l: k = 16 + l)
     auto cursors = [&](int k) { return ctr + kCursorBase + k * kRanges * kCursorStride; };
     FrameEvents local;
@@ -911,6 +928,8 @@ eos_status enqueue_frame(eos_frame_buffers& fb, const Frame& f, const FrameStrea
     // launches that do not count visits (their counts restate every ray's walk)
     const bool cull = f.cfg.cull != 0 && !f.batch && !f.count && f.width == 4 && !f.cfg.packets &&
                       f.sc.root4 >= 0 && f.sc.root4 != kDone && f.n_ids >= 64;
+    // the tile test zeroes the counters on its way
+    if (!cull) hipLaunchKernelGGL(k_zero_i32, dim3(16), dim3(256), 0, S, ctr, kCounterInts);
     F.start = rec(S);
     // Any-hit trace of levels [l0, l1] in one launch, then Phong of each level.
     auto shadow_and_phong = [&](int l0, int l1, hipStream_t st, size_t gstack_off, int slot) -> eos_status {
@@ -1048,6 +1067,7 @@ eos_status enqueue_frame(eos_frame_buffers& fb, const Frame& f, const FrameStrea
             ca.live_ctr = ctr + CTR_LIVE;
             ca.culled_ctr = ctr + CTR_CULLED;
             ca.scanned = nblocks > kCullSumBlocks;
+            ca.counters = ctr;
             hipLaunchKernelGGL(k_cull_tiles, dim3(nblocks), dim3(kCullBlock), 0, S, ca);
             if (ca.scanned)
                 hipLaunchKernelGGL(k_cull_scan, dim3(1), dim3(1024), 0, S, ca.block_live, nblocks, ca.live_ctr);
@@ -1130,7 +1150,7 @@ eos_status enqueue_frame(eos_frame_buffers& fb, const Frame& f, const FrameStrea
         EOS_HIP(hipStreamWaitEvent(S, fs.sync[1], 0));
     }
     ResolveArgs ra{(int)f.npix, fb.levels.as<uint8_t>(), fb.levcol.as<float4>(), f.rgba, f.rgb,
-                   f.aa.acc, f.aa.mode, f.aa.inv_n2};
+                   f.aa.acc, f.aa.mode, f.aa.inv_n2, ctr, static_cast<int*>(f.ctr_out)};
     if (f.resolve_after) EOS_HIP(hipStreamWaitEvent(S, f.resolve_after, 0));
     F.resolve0 = rec(S);
     if (f.tree) {
@@ -1151,24 +1171,28 @@ eos_status enqueue_frame(eos_frame_buffers& fb, const Frame& f, const FrameStrea
     return EOS_OK;
 }
 
-// Reads the frame's counters (synchronises the stream) into stats.
-// Counters of a frame as the host reads them: int counters, then the 64-bit
-// visit / test statistics (the device layout of the counter block's start).
-constexpr size_t kCounterBytes = 4 * CTR_COUNT + 8 * kStats;
-
 eos_status frame_stats(const Frame& f, const int* hctr, const unsigned long long* hstats, hipEvent_t* E,
                        const FrameEvents* F, eos_render_stats* st);
 
+// Waits for the frame and reads the counters it left in f.ctr_out.
 eos_status finish_frame(eos_frame_buffers& fb, const Frame& f, hipStream_t S, hipEvent_t* E, const FrameEvents* F,
                         eos_render_stats* st) {
-    int hctr[CTR_COUNT];
-    unsigned long long hstats[kStats];
-    int* ctr = fb.counters.as<int>();
-    unsigned long long* stats = reinterpret_cast<unsigned long long*>(fb.counters.as<char>() + 4 * CTR_COUNT);
-    EOS_HIP(hipMemcpyAsync(hctr, ctr, sizeof hctr, hipMemcpyDeviceToHost, S));
-    EOS_HIP(hipMemcpyAsync(hstats, stats, sizeof hstats, hipMemcpyDeviceToHost, S));
     EOS_HIP(hipStreamSynchronize(S));
-    return frame_stats(f, hctr, hstats, E, F, st);
+    const int* hctr = static_cast<const int*>(f.ctr_out);
+    for (int l = 0; l <= f.depth; ++l) fb.rec_hits[l] = hctr[CTR_HITS + l];
+    return frame_stats(f, hctr, reinterpret_cast<const unsigned long long*>(hctr + CTR_COUNT), E, F, st);
+}
+
+// Pinned memory for n frames' counters.
+eos_status ensure_counters(void** ptr, size_t* bytes, int n) {
+    const size_t need = kCounterBytes * (size_t)n;
+    if (*bytes >= need) return EOS_OK;
+    if (*ptr) (void)hipHostFree(*ptr);
+    *ptr = nullptr;
+    *bytes = 0;
+    EOS_HIP(hipHostMalloc(ptr, need, hipHostMallocDefault));
+    *bytes = need;
+    return EOS_OK;
 }
 
 eos_status frame_stats(const Frame& f, const int* hctr, const unsigned long long* hstats, hipEvent_t* E,
@@ -1267,6 +1291,8 @@ eos_status run_frame(eos_scene* s, const eos_camera* camp, int depth, bool count
     Frame f = make_frame(s, camp, depth, count, rgba_dev, rgb_dev, hits_dev, aa, row0, row1);
     f.walk_all = walk_all;
     EOS_TRY(ensure_buffers(s->fb, f, trace_grid_of(f)));
+    EOS_TRY(ensure_counters(&s->host_ctr, &s->host_ctr_bytes, 1));
+    f.ctr_out = s->host_ctr;
     FrameEvents fe;
     FrameStreams fs{s->stream, s->stream2, s->sync};
     if (launch_times) {
@@ -1289,7 +1315,7 @@ eos_status run_frame(eos_scene* s, const eos_camera* camp, int depth, bool count
 // frame i's shadow and reflection launches -- a few rays each, bound by the
 // longest ray's chain of steps -- still run.  Resolves are ordered (frame i's
 // after frame i - 1's), so outputs that alias end with the last frame.
-// Counters are copied per frame to pinned host memory and read after the last
+// Each frame leaves its counters in pinned host memory, read after the last
 // frame.
 namespace {
 // Runs prepared frames kFrameSlots in flight; per-frame stats (render_ms: the
@@ -1313,14 +1339,7 @@ eos_status run_pipelined(eos_scene* s, std::vector<Frame>& frames, eos_render_st
         if (e == hipSuccess) e = hipEventCreate(&s->seq_start);
         if (e != hipSuccess) return fail(EOS_ERR_HIP, std::string("frames in flight: ") + hipGetErrorString(e));
     }
-    const size_t need = kCounterBytes * (size_t)n;
-    if (s->host_ctr_bytes < need) {
-        if (s->host_ctr) (void)hipHostFree(s->host_ctr);
-        s->host_ctr = nullptr;
-        s->host_ctr_bytes = 0;
-        EOS_HIP(hipHostMalloc(&s->host_ctr, need, hipHostMallocDefault));
-        s->host_ctr_bytes = need;
-    }
+    EOS_TRY(ensure_counters(&s->host_ctr, &s->host_ctr_bytes, n));
     eos_frame_buffers* fbs[K];
     FrameStreams fs[K];
     for (int k = 0; k < K; ++k) {
@@ -1358,9 +1377,8 @@ eos_status run_pipelined(eos_scene* s, std::vector<Frame>& frames, eos_render_st
         EOS_TRY(ensure_buffers(*fbs[k], f, trace_grid_of(f)));
         f.resolve_after = i > 0 ? s->resolved[(i - 1) % slots] : nullptr;
         f.resolve_done = s->resolved[k];
+        f.ctr_out = static_cast<char*>(s->host_ctr) + kCounterBytes * (size_t)i;
         EOS_TRY(enqueue_frame(*fbs[k], f, fs[k], nullptr, nullptr));
-        EOS_HIP(hipMemcpyAsync(static_cast<char*>(s->host_ctr) + kCounterBytes * (size_t)i, fbs[k]->counters.ptr,
-                               kCounterBytes, hipMemcpyDeviceToHost, fs[k].S));
     }
     double total = 0.0;
     for (int k = 0; k < slots; ++k) EOS_HIP(hipEventRecord(s->seq_ev[k], fs[k].S));
@@ -1502,6 +1520,8 @@ struct BatchState {
     hipEvent_t ev[2] = {nullptr, nullptr};
     hipEvent_t sync[2] = {};
     Frame frame;
+    void* host_ctr = nullptr;   // pinned, for the process's life (like the graph that writes it)
+    size_t host_ctr_bytes = 0;
 };
 BatchState g_batch;
 
@@ -1538,6 +1558,7 @@ eos_status render_batch(eos_scene* const* scenes, const eos_camera* cams, int n,
         EOS_HIP(hipEventCreate(&b.ev[1]));
         for (hipEvent_t& e : b.sync) EOS_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     }
+    EOS_TRY(ensure_counters(&b.host_ctr, &b.host_ctr_bytes, 1));
     const FrameStreams fs{S, s0->stream2, b.sync};
     const bool same = same_batch(scenes, cams, n, o->depth, cfg);
     if (!same) {
@@ -1589,6 +1610,7 @@ eos_status render_batch(eos_scene* const* scenes, const eos_camera* cams, int n,
         if (f.xf) f.cfg.packets = 0;
         f.num_cu = s0->num_cu;
         f.rgba = b.rgba.as<uchar4>();
+        f.ctr_out = b.host_ctr;
         f.sc = view_of(s0);
         f.cam = b.host_table[0].cam;
         EOS_TRY(ensure_buffers(b.fb, f, trace_grid_of(f)));
