@@ -167,7 +167,7 @@ struct eos_frame_buffers {
     // Ray trees (scenes with transparent materials): level l holds at most
     // tcap[l] rays / hits at offset toff[l] of rayhit (hit index per ray; level
     // 0 per pixel), aux (Fresnel weight, children) and hitcol (colour per hit);
-    // surf / vis / queues then hold one level at a time.
+    // surf / vis then hold two levels, level l in slot l % 2, and the queues one.
     bool tree = false;
     size_t tcap[EOS_MAX_DEPTH + 1] = {}, toff[EOS_MAX_DEPTH + 2] = {};
     eos::DevBuf rayhit, aux, hitcol;
@@ -185,7 +185,7 @@ struct eos_scene {
     // overlapping level l+1's closest-hit trace on `stream`.  Both streams
     // keep the default priority.
     hipStream_t stream2 = nullptr;
-    hipEvent_t sync[2] = {};  // fork to and join from stream2 (no timing)
+    hipEvent_t sync[4] = {};  // fork to and join from stream2, ray trees: level slots shaded (no timing)
     int n_tri = 0, n_mat = 0, n_light = 0;
     // original-order inputs (device)
     eos::DevBuf verts, normals, matidx;
@@ -231,7 +231,7 @@ struct eos_scene {
     static constexpr int kFrameSlots = 2;
     eos_frame_buffers fbx[kFrameSlots - 1];
     hipStream_t xstream[kFrameSlots - 1][2] = {};
-    hipEvent_t xsync[kFrameSlots - 1][2] = {};
+    hipEvent_t xsync[kFrameSlots - 1][4] = {};
     hipEvent_t resolved[kFrameSlots] = {}, seq_start = nullptr, seq_ev[kFrameSlots] = {};
     // pinned host memory that kernels write: the frames' counters (k_resolve), and
     // small answers (adjoint and build error words, query error flag)

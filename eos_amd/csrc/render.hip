@@ -797,6 +797,7 @@ struct Frame {
     hipEvent_t resolve_after = nullptr;   // frames in flight: resolve after this event (the previous frame's)
     hipEvent_t resolve_done = nullptr;    // and record this one after it
     hipEvent_t first_ev[2] = {nullptr, nullptr};   // frames in flight: around the primary-ray launch
+    bool in_flight = false;   // another frame's launches run beside this one's
     bool count = false;
     bool walk_all = false; // every shadow ray is walked (else not those of lights that add nothing)
     LaunchCfg cfg;
@@ -841,12 +842,15 @@ struct FrameEvents {
 // any-hit work) and its Phong run on S2 after a fork event recorded behind
 // level 0's setup, overlapping the reflection levels' closest-hit traces on S;
 // the shadow rays of levels 1..depth follow on S in one launch after the last
-// setup; S joins S2 before the resolve.  The two traversals that can be in
+// setup; S joins S2 before the resolve.  Ray trees shade every level on S2 while S
+// traces the next one (set-up of level l + 2 waits for the shading of level l,
+// whose surfaces it overwrites; a 1365 x 767 glass frame 1036 -> 910 us, a 700 x 400
+// one 771 -> 618).  The two traversals that can be in
 // flight together use disjoint halves of the overflow stack area.
 struct FrameStreams {
     hipStream_t S = nullptr;
     hipStream_t S2 = nullptr;       // null: everything in order on S
-    hipEvent_t* sync = nullptr;     // [2]: fork, join
+    hipEvent_t* sync = nullptr;     // [4]: fork, join; ray trees: level slot 0 / 1 shaded
 };
 
 // Largest queue of a ray tree level (1 << 26 rays, or a frame's pixels if more).
@@ -883,7 +887,7 @@ eos_status ensure_buffers(eos_frame_buffers& fb, const Frame& f, int trace_grid)
         EOS_TRY(fb.aux.ensure(16 * fb.toff[f.depth + 1]));
         EOS_TRY(fb.hitcol.ensure(16 * fb.toff[f.depth + 1]));
     }
-    const int surf_levels = f.tree ? 1 : f.depth + 1;   // trees shade one level at a time
+    const int surf_levels = f.tree ? std::min(2, f.depth + 1) : f.depth + 1;   // trees: a slot per parity
     EOS_TRY(fb.hit0.ensure(16 * f.n_ids));
     EOS_TRY(fb.q[0].ensure(32 * cap));
     EOS_TRY(fb.q[1].ensure(32 * cap));
@@ -913,7 +917,9 @@ eos_status enqueue_frame(eos_frame_buffers& fb, const Frame& f, const FrameStrea
     unsigned long long* stats = reinterpret_cast<unsigned long long*>(fb.counters.as<char>() + 4 * CTR_COUNT);
     const unsigned shade_grid = (unsigned)f.num_cu * 8;
     const hipStream_t S = fs.S;
-    const bool two = fs.S2 != nullptr;
+    // ray trees in flight stay on one stream: the other frame fills the GPU (four
+    // samples of a 1365 x 767 glass frame 2649 us, 2878 on two streams)
+    const bool two = fs.S2 != nullptr && !(f.tree && f.in_flight);
     const hipStream_t S2 = two ? fs.S2 : fs.S;
     int ev = 0;
     auto rec = [&](hipStream_t st) -> int {
@@ -931,6 +937,8 @@ eos_status enqueue_frame(eos_frame_buffers& fb, const Frame& f, const FrameStrea
     // the tile test zeroes the counters on its way
     if (!cull) hipLaunchKernelGGL(k_zero_i32, dim3(16), dim3(256), 0, S, ctr, kCounterInts);
     F.start = rec(S);
+    // where a level's surfaces and visibility lie
+    auto slot_of = [&](int l) { return f.tree ? l & 1 : l; };
     // Any-hit trace of levels [l0, l1] in one launch, then Phong of each level.
     auto shadow_and_phong = [&](int l0, int l1, hipStream_t st, size_t gstack_off, int slot) -> eos_status {
         F.s[2 * slot] = rec(st);
@@ -956,8 +964,8 @@ eos_status enqueue_frame(eos_frame_buffers& fb, const Frame& f, const FrameStrea
             sh.count_ptr = ctr + CTR_HITS + l0;
             sh.count_mul = f.lstride;
             sh.nlev = l1 - l0 + 1;
-            sh.surf = fb.surf_at(f.tree ? 0 : l0);
-            sh.vis_out = fb.vis_at(f.tree ? 0 : l0);
+            sh.surf = fb.surf_at(slot_of(l0));
+            sh.vis_out = fb.vis_at(slot_of(l0));
             sh.surf_stride = (long long)fb.surf_stride();
             sh.vis_stride = (long long)fb.vis_stride();
             // level 0's shadow launch on the second stream shares the CUs with the
@@ -974,8 +982,7 @@ eos_status enqueue_frame(eos_frame_buffers& fb, const Frame& f, const FrameStrea
             // four close 1080p frames 8382 -> 8563)
             const int resident = f.xf || f.big ? kResidentXf : kResident;
             const int sgrid = st != S ? trace_grid_waves(f, std::min(f.cfg.waves_per_cu, 4 * (resident - 1))) : trace_grid;
-            EOS_TRY(launch_trace_any<MODE_SHADOW>(f, sgrid, st, sh,
-                                                  st != S));
+            EOS_TRY(launch_trace_any<MODE_SHADOW>(f, sgrid, st, sh, st != S && l0 == 0));
         }
         F.s[2 * slot + 1] = rec(st);
         // Phong of levels [l0, l1] in one launch (ray trees shade one level at a time)
@@ -988,8 +995,8 @@ eos_status enqueue_frame(eos_frame_buffers& fb, const Frame& f, const FrameStrea
         pa.npix = (int)f.npix;
         pa.lstride = f.lstride;
         pa.count_ptr = ctr + CTR_HITS + l0;
-        pa.surf = fb.surf_at(f.tree ? 0 : l0);
-        pa.vis = fb.vis_at(f.tree ? 0 : l0);
+        pa.surf = fb.surf_at(slot_of(l0));
+        pa.vis = fb.vis_at(slot_of(l0));
         pa.surf_stride = (long long)fb.surf_stride();
         pa.vis_stride = (long long)fb.vis_stride();
         pa.levcol = fb.levcol.as<float4>();
@@ -1096,7 +1103,7 @@ eos_status enqueue_frame(eos_frame_buffers& fb, const Frame& f, const FrameStrea
         sa.count_ptr = ctr + CTR_Q + l;
         sa.q_in = qin;
         sa.hit_in = l == 0 ? fb.hit0.as<float4>() : fb.hitq.as<float4>();
-        sa.surf_out = fb.surf_at(f.tree ? 0 : l);
+        sa.surf_out = fb.surf_at(slot_of(l));
         sa.hits_ctr = ctr + CTR_HITS + l;
         sa.q_out = qout;
         sa.q_out_ctr = ctr + CTR_Q + l + 1;
@@ -1106,11 +1113,12 @@ eos_status enqueue_frame(eos_frame_buffers& fb, const Frame& f, const FrameStrea
             sa.aux = fb.aux.as<float4>() + fb.toff[l];
         }
         sa.shadow_ctr = ctr + CTR_SHADOW + l;
-        sa.vis_out = f.count || f.walk_all ? nullptr : fb.vis_at(f.tree ? 0 : l);
+        sa.vis_out = f.count || f.walk_all ? nullptr : fb.vis_at(slot_of(l));
         sa.lstride = f.lstride;
         sa.levels = fb.levels.as<uint8_t>();
         sa.hit_ids = l == 0 ? f.hits : nullptr;
         sa.tile_live = l == 0 && cull ? fb.tile_flags(f.n_ids) : nullptr;
+        if (f.tree && two && l >= 2) EOS_HIP(hipStreamWaitEvent(S, fs.sync[2 + (l & 1)], 0));   // level l - 2 is shaded
         F.u[2 * l] = rec(S);
         if (l == 0) {
             if (f.batch)
@@ -1123,11 +1131,16 @@ eos_status enqueue_frame(eos_frame_buffers& fb, const Frame& f, const FrameStrea
         }
         F.u[2 * l + 1] = rec(S);
         if (f.tree) {
-            // ray trees: one level's surfaces at a time, shaded before the next level is set up
             if (l < f.depth)
                 hipLaunchKernelGGL(k_clamp_count, dim3(1), dim3(64), 0, S, ctr + CTR_Q + l + 1, (int)fb.tcap[l + 1],
                                    ctr + CTR_ERR);
-            EOS_TRY(shadow_and_phong(l, l, S, 0, l));
+            // shaded on S2 while the next level is traced
+            if (two) {
+                EOS_HIP(hipEventRecord(fs.sync[0], S));
+                EOS_HIP(hipStreamWaitEvent(S2, fs.sync[0], 0));
+            }
+            EOS_TRY(shadow_and_phong(l, l, S2, two ? gstack_ints(f, trace_grid) : 0, l));
+            if (two && l + 2 <= f.depth) EOS_HIP(hipEventRecord(fs.sync[2 + (l & 1)], S2));
         } else if (l == 0) {
             // level 0's shadow rays and shading overlap the reflection chain
             if (two) {
@@ -1145,7 +1158,7 @@ eos_status enqueue_frame(eos_frame_buffers& fb, const Frame& f, const FrameStrea
         for (int l0 = 1; l0 <= f.depth; l0 += span)
             EOS_TRY(shadow_and_phong(l0, std::min(f.depth, l0 + span - 1), S, 0, l0));
     }
-    if (two && !f.tree) {
+    if (two) {
         EOS_HIP(hipEventRecord(fs.sync[1], S2));
         EOS_HIP(hipStreamWaitEvent(S, fs.sync[1], 0));
     }
@@ -1347,12 +1360,13 @@ eos_status run_pipelined(eos_scene* s, std::vector<Frame>& frames, eos_render_st
         fs[k] = k == 0 ? FrameStreams{s->stream, s->stream2, s->sync}
                        : FrameStreams{s->xstream[k - 1][0], s->xstream[k - 1][1], s->xsync[k - 1]};
     }
+    const int slots = std::min(K, std::max(n, 1));
     for (Frame& f : frames) {
         f.cfg.waves_per_cu = f.cfg.frames_waves_per_cu;
         f.cfg.refill = f.cfg.frames_refill;
         f.cfg.batch = f.cfg.frames_batch;
+        f.in_flight = slots > 1;
     }
-    const int slots = std::min(K, std::max(n, 1));
     // launch_times: a pair of timing events per frame around its primary-ray
     // launch (the dispatch duration of that launch while frames overlap)
     while (launch_times && s->first_ev.size() < 2 * (size_t)n) {
@@ -1518,7 +1532,7 @@ struct BatchState {
     LaunchCfg cfg;
     hipGraphExec_t exec = nullptr;
     hipEvent_t ev[2] = {nullptr, nullptr};
-    hipEvent_t sync[2] = {};
+    hipEvent_t sync[4] = {};
     Frame frame;
     void* host_ctr = nullptr;   // pinned, for the process's life (like the graph that writes it)
     size_t host_ctr_bytes = 0;
