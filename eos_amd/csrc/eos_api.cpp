@@ -1,4 +1,5 @@
 // eos_api.cpp -- C ABI entry points: scene lifetime, parameters, diagnostics.
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <string>
@@ -122,6 +123,22 @@ static eos_status check_lights(const eos_light* l, int n) {
     return EOS_OK;
 }
 
+// The first index outside [lo, hi], or -1.  Blocks are tested without an early
+// exit, which the compiler vectorises (one branch per index took 0.3 ms of a
+// rebuild of 1M triangles).
+static int first_outside(const int32_t* index, int n, int32_t lo, int32_t hi) {
+    constexpr int kBlock = 4096;
+    for (int b = 0; b < n; b += kBlock) {
+        const int e = std::min(n, b + kBlock);
+        int bad = 0;
+        for (int i = b; i < e; ++i) bad |= (index[i] < lo) | (index[i] > hi);
+        if (bad)
+            for (int i = b; i < e; ++i)
+                if (index[i] < lo || index[i] > hi) return i;
+    }
+    return -1;
+}
+
 // glm 0.9.6 compute_inverse for a column-major 4x4 (glm/detail/type_mat4x4.inl:
 // 37-96): the 2x2 cofactors of the lower rows, combined per column as
 // (a - b) + c with alternating signs, the determinant from the first row and
@@ -198,11 +215,11 @@ eos_status eos_create_scene(const eos_scene_desc* d, eos_scene** out) {
     if (hipGetDeviceCount(&count) != hipSuccess || count == 0)
         return fail(EOS_ERR_NODEVICE, "eos_create_scene: no HIP device");
     // Material indices are validated on the host when they are host memory.
-    if (d->triangle_memory == EOS_MEM_HOST)
-        for (int i = 0; i < d->num_triangles; ++i)
-            if (d->material_index[i] < 0 || d->material_index[i] >= d->num_materials)
-                return fail(EOS_ERR_INVALID, "eos_create_scene: material index out of range at triangle " +
-                                                 std::to_string(i));
+    if (d->triangle_memory == EOS_MEM_HOST) {
+        const int bad = first_outside(d->material_index, d->num_triangles, 0, d->num_materials - 1);
+        if (bad >= 0)
+            return fail(EOS_ERR_INVALID, "eos_create_scene: material index out of range at triangle " + std::to_string(bad));
+    }
     int device = 0;
     EOS_HIP(hipGetDevice(&device));
     hipDeviceProp_t p;
@@ -294,11 +311,12 @@ eos_status eos_set_transforms(eos_scene* s, int32_t nt, const float* mats, const
                 r[4 * (kXfInvT + k) + c] = inv[4 * k + c];  // transpose(inverse)[c][k] = inverse[k][c]
             }
     }
-    if (memory == EOS_MEM_HOST)
-        for (int i = 0; i < s->n_tri; ++i)
-            if (index[i] < -1 || index[i] >= nt)
-                return fail(EOS_ERR_INVALID, "eos_set_transforms: transformation index out of range at triangle " +
-                                                 std::to_string(i));
+    if (memory == EOS_MEM_HOST) {
+        const int bad = first_outside(index, s->n_tri, -1, nt - 1);
+        if (bad >= 0)
+            return fail(EOS_ERR_INVALID, "eos_set_transforms: transformation index out of range at triangle " +
+                                             std::to_string(bad));
+    }
     s->n_xf = 0;
     EOS_TRY(copy_in(s->xf, rows.data(), rows.size() * sizeof(float), EOS_MEM_HOST, s->stream));
     EOS_TRY(copy_in(s->xf_index, index, (size_t)s->n_tri * sizeof(int32_t), memory, s->stream));
