@@ -193,7 +193,7 @@ struct eos_scene {
     // LBVH and sorted layouts
     // tree: the triangle geometry records, then the 4-wide nodes, in one allocation:
     // the traversal addresses both from one base with 32-bit byte offsets (a tree
-    // past 4 GiB, about 45 million triangles, takes kernels with 64-bit addresses)
+    // past 4 GiB, about 60 million triangles in leaves of four, takes kernels with 64-bit addresses)
     eos::DevBuf nodes, tree, shade;
     size_t nodes4_offset() const { return (48 * (size_t)n_tri + 127) & ~(size_t)127; }
     size_t tree_bytes(size_t nodes) const { return nodes4_offset() + 128 * nodes; }
