@@ -1110,6 +1110,15 @@ struct LaneStack {
 // triangle's local space.  LEAN: no group walk, and so no LDS for its stacks
 // (24 instead of 32 KiB per 256-thread workgroup), for a launch that runs
 // beside another stream's launches.
+// What bounds it: close-up frames VALU issue under divergence (42% of the lanes
+// active), incoherent rays the L1's one lane request per cycle and CU, short
+// launches their longest ray's chain of steps.  So a step waits for memory once
+// (nodes and triangles share their loads), pops without a fetch what the nearest
+// hit has overtaken, and spends few instructions on addresses and selects.
+// Measured against separate fetches, 64-bit addresses and entries without
+// distances: 4K frame of 4.2M triangles 2381 -> 2040 us, four close 1080p frames
+// 11939 -> 9940, 16-scene batch 5591 -> 5098, 1M random rays 629 -> 614.
+// At least 5 waves per SIMD (4 with transformations, whose walk needs more registers).
 template <int MODE, int WG, int STACK_LDS, bool COUNT, bool BATCH, int WIDTH, bool XF, bool LEAN = false,
           bool A64 = BATCH>
 __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(XF ? 4 : 5))) void k_trace(TraceArgs a) {
