@@ -1017,7 +1017,10 @@ __device__ __forceinline__ void trace_group(const TraceArgs& a, int n, int32_t* 
 // count visits keep the sorted order.
 // Idle lanes a wave needs before its walking lanes lend subtrees (measured,
 // frames identical: at 1, 16, 32, 48 idle lanes config C's single frame took
-// 2.21, 2.11, 2.11, 2.28 ms and config D's 64 sequential frames 102, 93, 84, 87 ms).
+// 2.21, 2.11, 2.11, 2.28 ms and config D's 64 sequential frames 102, 93, 84, 87 ms;
+// with the walk as it is now, at 8, 16, 24, 32, 40: 4K frame of 4.2M triangles 1808,
+// 1750, 1740, 1780, 1876 us, 16-scene batch 4416, 4286, 4201, 4139, 4161, 64 moving
+// instances 1946, 1896, 1838, 1807, 1838).
 #ifndef EOS_STEAL_IDLE
 #define EOS_STEAL_IDLE 32
 #endif
