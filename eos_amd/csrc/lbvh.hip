@@ -342,8 +342,11 @@ __global__ __launch_bounds__(256) void k_karras(const uint32_t* __restrict__ k, 
 // top - (top >> (k - 1)) on, top = the leaf count rounded up to a power of two;
 // level 0 is lbox.  (Boxing the tree level by level, each pass over every node
 // still open, took 64 launches, 0.74 ms of a 1.4 ms build of 1M triangles.)
+// An empty box is not a number, which fminf and fmaxf pass over: the union of
+// boxes that hold no number at all (triangles of NaN corners) stays so, as it
+// does where two children's boxes are joined.
 struct Box6 {
-    float v[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
+    float v[6] = {NAN, NAN, NAN, NAN, NAN, NAN};
     __device__ __forceinline__ void add(const Box6& o) {
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
