@@ -1,0 +1,56 @@
+// launch_plan.h -- how host code shapes launches and their scratch from sizes
+// alone.  Plain C++ (no HIP), so that the shapes are checked without a GPU at sizes
+// that no test renders.
+#pragma once
+#include <algorithm>
+#include <cstddef>
+
+#include "eos_c.h"
+
+namespace eos {
+
+// HIP refuses a launch dimension of 2^32 work items or more.
+constexpr size_t kMaxLaunchItems = (size_t)1 << 32;
+
+// ---- linear ray queries (every ray against every triangle) ---------------------
+constexpr int kLinTile = 256;           // triangles staged at a time, and threads of the scanning kernels
+constexpr int kLinMergeThreads = 256;   // four rays, a wave each
+constexpr size_t kLinBlocks = 2048;     // scanning workgroups wanted
+constexpr size_t kLinRunBytes = 16;     // one ray's run over one chunk of triangles
+constexpr size_t kLinRuns = (size_t)EOS_STATIC_MAX_RAYS;   // at most
+constexpr int kLinFewRays = 128;        // up to here a ray's triangles are shared out over lanes as well
+
+struct LinSplit {
+    int lanes_per_ray = 1;      // a power of two up to 64
+    int chunk = 0;              // triangles per chunk, a multiple of kLinTile
+    int n_chunks = 1;
+    size_t runs = 0;            // runs kept for the merge; 0: the scanning kernel writes the answers
+    unsigned scan_blocks = 0;   // times n_chunks
+    unsigned merge_blocks = 0;
+};
+
+// n rays (n >= 1) against n_tri triangles: as many chunks as give kLinBlocks
+// workgroups, at most one per kLinTile triangles, and runs within kLinRuns.  One
+// chunk needs no merge unless lanes share its rays: a merge there is a wave per
+// ray for a single run, 64 n work items, which passes the launch limit from 2^26
+// rays on.
+inline LinSplit linear_split(int n, int n_tri) {
+    LinSplit r;
+    if (n <= kLinFewRays)
+        while (r.lanes_per_ray < 64 && 2 * r.lanes_per_ray * n <= kLinTile) r.lanes_per_ray *= 2;
+    const size_t blocks = ((size_t)n * r.lanes_per_ray + kLinTile - 1) / kLinTile;
+    const size_t tiles = std::max<size_t>(1, ((size_t)n_tri + kLinTile - 1) / kLinTile);
+    size_t c = std::min(tiles, (kLinBlocks + blocks - 1) / blocks);
+    c = std::max<size_t>(1, std::min({c, kLinRuns / (size_t)n, (size_t)65535}));
+    const size_t per = (tiles + c - 1) / c;
+    r.chunk = (int)(per * kLinTile);
+    r.n_chunks = (int)((tiles + per - 1) / per);
+    r.scan_blocks = (unsigned)blocks;
+    if (r.n_chunks > 1 || r.lanes_per_ray > 1) {
+        r.runs = (size_t)n * (size_t)r.n_chunks;
+        r.merge_blocks = (unsigned)(((size_t)n + kLinMergeThreads / 64 - 1) / (kLinMergeThreads / 64));
+    }
+    return r;
+}
+
+}  // namespace eos

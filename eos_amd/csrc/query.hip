@@ -18,6 +18,7 @@
 #include <string>
 
 #include "eos_internal.h"
+#include "launch_plan.h"
 #include "trace.h"
 
 namespace eos {
@@ -56,8 +57,6 @@ __global__ __launch_bounds__(256) void k_query_hits(int n, const float* ro, cons
     write_hit(out, (size_t)i, true, P, N, __float_as_int(s0.w), h.x, h.z, h.w,
               __float_as_int(geo[3 * (size_t)slot + 2].y));
 }
-
-constexpr int kLinTile = 256;
 
 // src/Scene.cpp:159-201 in parallel.  The reference walks the triangles in index
 // order with two running bounds: Triangle::hit's `distance` (minTemp: a hit
@@ -145,6 +144,7 @@ struct LinRay {
 
 struct LinArgs {
     int n, n_tri, chunk, n_chunks;   // triangles per chunk, a multiple of kLinTile
+    bool finish;                     // one chunk: the scanning kernel writes the answers
     const float *ro, *rd;
     const float *verts, *normals;    // the scene's triangles in their original order
     const int32_t *matidx, *xfi;
@@ -153,95 +153,10 @@ struct LinArgs {
     float4* out;
 };
 
-// One run per ray and chunk of triangles, a workgroup per 256 rays and chunk:
-// every lane tests every triangle of the chunk, staged in LDS as (v1, e1, e2,
-// transformation) and read as broadcasts.  Bound by the tests' arithmetic (about
-// 60 instructions each), so what counts is that every CU has rays: the
-// triangles are split until the launch has kLinBlocks workgroups.
-__global__ __launch_bounds__(kLinTile) void k_query_linear(LinArgs a) {
-    __shared__ float4 tri[3 * kLinTile];
-    const int i = blockIdx.x * kLinTile + (int)threadIdx.x;
-    const bool act = i < a.n;
-    LinRay ray;
-    if (act) ray.load(a.ro, a.rd, (size_t)i);
-    LinRun run;
-    const int c0 = (int)blockIdx.y * a.chunk, c1 = min(a.n_tri, c0 + a.chunk);
-    for (int base = c0; base < c1; base += kLinTile) {
-        __syncthreads();
-        const int k = base + (int)threadIdx.x;
-        if (k < c1) {
-            const float* w = a.verts + 9 * (size_t)k;
-            const F3 v1 = f3(w[0], w[1], w[2]);
-            const F3 e1 = sub(f3(w[3], w[4], w[5]), v1), e2 = sub(f3(w[6], w[7], w[8]), v1);
-            tri[3 * threadIdx.x] = make_float4(v1.x, v1.y, v1.z, e1.x);
-            tri[3 * threadIdx.x + 1] = make_float4(e1.y, e1.z, e2.x, e2.y);
-            tri[3 * threadIdx.x + 2] = make_float4(e2.z, __int_as_float(a.xfi ? a.xfi[k] : -1), 0.0f, 0.0f);
-        }
-        __syncthreads();
-        if (!act) continue;
-        const int cnt = min(kLinTile, c1 - base);
-        for (int j = 0; j < cnt; ++j) {
-            const float4 p = tri[3 * j], q = tri[3 * j + 1], r = tri[3 * j + 2];
-            float t, u, v;
-            if (ray.test(a.xf, __float_as_int(r.y), f3(p.x, p.y, p.z), f3(p.w, q.x, q.y), f3(q.z, q.w, r.x), t, u, v))
-                run.hit(t, u, v, base + j);
-        }
-    }
-    if (act) a.part[(size_t)blockIdx.y * a.n + i] = run.pack();
-}
-
-// The same with few rays: P lanes (a power of two) share a ray, each a slice of
-// consecutive triangles of the chunk, and combine their runs in order.
-__global__ __launch_bounds__(kLinTile) void k_query_linear_few(LinArgs a, int P) {
-    const int lane_p = (int)threadIdx.x & (P - 1);
-    const int i = (int)(blockIdx.x * (kLinTile / P)) + (int)threadIdx.x / P;
-    const bool act = i < a.n;
-    const int c0 = (int)blockIdx.y * a.chunk, c1 = min(a.n_tri, c0 + a.chunk);
-    const int len = a.chunk / P;
-    LinRun run;
-    if (act) {
-        LinRay ray;
-        ray.load(a.ro, a.rd, (size_t)i);
-        const int k1 = min(c1, c0 + (lane_p + 1) * len);
-        for (int k = c0 + lane_p * len; k < k1; ++k) {
-            const float* w = a.verts + 9 * (size_t)k;
-            const F3 v1 = f3(w[0], w[1], w[2]);
-            const F3 e1 = sub(f3(w[3], w[4], w[5]), v1), e2 = sub(f3(w[6], w[7], w[8]), v1);
-            float t, u, v;
-            if (ray.test(a.xf, a.xfi ? a.xfi[k] : -1, v1, e1, e2, t, u, v)) run.hit(t, u, v, k);
-        }
-    }
-    float4 mine = run.pack();
-    for (int off = 1; off < P; off <<= 1) {
-        const float4 o = make_float4(__shfl_down(mine.x, off), __shfl_down(mine.y, off), __shfl_down(mine.z, off),
-                                     __shfl_down(mine.w, off));
-        run.then(LinRun::unpack(o));   // right for the lanes the next steps read
-        mine = run.pack();
-    }
-    if (act && lane_p == 0) a.part[(size_t)blockIdx.y * a.n + i] = mine;
-}
-
-// A wave per ray: the chunks' runs combined in order (each lane a stretch of
-// chunks, then the lanes), then the answer.  The kept hit's point goes through M
-// and its normal through transpose(inverse) without a second normalisation.
-__global__ __launch_bounds__(256) void k_linear_merge(LinArgs a) {
-    const int i = blockIdx.x * 4 + (int)(threadIdx.x >> 6);
-    if (i >= a.n) return;
-    const int lane = __lane_id();
-    const int per = (a.n_chunks + 63) / 64;
-    const int b1 = min(a.n_chunks, (lane + 1) * per);
-    LinRun run;
-    for (int b = lane * per; b < b1; ++b) run.then(LinRun::unpack(a.part[(size_t)b * a.n + i]));
-    float4 mine = run.pack();
-    for (int off = 1; off < 64; off <<= 1) {
-        const float4 o = make_float4(__shfl_down(mine.x, off), __shfl_down(mine.y, off), __shfl_down(mine.z, off),
-                                     __shfl_down(mine.w, off));
-        run.then(LinRun::unpack(o));
-        mine = run.pack();
-    }
-    if (lane != 0) return;
-    LinRay ray;
-    ray.load(a.ro, a.rd, (size_t)i);
+// A ray's answer from the run over all its triangles.  The kept hit's point goes
+// through M and its normal through transpose(inverse) without a second
+// normalisation.
+__device__ __forceinline__ void linear_answer(const LinArgs& a, int i, LinRay& ray, LinRun run) {
     if (run.nan) {
         // in index order, with both of the reference's bounds
         float min_temp = INFINITY;
@@ -277,45 +192,128 @@ __global__ __launch_bounds__(256) void k_linear_merge(LinArgs a) {
     write_hit(a.out, (size_t)i, run.found, P, N, a.matidx[run.best], run.t, run.u, run.v, run.best);
 }
 
-// How a linear query is split: workgroups wanted, the most runs kept (16 bytes
-// each), and the most rays whose triangles are shared out over lanes as well.
-constexpr size_t kLinBlocks = 2048;
-constexpr size_t kLinParts = (size_t)EOS_STATIC_MAX_RAYS;
-constexpr int kLinFewRays = 128;
+// One run per ray and chunk of triangles, a workgroup per 256 rays and chunk:
+// every lane tests every triangle of the chunk, staged in LDS as (v1, e1, e2,
+// transformation) and read as broadcasts.  Bound by the tests' arithmetic (about
+// 60 instructions each), so what counts is that every CU has rays: the
+// triangles are split until the launch has kLinBlocks workgroups.  Where one chunk
+// holds them all the answer is written here.
+__global__ __launch_bounds__(kLinTile) void k_query_linear(LinArgs a) {
+    __shared__ float4 tri[3 * kLinTile];
+    const int i = blockIdx.x * kLinTile + (int)threadIdx.x;
+    const bool act = i < a.n;
+    LinRay ray;
+    if (act) ray.load(a.ro, a.rd, (size_t)i);
+    LinRun run;
+    const int c0 = (int)blockIdx.y * a.chunk, c1 = min(a.n_tri, c0 + a.chunk);
+    for (int base = c0; base < c1; base += kLinTile) {
+        __syncthreads();
+        const int k = base + (int)threadIdx.x;
+        if (k < c1) {
+            const float* w = a.verts + 9 * (size_t)k;
+            const F3 v1 = f3(w[0], w[1], w[2]);
+            const F3 e1 = sub(f3(w[3], w[4], w[5]), v1), e2 = sub(f3(w[6], w[7], w[8]), v1);
+            tri[3 * threadIdx.x] = make_float4(v1.x, v1.y, v1.z, e1.x);
+            tri[3 * threadIdx.x + 1] = make_float4(e1.y, e1.z, e2.x, e2.y);
+            tri[3 * threadIdx.x + 2] = make_float4(e2.z, __int_as_float(a.xfi ? a.xfi[k] : -1), 0.0f, 0.0f);
+        }
+        __syncthreads();
+        if (!act) continue;
+        const int cnt = min(kLinTile, c1 - base);
+        for (int j = 0; j < cnt; ++j) {
+            const float4 p = tri[3 * j], q = tri[3 * j + 1], r = tri[3 * j + 2];
+            float t, u, v;
+            if (ray.test(a.xf, __float_as_int(r.y), f3(p.x, p.y, p.z), f3(p.w, q.x, q.y), f3(q.z, q.w, r.x), t, u, v))
+                run.hit(t, u, v, base + j);
+        }
+    }
+    if (!act) return;
+    if (a.finish) linear_answer(a, i, ray, run);
+    else a.part[(size_t)blockIdx.y * a.n + i] = run.pack();
+}
 
-// Chunks of triangles per ray, for n rays (n >= 1): as many as give kLinBlocks
-// workgroups, at most one per kLinTile triangles, and runs within kLinParts (one
-// chunk always).
-LinArgs linear_split(const eos_scene* s, int n, int& lanes_per_ray) {
+// The same with few rays: P lanes (a power of two) share a ray, each a slice of
+// consecutive triangles of the chunk, and combine their runs in order.
+__global__ __launch_bounds__(kLinTile) void k_query_linear_few(LinArgs a, int P) {
+    const int lane_p = (int)threadIdx.x & (P - 1);
+    const int i = (int)(blockIdx.x * (kLinTile / P)) + (int)threadIdx.x / P;
+    const bool act = i < a.n;
+    const int c0 = (int)blockIdx.y * a.chunk, c1 = min(a.n_tri, c0 + a.chunk);
+    const int len = a.chunk / P;
+    LinRun run;
+    if (act) {
+        LinRay ray;
+        ray.load(a.ro, a.rd, (size_t)i);
+        const int k1 = min(c1, c0 + (lane_p + 1) * len);
+        for (int k = c0 + lane_p * len; k < k1; ++k) {
+            const float* w = a.verts + 9 * (size_t)k;
+            const F3 v1 = f3(w[0], w[1], w[2]);
+            const F3 e1 = sub(f3(w[3], w[4], w[5]), v1), e2 = sub(f3(w[6], w[7], w[8]), v1);
+            float t, u, v;
+            if (ray.test(a.xf, a.xfi ? a.xfi[k] : -1, v1, e1, e2, t, u, v)) run.hit(t, u, v, k);
+        }
+    }
+    float4 mine = run.pack();
+    for (int off = 1; off < P; off <<= 1) {
+        const float4 o = make_float4(__shfl_down(mine.x, off), __shfl_down(mine.y, off), __shfl_down(mine.z, off),
+                                     __shfl_down(mine.w, off));
+        run.then(LinRun::unpack(o));   // right for the lanes the next steps read
+        mine = run.pack();
+    }
+    if (act && lane_p == 0) a.part[(size_t)blockIdx.y * a.n + i] = mine;
+}
+
+// A wave per ray of a query of several chunks: its runs combined in order (each
+// lane a stretch of chunks, then the lanes), then the answer.
+__global__ __launch_bounds__(kLinMergeThreads) void k_linear_merge(LinArgs a) {
+    const int i = blockIdx.x * (kLinMergeThreads / 64) + (int)(threadIdx.x >> 6);
+    if (i >= a.n) return;
+    const int lane = __lane_id();
+    const int per = (a.n_chunks + 63) / 64;
+    const int b1 = min(a.n_chunks, (lane + 1) * per);
+    LinRun run;
+    for (int b = lane * per; b < b1; ++b) run.then(LinRun::unpack(a.part[(size_t)b * a.n + i]));
+    float4 mine = run.pack();
+    for (int off = 1; off < 64; off <<= 1) {
+        const float4 o = make_float4(__shfl_down(mine.x, off), __shfl_down(mine.y, off), __shfl_down(mine.z, off),
+                                     __shfl_down(mine.w, off));
+        run.then(LinRun::unpack(o));
+        mine = run.pack();
+    }
+    if (lane != 0) return;
+    LinRay ray;
+    ray.load(a.ro, a.rd, (size_t)i);
+    linear_answer(a, i, ray, run);
+}
+
+// A linear query of n rays (n >= 1); part: room for the split's runs.
+LinArgs linear_args(const eos_scene* s, int n, const LinSplit& sp, const float* ro, const float* rd, float4* part,
+                    float4* out) {
     LinArgs a{};
     a.n = n;
     a.n_tri = s->n_tri;
-    int P = 1;
-    if (n <= kLinFewRays)
-        while (P < 64 && 2 * P * n <= kLinTile) P *= 2;
-    lanes_per_ray = P;
-    const size_t ray_blocks = ((size_t)n * P + kLinTile - 1) / kLinTile;
-    const size_t tiles = std::max<size_t>(1, ((size_t)s->n_tri + kLinTile - 1) / kLinTile);
-    size_t c = std::min(tiles, (kLinBlocks + ray_blocks - 1) / ray_blocks);
-    c = std::max<size_t>(1, std::min({c, kLinParts / (size_t)n, (size_t)65535}));
-    const size_t per = (tiles + c - 1) / c;
-    a.chunk = (int)(per * kLinTile);
-    a.n_chunks = (int)((tiles + per - 1) / per);
+    a.chunk = sp.chunk;
+    a.n_chunks = sp.n_chunks;
+    a.finish = sp.runs == 0;
     a.verts = s->verts.as<const float>();
     a.normals = s->normals.as<const float>();
     a.matidx = s->matidx.as<const int32_t>();
     a.xfi = s->n_xf > 0 ? s->xf_index.as<const int32_t>() : nullptr;
     a.xf = s->n_xf > 0 ? s->xf.as<const float4>() : nullptr;
+    a.ro = ro;
+    a.rd = rd;
+    a.part = part;
+    a.out = out;
     return a;
 }
 
-void launch_linear(const LinArgs& a, int P, hipStream_t S) {
-    const unsigned gx = (unsigned)(((size_t)a.n * P + kLinTile - 1) / kLinTile);
-    if (P > 1)
-        hipLaunchKernelGGL(k_query_linear_few, dim3(gx, (unsigned)a.n_chunks), dim3(kLinTile), 0, S, a, P);
+void launch_linear(const LinArgs& a, const LinSplit& sp, hipStream_t S) {
+    const dim3 grid(sp.scan_blocks, (unsigned)sp.n_chunks);
+    if (sp.lanes_per_ray > 1)
+        hipLaunchKernelGGL(k_query_linear_few, grid, dim3(kLinTile), 0, S, a, sp.lanes_per_ray);
     else
-        hipLaunchKernelGGL(k_query_linear, dim3(gx, (unsigned)a.n_chunks), dim3(kLinTile), 0, S, a);
-    hipLaunchKernelGGL(k_linear_merge, dim3((unsigned)(((size_t)a.n + 3) / 4)), dim3(256), 0, S, a);
+        hipLaunchKernelGGL(k_query_linear, grid, dim3(kLinTile), 0, S, a);
+    if (sp.runs > 0) hipLaunchKernelGGL(k_linear_merge, dim3(sp.merge_blocks), dim3(kLinMergeThreads), 0, S, a);
 }
 
 // The BVH traversal for caller-given rays: the default launch shape (256
@@ -343,11 +341,12 @@ __global__ void k_zero_i32_query(int* p, int n) {
 // ---- the allocation-free variant (eos_trace_rays_static) --------------------
 // Its scratch is this fixed array (one copy per GPU, held until the process
 // ends): the fetch cursors and the error flag in the first kStaticHeader bytes,
-// then the nearest-hit records (16 bytes per ray).  Host code reaches it only
+// then the nearest-hit records (16 bytes per ray) or a linear search's runs.  Host code reaches it only
 // through the address hipGetSymbolAddress gives on each device.
 constexpr size_t kStaticHeader = 4096;
 static_assert(4 * (size_t)kQueryCtrInts <= kStaticHeader, "cursors and flag fit the header");
 constexpr size_t kStaticBytes = kStaticHeader + 16 * (size_t)EOS_STATIC_MAX_RAYS;
+static_assert(kLinRunBytes * kLinRuns <= kStaticBytes - kStaticHeader, "a linear query's runs fit the records");
 __device__ __align__(256) unsigned char scratch[kStaticBytes];
 
 constexpr int kMaxDevices = 64;
@@ -379,13 +378,8 @@ eos_status trace_rays_static(eos_scene* s, int n, const float* o, const float* d
     float4* out = reinterpret_cast<float4*>(hits);
     const unsigned blocks = (unsigned)(((size_t)n + 255) / 256);
     if (opts->mode == EOS_QUERY_NEAREST_LINEAR) {
-        int P = 1;
-        LinArgs la = linear_split(s, n, P);
-        la.ro = o;
-        la.rd = d;
-        la.part = rec;
-        la.out = out;
-        launch_linear(la, P, S);
+        const LinSplit sp = linear_split(n, s->n_tri);
+        launch_linear(linear_args(s, n, sp, o, d, rec, out), sp, S);
         EOS_HIP(hipGetLastError());
         EOS_HIP(hipStreamSynchronize(S));
         return EOS_OK;
@@ -469,14 +463,9 @@ eos_status trace_rays(eos_scene* s, int n, const float* o, const float* d, const
     const unsigned blocks = (unsigned)((nn + 255) / 256);
     int err = 0;
     if (mode == EOS_QUERY_NEAREST_LINEAR) {
-        int P = 1;
-        LinArgs la = linear_split(s, n, P);
-        EOS_TRY(s->q_rec.ensure(16 * nn * (size_t)la.n_chunks));
-        la.ro = ro;
-        la.rd = rd;
-        la.part = s->q_rec.as<float4>();
-        la.out = out;
-        launch_linear(la, P, S);
+        const LinSplit sp = linear_split(n, s->n_tri);
+        EOS_TRY(s->q_rec.ensure(kLinRunBytes * sp.runs));
+        launch_linear(linear_args(s, n, sp, ro, rd, s->q_rec.as<float4>(), out), sp, S);
         EOS_HIP(hipGetLastError());
     } else {
         const LaunchCfg& cfg = s->cfg;

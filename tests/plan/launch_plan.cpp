@@ -1,0 +1,21 @@
+// The launch shapes of eos_amd/csrc/launch_plan.h behind a C interface.
+#include "launch_plan.h"
+
+extern "C" {
+
+// out: lanes per ray, chunk, chunks, runs, scan blocks, merge blocks, the scan
+// launch's and the merge launch's work items in x
+void plan_linear(int n, int n_tri, long long* out) {
+    const eos::LinSplit s = eos::linear_split(n, n_tri);
+    out[0] = s.lanes_per_ray;
+    out[1] = s.chunk;
+    out[2] = s.n_chunks;
+    out[3] = (long long)s.runs;
+    out[4] = s.scan_blocks;
+    out[5] = s.merge_blocks;
+    out[6] = (long long)s.scan_blocks * eos::kLinTile;
+    out[7] = (long long)s.merge_blocks * eos::kLinMergeThreads;
+}
+
+long long plan_max_launch_items() { return (long long)eos::kMaxLaunchItems; }
+}

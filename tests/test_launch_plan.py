@@ -1,0 +1,50 @@
+"""Launch shapes and scratch sizes worked out on the host (eos_amd/csrc/launch_plan.h),
+at sizes up to the largest an entry point takes."""
+import ctypes as C
+import os
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+INT_MAX = 2**31 - 1
+STATIC_MAX_RAYS = 1 << 20
+
+pytestmark = pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
+
+
+@pytest.fixture(scope="module")
+def plan(tmp_path_factory):
+    so = tmp_path_factory.mktemp("plan") / "libplan.so"
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-shared", "-fPIC",
+                    "-I", os.path.join(ROOT, "include"), "-I", os.path.join(ROOT, "eos_amd", "csrc"),
+                    os.path.join(ROOT, "tests", "plan", "launch_plan.cpp"), "-o", str(so)], check=True)
+    lib = C.CDLL(str(so))
+    lib.plan_max_launch_items.restype = C.c_longlong
+    return lib
+
+
+def _linear(plan, n, n_tri):
+    out = (C.c_longlong * 8)()
+    plan.plan_linear(n, n_tri, out)
+    return dict(zip(("lanes", "chunk", "chunks", "runs", "scan_blocks", "merge_blocks", "scan_items", "merge_items"),
+                    out))
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 64, 127, 128, 129, 256, 257, 4000, 20000, 300_000, 2**19 - 1, 2**19, 2**19 + 1,
+                               2**20, 2**20 + 1, 2**26 - 1, 2**26, 2**26 + 1, 2**30, INT_MAX])
+def test_linear_split(plan, n):
+    limit = plan.plan_max_launch_items()
+    for n_tri in (0, 1, 255, 256, 257, 5000, 13312, 1_000_000, 2**28 - 1):
+        r = _linear(plan, n, n_tri)
+        # every ray and every triangle is covered, by launches of a permitted size
+        assert r["scan_items"] >= n * r["lanes"] and r["scan_items"] < limit, (n, n_tri, r)
+        assert r["chunk"] % 256 == 0 and r["chunk"] * r["chunks"] >= n_tri and 1 <= r["chunks"] <= 65535
+        assert r["chunk"] * (r["chunks"] - 1) < max(n_tri, 1)              # no chunk is empty
+        assert r["merge_items"] < limit, (n, n_tri, r)
+        # one run per ray is kept only where several lanes or chunks share a ray
+        if r["chunks"] == 1 and r["lanes"] == 1:
+            assert r["runs"] == 0 and r["merge_blocks"] == 0
+        else:
+            assert r["runs"] == n * r["chunks"] <= STATIC_MAX_RAYS and r["merge_items"] >= 64 * n
