@@ -16,8 +16,9 @@ constexpr size_t kMaxLaunchItems = (size_t)1 << 32;
 constexpr int kLinTile = 256;           // triangles staged at a time, and threads of the scanning kernels
 constexpr int kLinMergeThreads = 256;   // four rays, a wave each
 constexpr size_t kLinBlocks = 2048;     // scanning workgroups wanted
-constexpr size_t kLinRunBytes = 16;     // one ray's run over one chunk of triangles
-constexpr size_t kLinRuns = (size_t)EOS_STATIC_MAX_RAYS;   // at most
+constexpr size_t kLinRunBytes = 32;     // one ray's run over one chunk of triangles, and its head
+constexpr size_t kLinRuns = (size_t)1 << 20;   // kept at most
+constexpr size_t kLinStaticRuns = (size_t)EOS_STATIC_MAX_RAYS / 2;   // by eos_trace_rays_static: 16 bytes per ray of scratch
 constexpr int kLinFewRays = 128;        // up to here a ray's triangles are shared out over lanes as well
 
 struct LinSplit {
@@ -30,18 +31,18 @@ struct LinSplit {
 };
 
 // n rays (n >= 1) against n_tri triangles: as many chunks as give kLinBlocks
-// workgroups, at most one per kLinTile triangles, and runs within kLinRuns.  One
+// workgroups, at most one per kLinTile triangles, and runs within max_runs.  One
 // chunk needs no merge unless lanes share its rays: a merge there is a wave per
 // ray for a single run, 64 n work items, which passes the launch limit from 2^26
 // rays on.
-inline LinSplit linear_split(int n, int n_tri) {
+inline LinSplit linear_split(int n, int n_tri, size_t max_runs) {
     LinSplit r;
     if (n <= kLinFewRays)
         while (r.lanes_per_ray < 64 && 2 * r.lanes_per_ray * n <= kLinTile) r.lanes_per_ray *= 2;
     const size_t blocks = ((size_t)n * r.lanes_per_ray + kLinTile - 1) / kLinTile;
     const size_t tiles = std::max<size_t>(1, ((size_t)n_tri + kLinTile - 1) / kLinTile);
     size_t c = std::min(tiles, (kLinBlocks + blocks - 1) / blocks);
-    c = std::max<size_t>(1, std::min({c, kLinRuns / (size_t)n, (size_t)65535}));
+    c = std::max<size_t>(1, std::min({c, max_runs / (size_t)n, (size_t)65535}));
     const size_t per = (tiles + c - 1) / c;
     r.chunk = (int)(per * kLinTile);
     r.n_chunks = (int)((tiles + per - 1) / per);

@@ -64,56 +64,110 @@ __global__ __launch_bounds__(256) void k_query_hits(int n, const float* ro, cons
 // accepted, the reading of its uninitialised start value) and minDist (999999
 // at first): an accepted hit is kept when 0 < t < minDist.  found: some triangle
 // accepted a hit (the query's return value), even when none was kept.
-//   While no accepted hit had t = 0, minDist <= minTemp, so a hit is kept when
-// 0 < t < minDist; after a hit at t = 0 nothing is kept any more.  So a run of
-// consecutive triangles is summed up by its first least t in (0, 999999) before
-// its first hit at t = 0, and two neighbouring runs combine in order.  Only a
-// hit whose t is not a number (a NaN passes Moller-Trumbore's comparisons, and
-// lifts both bounds) does not fit: it is flagged, and its ray is walked again in
-// index order.
-struct LinRun {
+//   Until an accepted hit has t = 0, a hit beyond minTemp is beyond minDist too, so
+// a hit is kept when 0 < t < minDist; after a hit at t = 0 nothing is kept.  A
+// hit whose t is not a number (a NaN passes Moller-Trumbore's comparisons) is
+// accepted, lifts minTemp and leaves minDist, so hits are kept again.  A run of
+// consecutive triangles is summed up by the first least t in (0, 999999) among the
+// hits that it keeps: `head` those before its first NaN hit, which count only if
+// no t = 0 is open before the run, and `best` those after it (without a NaN hit all
+// are in `best`); and by whether a t = 0 is open at its end.  Neighbouring runs
+// combine in order.
+struct LinHit {
     float t = 999999.0f, u = 0.0f, v = 0.0f;
-    int best = -1;
-    bool found = false, zero = false, nan = false;
-    __device__ __forceinline__ void hit(float ht, float hu, float hv, int tri) {
-        found = true;
-        if (!(ht == ht)) nan = true;
-        if (!zero && ht < t && ht > 0.0f) {
-            t = ht;
-            u = hu;
-            v = hv;
-            best = tri;
-        }
-        zero |= ht <= 0.0f;
+    int tri = -1;
+    __device__ __forceinline__ void then(const LinHit& o) {
+        if (o.t < t) *this = o;
     }
-    // this run, then the one of the triangles after it
-    __device__ __forceinline__ void then(const LinRun& o) {
-        if (!zero && o.t < t) {
-            t = o.t;
-            u = o.u;
-            v = o.v;
-            best = o.best;
+    __device__ __forceinline__ float4 pack() const {
+        return make_float4(t, u, v, __uint_as_float((uint32_t)(tri + 1)));
+    }
+    __device__ __forceinline__ static LinHit unpack(float4 p) {
+        LinHit h;
+        h.t = p.x;
+        h.u = p.y;
+        h.v = p.z;
+        h.tri = (int)(__float_as_uint(p.w) & 0x1FFFFFFFu) - 1;
+        return h;
+    }
+};
+struct LinRun {
+    LinHit best;
+    bool found = false, zero = false, nan = false;
+    __device__ __forceinline__ void hit(float t, float u, float v, int tri) {
+        found = true;
+        if (!zero && t < best.t && t > 0.0f) {
+            best.t = t;
+            best.u = u;
+            best.v = v;
+            best.tri = tri;
         }
-        found |= o.found;
-        zero |= o.zero;
-        nan |= o.nan;
+        zero |= t <= 0.0f;
     }
     // 16 bytes in memory: t, u, v, then the triangle + 1 (at most 2^28) and the flags
     __device__ __forceinline__ float4 pack() const {
-        const uint32_t w = (uint32_t)(best + 1) | (found ? 1u << 29 : 0u) | (zero ? 1u << 30 : 0u) | (nan ? 1u << 31 : 0u);
-        return make_float4(t, u, v, __uint_as_float(w));
+        const uint32_t w = (uint32_t)(best.tri + 1) | (found ? 1u << 29 : 0u) | (zero ? 1u << 30 : 0u) | (nan ? 1u << 31 : 0u);
+        return make_float4(best.t, best.u, best.v, __uint_as_float(w));
     }
-    __device__ __forceinline__ static LinRun unpack(float4 p) {
+};
+struct LinSum : LinRun {
+    LinHit head;
+    __device__ __forceinline__ void lift() {
+        if (!nan) {
+            head = best;
+            best = LinHit();
+            nan = true;
+        }
+        zero = false;
+    }
+    __device__ __forceinline__ void hit(float t, float u, float v, int tri) {
+        if (t == t) {
+            LinRun::hit(t, u, v, tri);
+        } else {
+            found = true;
+            lift();
+        }
+    }
+    // this run, then the one of the triangles after it
+    __device__ __forceinline__ void then(const LinSum& o) {
+        const LinHit& first = o.nan ? o.head : o.best;
+        if (!zero) best.then(first);
+        if (o.nan) {
+            lift();
+            best.then(o.best);
+        }
+        found |= o.found;
+        zero |= o.zero;
+    }
+    // the kept hit of the run over all triangles
+    __device__ __forceinline__ LinHit kept() const {
+        LinHit k = nan ? head : best;
+        if (nan) k.then(best);
+        return k;
+    }
+    __device__ __forceinline__ static bool has_head(float4 p) { return (__float_as_uint(p.w) >> 31) != 0; }
+    __device__ __forceinline__ static LinSum unpack(float4 p, float4 head) {
         const uint32_t w = __float_as_uint(p.w);
-        LinRun r;
-        r.t = p.x;
-        r.u = p.y;
-        r.v = p.z;
-        r.best = (int)(w & 0x1FFFFFFFu) - 1;
+        LinSum r;
+        r.best = LinHit::unpack(p);
         r.found = (w >> 29) & 1u;
         r.zero = (w >> 30) & 1u;
         r.nan = (w >> 31) & 1u;
+        if (r.nan) r.head = LinHit::unpack(head);
         return r;
+    }
+    // the wave's runs combined in lane order, `lanes` (a power of two) at a time:
+    // right in the first lane of each
+    __device__ __forceinline__ void reduce(int lanes) {
+        for (int off = 1; off < lanes; off <<= 1) {
+            const float4 p = shfl_down4(pack(), off);
+            float4 h = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            if (__ballot(nan) != 0) h = shfl_down4(head.pack(), off);
+            then(unpack(p, h));
+        }
+    }
+    __device__ __forceinline__ static float4 shfl_down4(float4 p, int off) {
+        return make_float4(__shfl_down(p.x, off), __shfl_down(p.y, off), __shfl_down(p.z, off), __shfl_down(p.w, off));
     }
 };
 
@@ -149,47 +203,36 @@ struct LinArgs {
     const float *verts, *normals;    // the scene's triangles in their original order
     const int32_t *matidx, *xfi;
     const float4* xf;
-    float4* part;                    // [n_chunks][n] runs
+    float4* part;                    // [n_chunks][n] runs, then their heads
     float4* out;
+    __device__ __forceinline__ void keep(int chunk_no, int i, const LinRun& run) const {
+        part[(size_t)chunk_no * n + i] = run.pack();
+    }
+    __device__ __forceinline__ void keep_head(int chunk_no, int i, const LinHit& head) const {
+        part[(size_t)n_chunks * n + (size_t)chunk_no * n + i] = head.pack();
+    }
+    __device__ __forceinline__ LinSum kept(int chunk_no, int i) const {
+        const size_t k = (size_t)chunk_no * n + i;
+        const float4 p = part[k];
+        return LinSum::unpack(p, LinSum::has_head(p) ? part[(size_t)n_chunks * n + k] : p);
+    }
 };
 
-// A ray's answer from the run over all its triangles.  The kept hit's point goes
-// through M and its normal through transpose(inverse) without a second
-// normalisation.
-__device__ __forceinline__ void linear_answer(const LinArgs& a, int i, LinRay& ray, LinRun run) {
-    if (run.nan) {
-        // in index order, with both of the reference's bounds
-        float min_temp = INFINITY;
-        run = LinRun();
-        run.found = true;
-        for (int k = 0; k < a.n_tri; ++k) {
-            const float* w = a.verts + 9 * (size_t)k;
-            const F3 v1 = f3(w[0], w[1], w[2]);
-            const F3 e1 = sub(f3(w[3], w[4], w[5]), v1), e2 = sub(f3(w[6], w[7], w[8]), v1);
-            float t, u, v;
-            if (ray.test(a.xf, a.xfi ? a.xfi[k] : -1, v1, e1, e2, t, u, v) && !(t > min_temp)) {
-                min_temp = t;
-                if (t < run.t && t > 0.0f) {
-                    run.t = t;
-                    run.u = u;
-                    run.v = v;
-                    run.best = k;
-                }
-            }
-        }
-    }
+// A ray's answer from the hit its search kept.  The hit's point goes through M and
+// its normal through transpose(inverse) without a second normalisation.
+__device__ __forceinline__ void linear_answer(const LinArgs& a, int i, const LinRay& ray, bool found, const LinHit& k) {
     F3 P = {0, 0, 0}, N = {0, 0, 0};
-    if (run.best < 0) {
-        write_hit(a.out, (size_t)i, run.found, P, N, -1, INFINITY, 0.0f, 0.0f, -1);
+    if (k.tri < 0) {
+        write_hit(a.out, (size_t)i, found, P, N, -1, INFINITY, 0.0f, 0.0f, -1);
         return;
     }
-    const float* nn = a.normals + 9 * (size_t)run.best;
-    const int xi = a.xfi ? a.xfi[run.best] : -1;
+    const float* nn = a.normals + 9 * (size_t)k.tri;
+    const int xi = a.xfi ? a.xfi[k.tri] : -1;
     const float4 s0 = make_float4(nn[0], nn[1], nn[2], 0.0f);
     const float4 s1 = make_float4(nn[3], nn[4], nn[5], __int_as_float(xi));
     const float4 s2 = make_float4(nn[6], nn[7], nn[8], 0.0f);
-    hit_surface(s0, s1, s2, a.xf, ray.o, ray.d, run.t, run.u, run.v, false, P, N);
-    write_hit(a.out, (size_t)i, run.found, P, N, a.matidx[run.best], run.t, run.u, run.v, run.best);
+    hit_surface(s0, s1, s2, a.xf, ray.o, ray.d, k.t, k.u, k.v, false, P, N);
+    write_hit(a.out, (size_t)i, found, P, N, a.matidx[k.tri], k.t, k.u, k.v, k.tri);
 }
 
 // One run per ray and chunk of triangles, a workgroup per 256 rays and chunk:
@@ -223,13 +266,25 @@ __global__ __launch_bounds__(kLinTile) void k_query_linear(LinArgs a) {
         for (int j = 0; j < cnt; ++j) {
             const float4 p = tri[3 * j], q = tri[3 * j + 1], r = tri[3 * j + 2];
             float t, u, v;
-            if (ray.test(a.xf, __float_as_int(r.y), f3(p.x, p.y, p.z), f3(p.w, q.x, q.y), f3(q.z, q.w, r.x), t, u, v))
+            if (ray.test(a.xf, __float_as_int(r.y), f3(p.x, p.y, p.z), f3(p.w, q.x, q.y), f3(q.z, q.w, r.x), t, u, v)) {
                 run.hit(t, u, v, base + j);
+                if (__builtin_expect(!(t == t), 0)) {
+                    // the head goes to memory at once (in registers it cost 100,000 rays
+                    // against 4,000 triangles 583 -> 716 us); a run over every triangle
+                    // has nothing before it, and goes on with what it holds
+                    if (!run.nan && !a.finish) {
+                        a.keep_head((int)blockIdx.y, i, run.best);
+                        run.best = LinHit();
+                    }
+                    run.nan = true;
+                    run.zero = false;
+                }
+            }
         }
     }
     if (!act) return;
-    if (a.finish) linear_answer(a, i, ray, run);
-    else a.part[(size_t)blockIdx.y * a.n + i] = run.pack();
+    if (a.finish) linear_answer(a, i, ray, run.found, run.best);
+    else a.keep((int)blockIdx.y, i, run);
 }
 
 // The same with few rays: P lanes (a power of two) share a ray, each a slice of
@@ -240,7 +295,7 @@ __global__ __launch_bounds__(kLinTile) void k_query_linear_few(LinArgs a, int P)
     const bool act = i < a.n;
     const int c0 = (int)blockIdx.y * a.chunk, c1 = min(a.n_tri, c0 + a.chunk);
     const int len = a.chunk / P;
-    LinRun run;
+    LinSum run;
     if (act) {
         LinRay ray;
         ray.load(a.ro, a.rd, (size_t)i);
@@ -253,14 +308,10 @@ __global__ __launch_bounds__(kLinTile) void k_query_linear_few(LinArgs a, int P)
             if (ray.test(a.xf, a.xfi ? a.xfi[k] : -1, v1, e1, e2, t, u, v)) run.hit(t, u, v, k);
         }
     }
-    float4 mine = run.pack();
-    for (int off = 1; off < P; off <<= 1) {
-        const float4 o = make_float4(__shfl_down(mine.x, off), __shfl_down(mine.y, off), __shfl_down(mine.z, off),
-                                     __shfl_down(mine.w, off));
-        run.then(LinRun::unpack(o));   // right for the lanes the next steps read
-        mine = run.pack();
-    }
-    if (act && lane_p == 0) a.part[(size_t)blockIdx.y * a.n + i] = mine;
+    run.reduce(P);
+    if (!act || lane_p != 0) return;
+    a.keep((int)blockIdx.y, i, run);
+    if (run.nan) a.keep_head((int)blockIdx.y, i, run.head);
 }
 
 // A wave per ray of a query of several chunks: its runs combined in order (each
@@ -271,19 +322,13 @@ __global__ __launch_bounds__(kLinMergeThreads) void k_linear_merge(LinArgs a) {
     const int lane = __lane_id();
     const int per = (a.n_chunks + 63) / 64;
     const int b1 = min(a.n_chunks, (lane + 1) * per);
-    LinRun run;
-    for (int b = lane * per; b < b1; ++b) run.then(LinRun::unpack(a.part[(size_t)b * a.n + i]));
-    float4 mine = run.pack();
-    for (int off = 1; off < 64; off <<= 1) {
-        const float4 o = make_float4(__shfl_down(mine.x, off), __shfl_down(mine.y, off), __shfl_down(mine.z, off),
-                                     __shfl_down(mine.w, off));
-        run.then(LinRun::unpack(o));
-        mine = run.pack();
-    }
+    LinSum run;
+    for (int b = lane * per; b < b1; ++b) run.then(a.kept(b, i));
+    run.reduce(64);
     if (lane != 0) return;
     LinRay ray;
     ray.load(a.ro, a.rd, (size_t)i);
-    linear_answer(a, i, ray, run);
+    linear_answer(a, i, ray, run.found, run.kept());
 }
 
 // A linear query of n rays (n >= 1); part: room for the split's runs.
@@ -346,7 +391,7 @@ __global__ void k_zero_i32_query(int* p, int n) {
 constexpr size_t kStaticHeader = 4096;
 static_assert(4 * (size_t)kQueryCtrInts <= kStaticHeader, "cursors and flag fit the header");
 constexpr size_t kStaticBytes = kStaticHeader + 16 * (size_t)EOS_STATIC_MAX_RAYS;
-static_assert(kLinRunBytes * kLinRuns <= kStaticBytes - kStaticHeader, "a linear query's runs fit the records");
+static_assert(kLinRunBytes * kLinStaticRuns <= kStaticBytes - kStaticHeader, "a linear query's runs fit the records");
 __device__ __align__(256) unsigned char scratch[kStaticBytes];
 
 constexpr int kMaxDevices = 64;
@@ -378,7 +423,7 @@ eos_status trace_rays_static(eos_scene* s, int n, const float* o, const float* d
     float4* out = reinterpret_cast<float4*>(hits);
     const unsigned blocks = (unsigned)(((size_t)n + 255) / 256);
     if (opts->mode == EOS_QUERY_NEAREST_LINEAR) {
-        const LinSplit sp = linear_split(n, s->n_tri);
+        const LinSplit sp = linear_split(n, s->n_tri, kLinStaticRuns);
         launch_linear(linear_args(s, n, sp, o, d, rec, out), sp, S);
         EOS_HIP(hipGetLastError());
         EOS_HIP(hipStreamSynchronize(S));
@@ -463,7 +508,7 @@ eos_status trace_rays(eos_scene* s, int n, const float* o, const float* d, const
     const unsigned blocks = (unsigned)((nn + 255) / 256);
     int err = 0;
     if (mode == EOS_QUERY_NEAREST_LINEAR) {
-        const LinSplit sp = linear_split(n, s->n_tri);
+        const LinSplit sp = linear_split(n, s->n_tri, kLinRuns);
         EOS_TRY(s->q_rec.ensure(kLinRunBytes * sp.runs));
         launch_linear(linear_args(s, n, sp, ro, rd, s->q_rec.as<float4>(), out), sp, S);
         EOS_HIP(hipGetLastError());

@@ -320,7 +320,8 @@ eos_status eos_trace_rays(eos_scene* scene, int32_t n, const float* origins, con
  * memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc): eos_trace_rays with no allocation.  Its scratch (fetch
  * cursors, error flag and, for EOS_QUERY_NEAREST, 16 bytes of hit record per
- * ray) is one fixed device array of the library, 4 KiB + 16 B x
+ * ray; for EOS_QUERY_NEAREST_LINEAR the partial results that its launches
+ * combine) is one fixed device array of the library, 4 KiB + 16 B x
  * EOS_STATIC_MAX_RAYS (16 MiB), held by every GPU the library runs on until the
  * process ends.  n above EOS_STATIC_MAX_RAYS fails with EOS_ERR_LIMIT; rays and
  * outputs must be device memory (opts->memory = EOS_MEM_DEVICE).  Calls on one

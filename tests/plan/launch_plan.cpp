@@ -4,9 +4,9 @@
 extern "C" {
 
 // out: lanes per ray, chunk, chunks, runs, scan blocks, merge blocks, the scan
-// launch's and the merge launch's work items in x
-void plan_linear(int n, int n_tri, long long* out) {
-    const eos::LinSplit s = eos::linear_split(n, n_tri);
+// launch's and the merge launch's work items in x, bytes of the runs
+void plan_linear(int n, int n_tri, int fixed_scratch, long long* out) {
+    const eos::LinSplit s = eos::linear_split(n, n_tri, fixed_scratch ? eos::kLinStaticRuns : eos::kLinRuns);
     out[0] = s.lanes_per_ray;
     out[1] = s.chunk;
     out[2] = s.n_chunks;
@@ -15,6 +15,7 @@ void plan_linear(int n, int n_tri, long long* out) {
     out[5] = s.merge_blocks;
     out[6] = (long long)s.scan_blocks * eos::kLinTile;
     out[7] = (long long)s.merge_blocks * eos::kLinMergeThreads;
+    out[8] = (long long)(s.runs * eos::kLinRunBytes);
 }
 
 long long plan_max_launch_items() { return (long long)eos::kMaxLaunchItems; }

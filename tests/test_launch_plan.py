@@ -25,19 +25,22 @@ def plan(tmp_path_factory):
     return lib
 
 
-def _linear(plan, n, n_tri):
-    out = (C.c_longlong * 8)()
-    plan.plan_linear(n, n_tri, out)
-    return dict(zip(("lanes", "chunk", "chunks", "runs", "scan_blocks", "merge_blocks", "scan_items", "merge_items"),
-                    out))
+def _linear(plan, n, n_tri, static):
+    out = (C.c_longlong * 9)()
+    plan.plan_linear(n, n_tri, int(static), out)
+    return dict(zip(("lanes", "chunk", "chunks", "runs", "scan_blocks", "merge_blocks", "scan_items", "merge_items",
+                     "bytes"), out))
 
 
 @pytest.mark.parametrize("n", [1, 2, 3, 64, 127, 128, 129, 256, 257, 4000, 20000, 300_000, 2**19 - 1, 2**19, 2**19 + 1,
                                2**20, 2**20 + 1, 2**26 - 1, 2**26, 2**26 + 1, 2**30, INT_MAX])
-def test_linear_split(plan, n):
+@pytest.mark.parametrize("static", [False, True])
+def test_linear_split(plan, n, static):
+    if static and n > STATIC_MAX_RAYS:
+        pytest.skip("refused by eos_trace_rays_static")
     limit = plan.plan_max_launch_items()
     for n_tri in (0, 1, 255, 256, 257, 5000, 13312, 1_000_000, 2**28 - 1):
-        r = _linear(plan, n, n_tri)
+        r = _linear(plan, n, n_tri, static)
         # every ray and every triangle is covered, by launches of a permitted size
         assert r["scan_items"] >= n * r["lanes"] and r["scan_items"] < limit, (n, n_tri, r)
         assert r["chunk"] % 256 == 0 and r["chunk"] * r["chunks"] >= n_tri and 1 <= r["chunks"] <= 65535
@@ -47,4 +50,5 @@ def test_linear_split(plan, n):
         if r["chunks"] == 1 and r["lanes"] == 1:
             assert r["runs"] == 0 and r["merge_blocks"] == 0
         else:
-            assert r["runs"] == n * r["chunks"] <= STATIC_MAX_RAYS and r["merge_items"] >= 64 * n
+            assert r["runs"] == n * r["chunks"] and r["merge_items"] >= 64 * n
+            assert r["bytes"] <= (16 if static else 32) * STATIC_MAX_RAYS
