@@ -54,4 +54,23 @@ inline LinSplit linear_split(int n, int n_tri, size_t max_runs) {
     return r;
 }
 
+// ---- tree queries (eos_trace_rays) ----------------------------------------------
+constexpr int kQueryThreads = 256;
+
+// Workgroups of a query's traversal launch: room for the walk of a whole wave per
+// ray (two waves per ray; waves beyond the rays leave at once), never more than the
+// persistent grid of `resident` workgroups.  With a quad per ray the launch was too
+// small for any group walk: 1,000 host rays against 70k triangles 142 us, now 83.
+inline int query_grid(size_t n, int resident) {
+    return (int)std::min<size_t>((size_t)resident, std::max<size_t>(1, (128 * n + kQueryThreads - 1) / kQueryThreads));
+}
+
+// Lanes of that launch that can have a stack outgrow LDS: those of the walk with a
+// ray per lane, whose waves beyond the ones that n rays fill leave before they touch
+// it.  Group and wave walks keep their stacks in LDS.  (Sized for the whole grid, a
+// scene's first query of 1,000 rays allocated 40 MiB.)
+inline size_t query_stack_lanes(size_t n, int grid) {
+    return std::min((size_t)grid * kQueryThreads, 64 * ((n + 63) / 64));
+}
+
 }  // namespace eos

@@ -515,14 +515,10 @@ eos_status trace_rays(eos_scene* s, int n, const float* o, const float* d, const
     } else {
         const LaunchCfg& cfg = s->cfg;
         const int trace_grid = std::max(1, s->num_cu * cfg.waves_per_cu / 4);
-        // room for the walk of a whole wave per ray (two waves per ray; waves beyond
-        // the rays leave at once), never more workgroups than the persistent grid.
-        // With a quad per ray the launch was too small for any group walk: 1,000
-        // host rays against 70k triangles 142 us, now 83
-        const int grid = (int)std::min<size_t>((size_t)trace_grid, std::max<size_t>(1, (128 * nn + 255) / 256));
+        const int grid = query_grid(nn, trace_grid);
         const int maxs = s->width == 4 ? kMaxStack4 : kMaxStack;
         EOS_TRY(s->q_ctr.ensure(4 * (size_t)kQueryCtrInts));
-        EOS_TRY(s->q_gstack.ensure(4 * (size_t)grid * 256 * (maxs - 16)));
+        EOS_TRY(s->q_gstack.ensure(4 * query_stack_lanes(nn, grid) * (size_t)(maxs - 16)));
         int* ctr = s->q_ctr.as<int>();
         hipLaunchKernelGGL(k_zero_i32_query, dim3(1), dim3(256), 0, S, ctr, kQueryCtrInts);
         TraceArgs a{};

@@ -18,5 +18,12 @@ void plan_linear(int n, int n_tri, int fixed_scratch, long long* out) {
     out[8] = (long long)(s.runs * eos::kLinRunBytes);
 }
 
+// out: workgroups, lanes with an overflow stack
+void plan_query(long long n, int resident, long long* out) {
+    const int grid = eos::query_grid((size_t)n, resident);
+    out[0] = grid;
+    out[1] = (long long)eos::query_stack_lanes((size_t)n, grid);
+}
+
 long long plan_max_launch_items() { return (long long)eos::kMaxLaunchItems; }
 }

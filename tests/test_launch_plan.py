@@ -52,3 +52,18 @@ def test_linear_split(plan, n, static):
         else:
             assert r["runs"] == n * r["chunks"] and r["merge_items"] >= 64 * n
             assert r["bytes"] <= (16 if static else 32) * STATIC_MAX_RAYS
+
+
+@pytest.mark.parametrize("resident", [1, 64, 1280, 4096])
+def test_query_stacks(plan, resident):
+    out = (C.c_longlong * 2)()
+    for n in (1, 2, 63, 64, 65, 100, 255, 256, 257, 1000, 5000, 20000, 81919, 81920, 81921, 1_000_003, INT_MAX):
+        plan.plan_query(C.c_longlong(n), resident, out)
+        grid, lanes = out
+        assert 1 <= grid <= resident and grid * 256 < plan.plan_max_launch_items()
+        # a wave beyond the ceil(n / 64) that a ray per lane fills leaves at once; every wave
+        # before has room for each of its lanes
+        walking = min(4 * grid, (n + 63) // 64)
+        assert 64 * walking == lanes, (n, grid, lanes)
+        # no more than the rays, but for the last wave
+        assert lanes < n + 64
