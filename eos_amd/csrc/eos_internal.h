@@ -149,8 +149,9 @@ struct eos_frame_buffers {
     int lslots = 1;         // light slots per surface
     size_t surf_stride() const { return 2 * cap; }                // float4 per level
     size_t vis_stride() const { return cap * (size_t)lslots; }    // bytes per level
-    float4* surf_at(int l) { return surf.as<float4>() + (size_t)l * surf_stride(); }
-    uint8_t* vis_at(int l) { return vis.as<uint8_t>() + (size_t)l * vis_stride(); }
+    size_t surf_first(int l) const { return tree ? tslot[l & 1] : (size_t)l * cap; }   // surfaces before level l's
+    float4* surf_at(int l) { return surf.as<float4>() + 2 * surf_first(l); }
+    uint8_t* vis_at(int l) { return vis.as<uint8_t>() + surf_first(l) * (size_t)lslots; }
     eos::DevBuf levcol;     // float4 [(D+1) * npix]  level colour rgb + reflection weight
     eos::DevBuf levels;     // uint8  [npix]
     eos::DevBuf counters;   // int64  [64]
@@ -167,9 +168,11 @@ struct eos_frame_buffers {
     // Ray trees (scenes with transparent materials): level l holds at most
     // tcap[l] rays / hits at offset toff[l] of rayhit (hit index per ray; level
     // 0 per pixel), aux (Fresnel weight, children) and hitcol (colour per hit);
-    // surf / vis then hold two levels, level l in slot l % 2, and the queues one.
+    // the queues then hold one level, and surf / vis two, level l in slot l % 2 from
+    // tslot[l % 2] on, each slot as large as its largest level (one slot for all
+    // levels where a frame runs on one stream).
     bool tree = false;
-    size_t tcap[EOS_MAX_DEPTH + 1] = {}, toff[EOS_MAX_DEPTH + 2] = {};
+    size_t tcap[EOS_MAX_DEPTH + 1] = {}, toff[EOS_MAX_DEPTH + 2] = {}, tslot[2] = {};
     eos::DevBuf rayhit, aux, hitcol;
     size_t npix = 0, n_ids = 0;
     int depth = -1, n_light = -1;

@@ -867,11 +867,16 @@ int chain_shadow_span(const Frame& f) {
     return (int)std::min<size_t>((size_t)std::max(f.depth, 1), std::max<size_t>(1, kMaxItems / per_level));
 }
 
+// Ray trees in flight stay on one stream: the other frame fills the GPU (four
+// samples of a 1365 x 767 glass frame 2649 us, 2878 on two streams).
+bool one_stream(const Frame& f) { return f.tree && f.in_flight; }
+
 eos_status ensure_buffers(eos_frame_buffers& fb, const Frame& f, int trace_grid) {
     if (f.n_ids > kMaxItems || f.npix * (size_t)std::max(f.lstride, 1) > kMaxItems)
         return fail(EOS_ERR_LIMIT, "frame too large: pixels times light slots must stay below 2^31 (" +
                                        std::to_string(f.npix) + " pixels, " + std::to_string(f.lstride) + " lights)");
     size_t cap = f.npix;
+    size_t surfaces = cap * (size_t)(f.depth + 1);   // held in surf and vis
     fb.tree = f.tree;
     if (f.tree) {
         // level l holds at most twice the rays of level l - 1 (two children per hit),
@@ -886,16 +891,24 @@ eos_status ensure_buffers(eos_frame_buffers& fb, const Frame& f, int trace_grid)
         EOS_TRY(fb.rayhit.ensure(4 * fb.toff[f.depth + 1]));
         EOS_TRY(fb.aux.ensure(16 * fb.toff[f.depth + 1]));
         EOS_TRY(fb.hitcol.ensure(16 * fb.toff[f.depth + 1]));
+        // a second slot only where a level is shaded while the next one is set up (held
+        // for frames in flight as well, and both as large as the last level, it was 0.5 GB
+        // of a 1080p frame of depth 3, in each of two frames in flight)
+        size_t slot[2] = {0, 0};
+        for (int l = 0; l <= f.depth; ++l) slot[l & 1] = std::max(slot[l & 1], fb.tcap[l]);
+        const bool one = one_stream(f);
+        fb.tslot[0] = 0;
+        fb.tslot[1] = one ? 0 : slot[0];
+        surfaces = one ? cap : slot[0] + slot[1];
     }
-    const int surf_levels = f.tree ? std::min(2, f.depth + 1) : f.depth + 1;   // trees: a slot per parity
     EOS_TRY(fb.hit0.ensure(16 * f.n_ids));
     EOS_TRY(fb.q[0].ensure(32 * cap));
     EOS_TRY(fb.q[1].ensure(32 * cap));
     EOS_TRY(fb.hitq.ensure(16 * cap));
     fb.cap = cap;
     fb.lslots = std::max(f.lstride, 1);
-    EOS_TRY(fb.surf.ensure(16 * fb.surf_stride() * (size_t)surf_levels));
-    EOS_TRY(fb.vis.ensure(fb.vis_stride() * (size_t)surf_levels));
+    EOS_TRY(fb.surf.ensure(32 * surfaces));
+    EOS_TRY(fb.vis.ensure(surfaces * (size_t)fb.lslots));
     EOS_TRY(fb.levcol.ensure(16 * f.npix * (size_t)(f.depth + 1)));
     EOS_TRY(fb.levels.ensure(f.npix));
     EOS_TRY(fb.counters.ensure(4 * (size_t)kCounterInts));
@@ -917,9 +930,7 @@ eos_status enqueue_frame(eos_frame_buffers& fb, const Frame& f, const FrameStrea
     unsigned long long* stats = reinterpret_cast<unsigned long long*>(fb.counters.as<char>() + 4 * CTR_COUNT);
     const unsigned shade_grid = (unsigned)f.num_cu * 8;
     const hipStream_t S = fs.S;
-    // ray trees in flight stay on one stream: the other frame fills the GPU (four
-    // samples of a 1365 x 767 glass frame 2649 us, 2878 on two streams)
-    const bool two = fs.S2 != nullptr && !(f.tree && f.in_flight);
+    const bool two = fs.S2 != nullptr && !one_stream(f);
     const hipStream_t S2 = two ? fs.S2 : fs.S;
     int ev = 0;
     auto rec = [&](hipStream_t st) -> int {
@@ -942,8 +953,6 @@ eos_status enqueue_frame(eos_frame_buffers& fb, const Frame& f, const FrameStrea
     // random scenes 4434 us with four, 3993 with two or none; four glass samples 2647,
     // 2497, 2576; a chain frame of 4.2M triangles 1729, 1732, 1904)
     const int scatter = f.batch || f.tree ? std::min(f.cfg.scatter, 2) : f.cfg.scatter;
-    // where a level's surfaces and visibility lie
-    auto slot_of = [&](int l) { return f.tree ? l & 1 : l; };
     // Any-hit trace of levels [l0, l1] in one launch, then Phong of each level.
     auto shadow_and_phong = [&](int l0, int l1, hipStream_t st, size_t gstack_off, int slot) -> eos_status {
         F.s[2 * slot] = rec(st);
@@ -969,8 +978,8 @@ eos_status enqueue_frame(eos_frame_buffers& fb, const Frame& f, const FrameStrea
             sh.count_ptr = ctr + CTR_HITS + l0;
             sh.count_mul = f.lstride;
             sh.nlev = l1 - l0 + 1;
-            sh.surf = fb.surf_at(slot_of(l0));
-            sh.vis_out = fb.vis_at(slot_of(l0));
+            sh.surf = fb.surf_at(l0);
+            sh.vis_out = fb.vis_at(l0);
             sh.surf_stride = (long long)fb.surf_stride();
             sh.vis_stride = (long long)fb.vis_stride();
             // level 0's shadow launch on the second stream shares the CUs with the
@@ -1000,8 +1009,8 @@ eos_status enqueue_frame(eos_frame_buffers& fb, const Frame& f, const FrameStrea
         pa.npix = (int)f.npix;
         pa.lstride = f.lstride;
         pa.count_ptr = ctr + CTR_HITS + l0;
-        pa.surf = fb.surf_at(slot_of(l0));
-        pa.vis = fb.vis_at(slot_of(l0));
+        pa.surf = fb.surf_at(l0);
+        pa.vis = fb.vis_at(l0);
         pa.surf_stride = (long long)fb.surf_stride();
         pa.vis_stride = (long long)fb.vis_stride();
         pa.levcol = fb.levcol.as<float4>();
@@ -1108,7 +1117,7 @@ eos_status enqueue_frame(eos_frame_buffers& fb, const Frame& f, const FrameStrea
         sa.count_ptr = ctr + CTR_Q + l;
         sa.q_in = qin;
         sa.hit_in = l == 0 ? fb.hit0.as<float4>() : fb.hitq.as<float4>();
-        sa.surf_out = fb.surf_at(slot_of(l));
+        sa.surf_out = fb.surf_at(l);
         sa.hits_ctr = ctr + CTR_HITS + l;
         sa.q_out = qout;
         sa.q_out_ctr = ctr + CTR_Q + l + 1;
@@ -1118,7 +1127,7 @@ eos_status enqueue_frame(eos_frame_buffers& fb, const Frame& f, const FrameStrea
             sa.aux = fb.aux.as<float4>() + fb.toff[l];
         }
         sa.shadow_ctr = ctr + CTR_SHADOW + l;
-        sa.vis_out = f.count || f.walk_all ? nullptr : fb.vis_at(slot_of(l));
+        sa.vis_out = f.count || f.walk_all ? nullptr : fb.vis_at(l);
         sa.lstride = f.lstride;
         sa.levels = fb.levels.as<uint8_t>();
         sa.hit_ids = l == 0 ? f.hits : nullptr;
