@@ -7,6 +7,7 @@
 #include <vector>
 
 #include "../../include/eos_c.h"
+#include "launch_plan.h"
 
 namespace eos {
 
@@ -119,14 +120,14 @@ struct LaunchCfg {
     int workgroup = 256;
     int stack_lds = 16;
     int waves_per_cu = 20;
-    int refill = 16;
+    int refill = kRefillDefault;
     int batch = 64;        // most items a traversal wave claims per fetch
     int packets = 0;       // primary rays as one 8x8 packet per wave (4-wide tree)
     int coop = 0;          // quad-cooperative walk (0: never; work stealing serves the short launches)
     int group = 1;         // group walk (16 lanes per ray) for launches with at most one item per 16 lanes
     int group_lanes = 64;  // widest group: a whole wave per ray for launches of at most one item per two waves
     int steal = 1;         // per-lane walk: idle lanes of a drained wave help its remaining rays
-    int scatter = 4;       // launches of at most four items per lane claim them in scattered order
+    int scatter = kScatterDefault;   // launches of at most four items per lane claim them in scattered order
     int cull = 1;          // single-scene frames: primary tiles whose rays all miss the root's child boxes are not traced
     // frames two in flight share the GPU: fewer waves per launch, larger claims
     int frames_waves_per_cu = 16;

@@ -18,7 +18,6 @@
 #include <string>
 
 #include "eos_internal.h"
-#include "launch_plan.h"
 #include "trace.h"
 
 namespace eos {
@@ -528,18 +527,13 @@ eos_status trace_rays(eos_scene* s, int n, const float* o, const float* d, const
         a.cursor = ctr;
         a.err = ctr + kRanges * kCursorStride;
         a.gstack = s->q_gstack.as<int32_t>();
-        // a caller's rays diverge from the first node, so a refill that waits for twice as
-        // many idle lanes loses little and is paid half as often (1M nearest rays 543 ->
-        // 521 us, 500,000 occlusion rays 408 -> 379)
-        a.refill = std::min(64, 2 * cfg.refill);
+        a.refill = query_refill(cfg.refill);
         a.batch = cfg.batch;
         a.coop = cfg.coop;
         a.group = cfg.group;
         a.group_lanes = cfg.group_lanes;
         a.steal = cfg.steal;
-        // rays of a caller come in any order: claims are scattered only while a lane has
-        // one ray (1M rays 568 us with up to four per lane scattered, 555 without)
-        a.scatter = std::min(cfg.scatter, 1);
+        a.scatter = query_scatter(cfg.scatter);
         a.ray_o = ro;
         a.ray_d = rd;
         if (mode == EOS_QUERY_OCCLUDED) {

@@ -948,11 +948,7 @@ eos_status enqueue_frame(eos_frame_buffers& fb, const Frame& f, const FrameStrea
     // the tile test zeroes the counters on its way
     if (!cull) hipLaunchKernelGGL(k_zero_i32, dim3(16), dim3(256), 0, S, ctr, kCounterInts);
     F.start = rec(S);
-    // Batched frames and ray trees scatter their claims only up to two items per
-    // lane: beyond that the order's locality is worth more than the balance (16
-    // random scenes 4434 us with four, 3993 with two or none; four glass samples 2647,
-    // 2497, 2576; a chain frame of 4.2M triangles 1729, 1732, 1904)
-    const int scatter = f.batch || f.tree ? std::min(f.cfg.scatter, 2) : f.cfg.scatter;
+    const int scatter = frame_scatter(f.cfg.scatter, f.batch || f.tree);
     // Any-hit trace of levels [l0, l1] in one launch, then Phong of each level.
     auto shadow_and_phong = [&](int l0, int l1, hipStream_t st, size_t gstack_off, int slot) -> eos_status {
         F.s[2 * slot] = rec(st);

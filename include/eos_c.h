@@ -355,7 +355,8 @@ typedef struct eos_launch_config {
     int32_t workgroup;        /* 64, 128 or 256 threads */
     int32_t stack_lds;        /* per-lane LDS stack entries: 8, 16 or 32 */
     int32_t waves_per_cu;     /* persistent waves per CU launched */
-    int32_t refill;           /* idle lanes that trigger a refill, 1..64 */
+    int32_t refill;           /* idle lanes that trigger a refill, 1..64 (the default, 16, stands for 32 in
+                                 ray queries) */
     int32_t batch;            /* ray batch: most items a wave claims per fetch, 1..4096 */
     int32_t primary_packets;  /* 1: primary rays walk the 4-wide tree as 8x8-pixel packets, one per wave
                                  (pays off when triangles cover many pixels; 0, the default, walks per ray) */
@@ -374,7 +375,9 @@ typedef struct eos_launch_config {
                                  never do); 0: each ray is walked by one lane to the end */
     int32_t scatter;          /* launches with at most scatter x lanes items claim them in a scattered
                                  order (item i * p mod n, p prime), so neighbouring rays -- often long
-                                 together -- go to different waves; 0: never.  Results do not change */
+                                 together -- go to different waves; 0: never.  Results do not change (the
+                                 default, 4, stands for 2 in batched frames and frames with transparent
+                                 materials, and for 1 in ray queries) */
     int32_t group_lanes;      /* widest group walk: 64 (launches with at most group x lanes/128 items walk
                                  each ray with a whole wave, 16 nodes per step) or 16 (never wider) */
     int32_t cull;             /* 1: before a single scene's primary rays (4-wide tree) are traced, a tile

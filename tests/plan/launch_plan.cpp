@@ -25,5 +25,13 @@ void plan_query(long long n, int resident, long long* out) {
     out[1] = (long long)eos::query_stack_lanes((size_t)n, grid);
 }
 
+// out: scatter of chain frames, of batches and ray trees, of queries; refill of queries
+void plan_knobs(int refill, int scatter, int* out) {
+    out[0] = eos::frame_scatter(scatter, false);
+    out[1] = eos::frame_scatter(scatter, true);
+    out[2] = eos::query_scatter(scatter);
+    out[3] = eos::query_refill(refill);
+}
+
 long long plan_max_launch_items() { return (long long)eos::kMaxLaunchItems; }
 }

@@ -67,3 +67,16 @@ def test_query_stacks(plan, resident):
         assert 64 * walking == lanes, (n, grid, lanes)
         # no more than the rays, but for the last wave
         assert lanes < n + 64
+
+
+def test_a_callers_knobs_are_taken_as_they_are(plan):
+    from eos_amd import _lib as E
+    refill, scatter = E.Scene.DEFAULT_LAUNCH["refill"], E.Scene.DEFAULT_LAUNCH["scatter"]
+    out = (C.c_int * 4)()
+    for r in range(1, 65):
+        for s in range(0, 65):
+            plan.plan_knobs(r, s, out)
+            assert out[0] == s
+            assert out[1] == (2 if s == scatter else s)
+            assert out[2] == (1 if s == scatter else s)
+            assert out[3] == (32 if r == refill else r)
