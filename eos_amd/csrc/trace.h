@@ -64,10 +64,10 @@ __device__ __forceinline__ bool tile_pixel(int r, int tiles_x, int W, int H, int
 }
 
 // 1.0f / x, correctly rounded: the hardware's estimate and one Newton step with
-// fused multiply-adds give the IEEE quotient for every x with 2^-126 <= |x| < 2^126
-// (all such floats checked against the division); larger ones divide.  Below
-// 2^-126 the value differs (the one caller rejects those determinants whatever
-// their reciprocal).  Three instructions instead of the division's eleven.
+// fused multiply-adds give the IEEE quotient below 2^126 (tests/test_gpu_determinants.py
+// compares every float from 10^-5 up); larger ones divide.  The one caller rejects
+// smaller determinants whatever their reciprocal, which is another one below
+// 2^-126.  Three instructions instead of the division's eleven.
 __device__ __forceinline__ float reciprocal(float x) {
     float r = __builtin_amdgcn_rcpf(x);
     r = __builtin_fmaf(__builtin_fmaf(-x, r, 1.0f), r, r);
