@@ -10,16 +10,19 @@ resident in HBM and the RGBA8 output written to device memory.
 value = (primary + shadow + secondary rays per frame) * steps / wall time, the
 steps rendered by eos_render_frames (two frames in flight: a frame's primary
 rays trace while the previous frame's shadow and reflection launches finish);
-single_frame reports one eos_render call per frame (latency).
+single_frame reports one eos_render call per frame (latency).  Shadow rays toward
+a light that adds nothing to its surface are counted and not walked.
 
 Also reported:
   roofline      dominant kernel (the primary-ray closest-hit launch): algorithmic
                 bytes per launch = 128 B per 4-wide node visit (64 B per binary
                 node visit) + 36 B per triangle test + 16 B hit record per ray, from the counting variant of the same
-                traversal (deterministic, so equal to the timed launches), less the
-                root visit and hit record of each primary ray the tile test resolved
-                (the timed launch does neither for them), divided by the launch's
-                mean duration (tile test included) from HIP events on its stream.
+                traversal, less the root visit and hit record of each primary ray the
+                tile test resolved (the timed launch does neither for them), divided by
+                the launch's mean duration (tile test included) from HIP events on its
+                stream.  An upper bound: the timed walk drops pending nodes that lie
+                behind the nearest hit without reading them, the counting walk visits
+                them.  traffic and l2_hit_rate are those of the committed profile.
   cpu_baseline  the timing-faithful port of the reference's OpenMP CPU path on a
                 stratified pixel sample of the same frame.
   aa            the config C frame with 2x2 anti-aliasing samples per pixel
@@ -56,6 +59,9 @@ sys.path.insert(0, ROOT)
 HBM_PEAK_GBS = 8000.0
 NODE_BYTES = {2: 64, 4: 128}   # binary node / 4-wide node
 TRI_BYTES, HIT_BYTES = 36, 16
+ACHIEVED_NOTE = ("upper bound: bytes of the counting walk over the time of the timed walk, which drops pending nodes "
+                 "behind the nearest hit without reading them")
+TRAFFIC_NOTE = "HBM bytes and L2 hit rate as counted in the committed profile, over this run's launch time"
 
 
 def _profile(workload: str) -> dict:
@@ -346,17 +352,18 @@ def _primary_roofline(counted, per, width_bytes, n_ids):
             "primary_culled": culled,
             "node_visits": int(counted["closest_visits_first"]), "tri_tests": int(counted["closest_tests_first"]),
             "achieved": round(alg / (t * 1e-3) / 1e9, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-            "frac": round(alg / (t * 1e-3) / 1e9 / HBM_PEAK_GBS, 4)}
+            "frac": round(alg / (t * 1e-3) / 1e9 / HBM_PEAK_GBS, 4), "achieved_note": ACHIEVED_NOTE}
 
 
 def _with_traffic(roof: dict, prefix: str) -> dict:
-    """Adds the measured HBM bytes and L2 hit rate of the launch (rocprofv3
-    --pmc, profiles/traffic_config_c.json) to a roofline block."""
+    """Adds the HBM bytes and L2 hit rate of the launch as the committed profile
+    counted them (rocprofv3 --pmc, profiles/traffic_config_c.json; not this run) to
+    a roofline block."""
     prof = _profile("config_c")
     traffic = prof.get(prefix + roof["kernel"])
     t = roof["launch_ms"]
     roof.update({"traffic": traffic, "l2_hit_rate": prof.get(prefix + roof["kernel"] + "_l2_hit_rate"),
-                 "traffic_source": prof.get("source"),
+                 "traffic_source": prof.get("source"), "traffic_note": TRAFFIC_NOTE,
                  "hbm_achieved": round(traffic / (t * 1e-3) / 1e9, 2) if traffic else None,
                  "hbm_frac": round(traffic / (t * 1e-3) / 1e9 / HBM_PEAK_GBS, 4) if traffic else None})
     return roof
@@ -673,7 +680,8 @@ def main() -> int:
                      "launch_ms_in_flight": round(t_first_flight, 4),
                      "frac_in_flight": round(alg_bytes / (t_first_flight * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
                      "l2_hit_rate": l2_hit,
-                     "traffic_source": prof.get("source"),
+                     "traffic_source": prof.get("source"), "traffic_note": TRAFFIC_NOTE,
+                     "achieved_note": ACHIEVED_NOTE,
                      "alg_bytes_per_launch": int(alg_bytes),
                      "primary_culled": culled,
                      "node_visits": int(counted["closest_visits_first"]),
@@ -684,7 +692,9 @@ def main() -> int:
                      "hbm_achieved": round(traffic / (t_first * 1e-3) / 1e9, 2) if traffic else None,
                      "hbm_frac": round(traffic / (t_first * 1e-3) / 1e9 / HBM_PEAK_GBS, 4) if traffic else None},
         "rays_per_frame": {"primary": st["primary_rays"], "shadow": st["shadow_rays"],
-                           "secondary": st["secondary_rays"], "hits": st["hits"]},
+                           "secondary": st["secondary_rays"], "hits": st["hits"],
+                           "note": "value counts one shadow ray per hit and light; those toward a light that adds "
+                                   "nothing to its surface (about a fifth of them here) are answered without a walk"},
         "gpu_ms": {"render": round(mean("render_ms"), 4),
                    "trace_closest": round(float(np.mean([p["trace_closest_ms"] for p in per_t])), 4),
                    "trace_shadow": round(float(np.mean([p["trace_shadow_ms"] for p in per_t])), 4),

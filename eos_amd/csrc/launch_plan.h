@@ -61,21 +61,27 @@ inline LinSplit linear_split(int n, int n_tri, size_t max_runs) {
 constexpr int kRefillDefault = 16, kScatterDefault = 4;
 
 // Batched frames and ray trees scatter their claims up to two items per lane: beyond
-// that the order's locality is worth more than the balance (16 random scenes 4434 us
-// with four, 3993 with two or none; four glass samples in flight 2647 with four, 2497 with two, 2576 with none;
-// single 1080p glass frames of depth 3 1245-1255 with any of 0 to 6; a chain frame of
-// 4.2M triangles 1729 with four, 1732, 1904).
+// that the order's locality is worth more than the balance.  16 random scenes 4434 us
+// with four, 3993 with two or none; eight of 30,000 triangles 2027 with five, 1916
+// with two; three or sixteen small ones, whose launches have one item per lane, the
+// same with one to five, 5-12% more with none.  Four glass samples in flight 2647 with
+// four, 2497 with two, 2576 with none; single glass frames of 700 x 400 to 1920 x 1080
+// within 4% with any.  A chain frame of 4.2M triangles 1729 with four, 1732 with two,
+// 1904 with none.
 inline int frame_scatter(int scatter, bool batch_or_tree) {
     return batch_or_tree && scatter == kScatterDefault ? 2 : scatter;
 }
 
 // A caller's rays diverge from the first node, so a refill that waits for twice as
-// many idle lanes loses little and is paid half as often (1M nearest rays 543 ->
-// 521 us, 500,000 occlusion rays 408 -> 379).
+// many idle lanes loses little and is paid half as often: 1M nearest rays 543 ->
+// 521 us, 500,000 occlusion rays 408 -> 379; over four scenes, both modes and 3,000
+// to 1M rays 32 idle lanes against 17 are 0-10% faster, but for 30,000 nearest rays
+// among random triangles, 3% slower.
 inline int query_refill(int refill) { return refill == kRefillDefault ? 2 * refill : refill; }
 
 // Rays of a caller come in any order: claims are scattered only while a lane has
-// one ray (1M rays 568 us with up to four per lane scattered, 555 without).
+// one ray (1M rays 568 us with up to four per lane scattered, 555 without; 1M
+// occlusion rays 3-5% slower scattered, fewer rays the same).
 inline int query_scatter(int scatter) { return scatter == kScatterDefault ? 1 : scatter; }
 
 // ---- tree queries (eos_trace_rays) ----------------------------------------------

@@ -982,8 +982,9 @@ eos_status enqueue_frame(eos_frame_buffers& fb, const Frame& f, const FrameStrea
             // reflection chain: it takes the kernel without the group walk, whose
             // 24 KiB of LDS per workgroup (32 KiB with it) leave the chain's
             // workgroups room (hit-dense 4K frame 17.3 -> 16.5 ms, config E
-            // 1.84 -> 1.80 ms); its launches are large, so the group walk would
-            // not be taken there anyway
+            // 1.84 -> 1.80 ms); a small frame's launch (256 x 256, one light: 65,536
+            // shadow rays at most, against 16,384 up to which 16 lanes take a ray)
+            // takes it too and walks each ray with a lane
             // and its grid leaves one wave slot per SIMD free: with every slot taken
             // (a set-up workgroup of the chain has no registers left either) the
             // chain waits for the end of this launch: 64 moving instances 2535 ->
